@@ -77,7 +77,7 @@ def build_solver(precision: str = "fp32") -> str:
     tmp = solver + ".tmp"
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     core_name = os.path.basename(core)[3:-3]  # libX.so -> X
-    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+    _run([os.environ.get("CXX", "g++"), "-O3", "-std=c++17", "-fPIC", "-shared",
           "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", "-Wno-unused-result", *_defines(precision),
           "-I", os.path.join(ROOT, "include"), "-I", os.path.join(rocm, "include"),
           os.path.join(PKG, "cpp", "solver_capi.cpp"), "-L", LIB_DIR, "-l" + core_name,

@@ -15,20 +15,21 @@
 //               serve later steps while bodies move less than s/2 (the step
 //               decides on the device when to rebuild); s = 0 gives lists
 //               for the current positions only.
-//  narrow phase one wavefront per candidate pair. A's nodes are swept in
-//               chunks of 64 (one node per lane). A chunk is skipped when its
-//               bounding sphere cannot satisfy the node test (the same three
-//               bounds at chunk level: sphere, stencil, SDF box, Lipschitz).
-//               Each remaining node evaluates the reference's predicate
-//               exactly in FP64: stencil membership of the target's cell,
-//               bounding sphere (particle targets, lower index only), SDF box
-//               and -phi >= 0. The wave counts its contacts, reserves that
-//               many history records, then recomputes each contact's normal
-//               and point, takes its previous spring (keyed by (A, target,
-//               node)), applies the linear spring-dashpot law and writes the
-//               updated spring. Forces and torques are summed per pair in
-//               node order, serially, so the result does not depend on the
-//               schedule.
+//  narrow phase runs of one to eight candidate pairs per wavefront
+//               (sweepRun). Node groups of 16 and then nodes are culled in the
+//               target's frame by a code per SDF cell (how far the nearest
+//               cell with phi <= 0 is); each remaining node evaluates the
+//               reference's predicate exactly in FP64: stencil membership of
+//               the target's cell, bounding sphere (particle targets, lower
+//               index only), SDF box and -phi >= 0. The contacts' normals and
+//               points are staged in node order and history records reserved;
+//               then one thread per pair takes each contact's previous spring
+//               (keyed by (A, target, node)), applies the linear
+//               spring-dashpot law and writes the updated spring. Forces and
+//               torques are summed per pair in node order, serially, so the
+//               result does not depend on the schedule. (The single-set entry
+//               and law mode 2 sweep one pair per wave by 64-node chunks,
+//               with the same predicate.)
 //
 // All culls are conservative with a relative margin of 1e-5 on reaches (a
 // unit quaternion stored in FP32 scales vectors by up to 1 +- 2.4e-7), so
@@ -364,7 +365,6 @@ struct NarrowMulti {
   NarrowCommon c;
   const int* gate;
   int nsets;
-  int wallSet;  // set swept by kWallGroups (kCullSweep leaves it out), or -1
   NarrowSet s[kMaxSets];
 };
 
@@ -447,29 +447,6 @@ __device__ __forceinline__ bool nodeHit(V3 p, const Target& tg, I3 tcell, const 
   const I3 c = clampedCell(p, g);
   return abs(tcell.x - c.x) <= 1 && abs(tcell.y - c.y) <= 1 && abs(tcell.z - c.z) <= 1;
 }
-// nodeHit in two halves, so that the SDF fetches of several nodes can be in
-// flight together: the tests before the fetch (target cell id valid, sphere,
-// SDF box) with the cell's location, then the tests after it (phi <= 0, the
-// node's cell in the target's stencil).
-template <int SET>
-__device__ __forceinline__ bool nodeCell(V3 p, const Target& tg, const fdm_grid& g, double RB,
-                                         Sample& s, int& base) {
-  if (tg.hash < 0 || (long long)tg.hash >= g.num) return false;
-  const V3 rel = vsub(p, tg.x);
-  if (SET == FDM_SET_PARTICLE) {
-    if (vlen2(rel) > RB * RB) return false;
-  }
-  const V3 local = toLocal(rel, tg);
-  if (!sdfLocate(local, tg.t, s, base)) return false;
-  return !(SET == FDM_SET_WALL && planeClear(local, tg.t));
-}
-__device__ __forceinline__ bool nodeHitAt(V3 p, const Sample& s, I3 tcell, const fdm_grid& g) {
-  const double ov = -trilinear(s.x, s.y, s.z, s.c);
-  if (!(ov >= 0.)) return false;
-  const I3 c = clampedCell(p, g);
-  return abs(tcell.x - c.x) <= 1 && abs(tcell.y - c.y) <= 1 && abs(tcell.z - c.z) <= 1;
-}
-
 __device__ __forceinline__ int findPrevPair(const NarrowSet& a, int p, int A, int T, int& off) {
   // lists kept from the previous step hold the pair at the same index
   if (p < min(ldu(a.prev.total), a.prev.capacity) && ldu(a.prev.pairA + p) == A &&
@@ -558,17 +535,6 @@ struct HitSlots {
   double nrm[3][kMaxHits];
   double ov[kMaxHits];
   int node[kMaxHits];
-};
-
-// Nodes of one pair that passed the tests before the SDF fetch (sphere, SDF
-// box), per wave in LDS, in node order: position, fractional cell position,
-// first corner of the cell, node id; and the hit mask of each chunk.
-struct CandSlots {
-  double px[kMaxHits], py[kMaxHits], pz[kMaxHits];
-  double fx[kMaxHits], fy[kMaxHits], fz[kMaxHits];
-  int base[kMaxHits];
-  int node[kMaxHits];
-  unsigned long long chunkHits[FDM_MAX_CHUNKS];
 };
 
 // One wave per candidate pair: chunk culls (one chunk per lane), the node
@@ -881,616 +847,524 @@ __device__ __forceinline__ void stageHit(double* g, V3 pc, V3 nrm, double ov, in
   g[7] = (double)k;
 }
 
-// Node sweep of one kept pair (one wave): the culls and exact predicate of
-// processPair; the contacts' geometry is staged in node order (through LDS,
-// or recomputed chunk by chunk past kMaxHits) for the contact-law kernel,
-// and the pair's record range is reserved.
-// CULL: first take the particle-level pre-cull test (sphere, SDF box,
-// Lipschitz bound at this step's positions) from the same values, and leave
-// empty record ranges when it rejects the pair.
-// NPL (nodes per lane and iteration): 1 sweeps one surviving chunk at a
-// time; 2 two chunks at a time; 3 first collects, chunk by chunk, the nodes
-// that pass the tests before the SDF fetch into LDS (in node order) and then
-// fetches the SDF cells of up to 64 of them at once, so that a pair whose
-// few candidate nodes are spread over several chunks waits for one round of
-// fetches instead of one per chunk.
-template <int SET, bool CULL = false, int NPL = 1>
-__device__ void sweepPair(const NarrowCommon& C, const NarrowSet& S, const NarrowScratch& X, int w,
-                          int p, int lane, HitSlots& hs, int pool, CandSlots* cs = nullptr) {
-  const int A = ldu(S.pairs.pairA + p);
-  const int T = ldu(S.pairs.pairT + p);
-  const int n = C.P.n;
-  const fdm_template& tA = tmplOf(C.pgeo, ldu(C.P.geo + A));
-  const PairFrame fr = pairFrame<SET>(C, S, A);
-  const Q4 qA = detectQA<SET>(C, fr, A);
-  const V3 xA = detectPosA<SET>(C, fr, A);
-  const fdm_grid& tgrid = *fr.tgrid;
-  Target tg;
-  V3 armB;
-  resolveTarget<SET>(C, S, p, T, fr, tg, armB);
-  if (CULL) {
-    const double RA = tA.radius * kReach;
-    const double reachT = SET == FDM_SET_PARTICLE ? tg.t.radius : tg.t.boxReach;
-    const V3 d = vsub(xA, tg.x);
-    const double rs = RA + reachT * kReach;
-    bool keep = vlen2(d) <= rs * rs;
-    if (keep) {
-      const V3 local = toLocal(d, tg);
-      // (no Lipschitz test at the pair level here: it would put an SDF fetch
-      // before the chunk culls, whose own Lipschitz tests reject the same
-      // pairs with their fetches in flight together)
-      keep = !outsideBox(local, RA, tg.t);
-    }
-    if (!keep) {
-      if (lane == 0) {
-        S.pairs.recOff[p] = 0;
-        S.pairs.recCnt[p] = 0;
-        if (X.lawHead) *reinterpret_cast<int4*>(X.lawHead + 8 * (size_t)w) = make_int4(0, 0, 0, 0);
-      }
-      return;
-    }
+// ------------------------------------------------------------------- sweep
+// What the culls need of one pair, in FP32 (margins below). With SDF grids:
+// a point s of A's template frame has the index coordinates m s + t in the
+// target's grid; a plane wall uses row 0 as its value there.
+struct alignas(16) CullRec {
+  float m[9], t[3];
+  float centre[3], radius;   // target's centre in index coordinates, bounding radius (spacings)
+  float top[3], eps;         // nodes per axis - 1; slack of an index coordinate
+  float scale, planeSlack;   // spacings per length (plane walls: |gradient|)
+  int size[2];               // cells per axis, x and y
+  long long cells;           // first cell code; -1: a plane wall
+  int groupStart, groupCount;
+};
+// What the exact predicate needs of one pair.
+struct PairCtx {
+  double qA[4], xA[3], qT[4], xT[3], ih;
+  int geoA, geoT, hash, inst;
+};
+constexpr int kRunMax = 8;                  // pairs of one wave and item
+constexpr int kUnitLanes = FDM_GROUP;       // groups per unit of the group cull, nodes per group
+constexpr int kMaxBlocks = FDM_CHUNK * FDM_MAX_CHUNKS / (FDM_GROUP * kUnitLanes);  // units per pair
+constexpr int kLiveMax = 256;
+// Per-wave LDS of the sweep.
+struct SweepSlots {
+  CullRec cull[kRunMax];
+  PairCtx ctx[kRunMax];
+  double pc[3][kMaxHits], nrm[3][kMaxHits], ov[kMaxHits];  // the run's hits in the order found
+  unsigned long long chunks[kRunMax];                      // chunks of the pair holding hits
+  int hit[kMaxHits];                                       // pair of the run << 16 | node
+  int cand[64];  // nodes that passed the cell test, not yet tested exactly (same coding)
+  int total[kRunMax], gbase[kRunMax];
+  unsigned short unit[kRunMax * kMaxBlocks];  // pair << 8 | block of groups
+  unsigned short live[kLiveMax];              // pair << 8 | surviving group
+};
+template <bool MANY>
+__device__ __forceinline__ fdm_grid particleGrid(const NarrowCommon& C, int inst) {
+  if (MANY) return ldu(C.inst.pgrid + inst);
+  // (opaque in every run: what is computed from them, as the periods, would
+  // otherwise be kept in VGPRs over the wave's whole loop)
+  fdm_grid g = C.pgrid;
+  asm volatile("" : "+s"(g.min.x), "+s"(g.min.y), "+s"(g.max.x), "+s"(g.max.y));
+  return g;
+}
+template <int SET, bool MANY>
+__device__ __forceinline__ fdm_grid targetGrid(const NarrowCommon& C, const NarrowSet& S, int inst) {
+  if (MANY) return SET == FDM_SET_WALL ? ldu(C.inst.wgrid + inst) : ldu(C.inst.pgrid + inst);
+  return S.grid;
+}
+__device__ __forceinline__ float clampTo(float u, float hi) { return __builtin_amdgcn_fmed3f(u, 0.f, hi); }
+// The code of the SDF cell nearest to index coordinates u (their clamped
+// values in c), and the cell's indices.
+__device__ __forceinline__ int cellCode(const CullRec& k, const unsigned char* cells, const float u[3],
+                                        float c[3], int i[3]) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    c[a] = clampTo(u[a], k.top[a]);
+    i[a] = min((int)c[a], (int)k.top[a] - 1);
   }
-  const double RB = tg.t.radius;
-  const I3 tcell = decodeHash(tg.hash, tgrid);
-  const fdm_real* nodes = C.pgeo.nodes + 3 * (size_t)tA.nodeStart;
-  const float4* chunks = reinterpret_cast<const float4*>(C.pgeo.chunks) + tA.chunkStart;
-  const int nChunks = tA.chunkCount;
-  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-
-  bool live = false;
-  if (lane < nChunks) {
-    const float4 ch = chunks[lane];
-    const V3 cw = vadd(qrotate(qA, {(double)ch.x, (double)ch.y, (double)ch.z}), xA);
-    const double rc = (double)ch.w * kReach;
-    live = true;
-    if (SET == FDM_SET_PARTICLE) {
-      const double rr = (RB + rc) * (1.0 + 1e-9);
-      if (vlen2(vsub(cw, tg.x)) > rr * rr) live = false;
-    }
-    if (live) {
-      I3 lo, hi;
-      cellRange(cw, rc, tgrid, lo, hi);
-      if (!cellNear(tcell, lo, hi)) live = false;
-    }
-    if (live) {
-      const V3 lc = toLocal(vsub(cw, tg.x), tg);
-      if (outsideBox(lc, rc, tg.t) || levelClear(lc, rc, tg.t, tg.sdf)) live = false;
-    }
-  }
-  const unsigned long long liveChunks = ballot64(live);
-  // An affine (plane-wall) target: the plane's value at node s of A is
-  // affine in s, plane(toLocal(R_A s + x_A - x_T)) = c0 + u . s with
-  // g = R_T a (a: the plane's gradient), u = R_A^T g, c0 = plane_3 +
-  // g . (x_A - x_T) (the rotation formula's transpose is the conjugate's,
-  // for any quaternion). A node with c0 + u . s above the plane's slack has
-  // phi > 0 (the slack covers this evaluation's rounding as well), so its
-  // transform and SDF fetch are skipped.
-  const bool planeNodes = SET == FDM_SET_WALL && tg.t.affine;
-  V3 pu = {0., 0., 0.};
-  double pc0 = 0.;
-  if (planeNodes && liveChunks) {
-    const V3 ga = toWorld({tg.t.plane[0], tg.t.plane[1], tg.t.plane[2]}, tg);
-    pu = qrotateT(ga, qA);
-    pc0 = tg.t.plane[3] + vdot(ga, vsub(xA, tg.x));
-  }
-  auto planeSkip = [&](V3 sn) {
-    return planeNodes && pc0 + pu.x * sn.x + pu.y * sn.y + pu.z * sn.z > tg.t.planeSlack;
-  };
-  // the previous step's record range of the pair, for the law's header (its
-  // scalar loads complete while the nodes are swept)
-  int prevOff = 0;
-  const int prevCnt = X.lawHead && liveChunks ? findPrevPair(S, p, A, T, prevOff) : 0;
-
-  unsigned long long myMask = 0ull;
-  int total = 0;
-  // a hit's contact geometry, into LDS slot `slot` (node order)
-  auto stage = [&](int slot, int k, V3 pn, const Sample& sm) {
-    const double ov = -trilinear(sm.x, sm.y, sm.z, sm.c);
-    const V3 nrm = vnormalize(toWorld(gradientIntX(sm.x, sm.y, sm.z, sm.c), tg));
-    const V3 pc = vadd(pn, vmul(nrm, 0.5 * ov));
-    hs.pc[0][slot] = pc.x;
-    hs.pc[1][slot] = pc.y;
-    hs.pc[2][slot] = pc.z;
-    hs.nrm[0][slot] = nrm.x;
-    hs.nrm[1][slot] = nrm.y;
-    hs.nrm[2][slot] = nrm.z;
-    hs.ov[slot] = ov;
-    hs.node[slot] = k;
-  };
-  if (NPL == 3) {
-    if (lane < nChunks) cs->chunkHits[lane] = 0ull;
-    int ncand = 0;
-    // SDF fetch and predicate of the collected candidates, their hits staged
-    // in node order
-    auto flush = [&]() {
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      bool hit = false;
-      Sample sm;
-      V3 pn = {0., 0., 0.};
-      int k = 0;
-      if (lane < ncand) {
-        pn = {cs->px[lane], cs->py[lane], cs->pz[lane]};
-        sm.x = cs->fx[lane];
-        sm.y = cs->fy[lane];
-        sm.z = cs->fz[lane];
-        k = cs->node[lane];
-        sdfCorners(tg.sdf + cs->base[lane], tg.t, sm);
-        hit = nodeHitAt(pn, sm, tcell, tgrid);
-      }
-      const unsigned long long m = ballot64(hit);
-      if (hit) {
-        const int slot = total + __popcll(m & lt);
-        if (slot < kMaxHits) stage(slot, k, pn, sm);
-        atomicOr(&cs->chunkHits[k / FDM_CHUNK], 1ull << (k % FDM_CHUNK));
-      }
-      total += __popcll(m);
-      ncand = 0;
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    };
-    fdm_real cx = 0, cy = 0, cz = 0;
-    if (liveChunks) {
-      const int k0 = __builtin_ctzll(liveChunks) * FDM_CHUNK + lane;
-      if (k0 < tA.nodeCount) {
-        cx = nodes[3 * k0];
-        cy = nodes[3 * k0 + 1];
-        cz = nodes[3 * k0 + 2];
-      }
-    }
-    for (unsigned long long lcm = liveChunks; lcm; lcm &= lcm - 1ull) {
-      const int c = __builtin_ctzll(lcm);
-      const int k = c * FDM_CHUNK + lane;
-      const V3 sn = {(double)cx, (double)cy, (double)cz};
-      const unsigned long long rest = lcm & (lcm - 1ull);
-      if (rest) {
-        const int k2 = __builtin_ctzll(rest) * FDM_CHUNK + lane;
-        if (k2 < tA.nodeCount) {
-          cx = nodes[3 * k2];
-          cy = nodes[3 * k2 + 1];
-          cz = nodes[3 * k2 + 2];
-        }
-      }
-      bool ok = false;
-      Sample sm;
-      int b = 0;
-      V3 pn = {0., 0., 0.};
-      if (k < tA.nodeCount && !planeSkip(sn)) {
-        pn = vadd(qrotate(qA, sn), xA);
-        ok = nodeCell<SET>(pn, tg, tgrid, RB, sm, b);
-      }
-      const unsigned long long m = ballot64(ok);
-      if (ncand + __popcll(m) > kMaxHits) flush();
-      if (ok) {
-        const int slot = ncand + __popcll(m & lt);
-        cs->px[slot] = pn.x;
-        cs->py[slot] = pn.y;
-        cs->pz[slot] = pn.z;
-        cs->fx[slot] = sm.x;
-        cs->fy[slot] = sm.y;
-        cs->fz[slot] = sm.z;
-        cs->base[slot] = b;
-        cs->node[slot] = k;
-      }
-      ncand += __popcll(m);
-    }
-    if (ncand > 0) flush();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (lane < nChunks) myMask = cs->chunkHits[lane];
-  }
-  if (NPL == 2) {
-    // two surviving chunks per iteration (128 nodes in flight per wave): each
-    // lane tests node `lane` of both, the second chunk's SDF fetches issued
-    // before the first chunk's values are used; hits staged in node order
-    for (unsigned long long lcm = liveChunks; lcm;) {
-      const int c = __builtin_ctzll(lcm);
-      lcm &= lcm - 1ull;
-      const int c2 = lcm ? __builtin_ctzll(lcm) : -1;
-      if (lcm) lcm &= lcm - 1ull;
-      const int k = c * FDM_CHUNK + lane, k2 = c2 * FDM_CHUNK + lane;
-      V3 s1 = {0., 0., 0.}, s2 = {0., 0., 0.};
-      if (k < tA.nodeCount) s1 = {(double)nodes[3 * k], (double)nodes[3 * k + 1], (double)nodes[3 * k + 2]};
-      if (c2 >= 0 && k2 < tA.nodeCount)
-        s2 = {(double)nodes[3 * k2], (double)nodes[3 * k2 + 1], (double)nodes[3 * k2 + 2]};
-      const bool has = k < tA.nodeCount && !planeSkip(s1);
-      const bool has2 = c2 >= 0 && k2 < tA.nodeCount && !planeSkip(s2);
-      V3 pn = {0., 0., 0.}, pn2 = {0., 0., 0.};
-      if (has) pn = vadd(qrotate(qA, s1), xA);
-      if (has2) pn2 = vadd(qrotate(qA, s2), xA);
-      Sample sm, sm2;
-      int b1 = 0, b2 = 0;
-      bool in1 = has && nodeCell<SET>(pn, tg, tgrid, RB, sm, b1);
-      bool in2 = has2 && nodeCell<SET>(pn2, tg, tgrid, RB, sm2, b2);
-      if (in1) sdfCorners(tg.sdf + b1, tg.t, sm);
-      if (in2) sdfCorners(tg.sdf + b2, tg.t, sm2);
-      const bool hit = in1 && nodeHitAt(pn, sm, tcell, tgrid);
-      const bool hit2 = in2 && nodeHitAt(pn2, sm2, tcell, tgrid);
-      const unsigned long long m = ballot64(hit), m2 = ballot64(hit2);
-      if (lane == c) myMask = m;
-      if (c2 >= 0 && lane == c2) myMask = m2;
-      if (hit) {
-        const int slot = total + __popcll(m & lt);
-        if (slot < kMaxHits) stage(slot, k, pn, sm);
-      }
-      total += __popcll(m);
-      if (hit2) {
-        const int slot = total + __popcll(m2 & lt);
-        if (slot < kMaxHits) stage(slot, k2, pn2, sm2);
-      }
-      total += __popcll(m2);
-    }
-  }
-  fdm_real nx = 0, ny = 0, nz = 0;
-  if (NPL == 1 && liveChunks) {
-    const int k0 = __builtin_ctzll(liveChunks) * FDM_CHUNK + lane;
-    if (k0 < tA.nodeCount) {
-      nx = nodes[3 * k0];
-      ny = nodes[3 * k0 + 1];
-      nz = nodes[3 * k0 + 2];
-    }
-  }
-  for (unsigned long long lcm = NPL == 1 ? liveChunks : 0ull; lcm; lcm &= lcm - 1ull) {
-    const int c = __builtin_ctzll(lcm);
-    const int k = c * FDM_CHUNK + lane;
-    const V3 s = {(double)nx, (double)ny, (double)nz};
-    const unsigned long long rest = lcm & (lcm - 1ull);
-    if (rest) {
-      const int k2 = __builtin_ctzll(rest) * FDM_CHUNK + lane;
-      if (k2 < tA.nodeCount) {
-        nx = nodes[3 * k2];
-        ny = nodes[3 * k2 + 1];
-        nz = nodes[3 * k2 + 2];
-      }
-    }
-    bool hit = false;
-    Sample sm;
-    V3 pn;
-    if (k < tA.nodeCount && !planeSkip(s)) {
-      pn = vadd(qrotate(qA, s), xA);
-      hit = nodeHit<SET>(pn, tg, tcell, tgrid, RB, sm);
-    }
-    const unsigned long long m = ballot64(hit);
-    if (lane == c) myMask = m;
-    if (hit) {
-      const int slot = total + __popcll(m & lt);
-      if (slot < kMaxHits) {
-        const double ov = -trilinear(sm.x, sm.y, sm.z, sm.c);
-        const V3 nrm = vnormalize(toWorld(gradientIntX(sm.x, sm.y, sm.z, sm.c), tg));
-        const V3 pc = vadd(pn, vmul(nrm, 0.5 * ov));
-        hs.pc[0][slot] = pc.x;
-        hs.pc[1][slot] = pc.y;
-        hs.pc[2][slot] = pc.z;
-        hs.nrm[0][slot] = nrm.x;
-        hs.nrm[1][slot] = nrm.y;
-        hs.nrm[2][slot] = nrm.z;
-        hs.ov[slot] = ov;
-        hs.node[slot] = k;
-      }
-    }
-    total += __popcll(m);
-  }
-
-  // the record and staging reservations and the mirror slot, their atomics
-  // issued together by lane 0 (one round trip instead of three)
-  int base = 0, gbase = 0, mpos = 0;
-  const bool mirrored = SET != FDM_SET_WALL && total > 0 && T != A;
-  if (total > 0) {
-    int rb = 0, gb = 0;
-    if (lane == 0) {
-      rb = atomicAdd(S.pairs.recTotal + pool * FDM_REC_STRIDE, total);
-      gb = atomicAdd(X.hitCount + pool * FDM_REC_STRIDE, total);
-      if (mirrored) mpos = atomicAdd(&S.mirror.count[T], 1);
-    }
-    rb = readlaneI(rb, 0);
-    gb = readlaneI(gb, 0);
-    const int rCap = S.pairs.recCapacity / FDM_REC_POOLS, gCap = X.hitCapacity / FDM_REC_POOLS;
-    if (rb + total > rCap || gb + total > gCap) {
-      if (lane == 0)
-        atomicOr(C.status, rb + total > rCap ? FDM_STATUS_RECORD_OVERFLOW : FDM_STATUS_STAGING_OVERFLOW);
-      total = 0;
-    } else {
-      base = pool * rCap + rb;
-      gbase = pool * gCap + gb;
-    }
-  }
-  if (total > 0 && total <= kMaxHits) {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (lane < total)
-      stageHit(X.hitGeom + 8 * (size_t)(gbase + lane), {hs.pc[0][lane], hs.pc[1][lane], hs.pc[2][lane]},
-               {hs.nrm[0][lane], hs.nrm[1][lane], hs.nrm[2][lane]}, hs.ov[lane], hs.node[lane]);
-  } else if (total > 0) {
-    // more contacts than slots: recompute each chunk's hits
-    const unsigned long long chunksWith = ballot64(myMask != 0ull);
-    int running = 0;
-    for (unsigned long long cw = chunksWith; cw; cw &= cw - 1ull) {
-      const int c = __builtin_ctzll(cw);
-      const unsigned lo32 = __builtin_amdgcn_readlane((unsigned)myMask, c);
-      const unsigned hi32 = __builtin_amdgcn_readlane((unsigned)(myMask >> 32), c);
-      const unsigned long long m = ((unsigned long long)hi32 << 32) | lo32;
-      if ((m >> lane) & 1ull) {
-        const int k = c * FDM_CHUNK + lane;
-        const V3 s = {(double)nodes[3 * k], (double)nodes[3 * k + 1], (double)nodes[3 * k + 2]};
-        const V3 pn = vadd(qrotate(qA, s), xA);
-        Sample sm;
-        nodeHit<SET>(pn, tg, tcell, tgrid, RB, sm);
-        const double ov = -trilinear(sm.x, sm.y, sm.z, sm.c);
-        const V3 nrm = vnormalize(toWorld(gradientIntX(sm.x, sm.y, sm.z, sm.c), tg));
-        const V3 pc = vadd(pn, vmul(nrm, 0.5 * ov));
-        stageHit(X.hitGeom + 8 * (size_t)(gbase + running + __popcll(m & lt)), pc, nrm, ov, k);
-      }
-      running += __popcll(m);
-    }
-  }
-  if (lane == 0) {
-    S.pairs.recOff[p] = base;
-    S.pairs.recCnt[p] = total;
-    X.workHit[w] = gbase;
-    if (X.lawHead) {
-      int4* h = reinterpret_cast<int4*>(X.lawHead + 8 * (size_t)w);
-      h[0] = make_int4(total, base, gbase, A);
-      if (total > 0) h[1] = make_int4(T, prevOff, prevCnt, 0);
-    }
-    // (a pair whose reservation overflowed keeps its mirror slot, with no
-    // records and zero sums: the slot count and the list agree, and the
-    // target's fold adds nothing stale)
-    if (mirrored) {
-      if (mpos < S.mirror.capacity) S.mirror.list[(size_t)T * S.mirror.capacity + mpos] = p;
-      else atomicOr(C.status, FDM_STATUS_BUCKET_OVERFLOW);
-      if (total == 0)
-        for (int c = 0; c < 3; ++c) {
-          S.pairs.sumF[3 * (size_t)p + c] = 0.;
-          S.pairs.sumTB[3 * (size_t)p + c] = 0.;
-        }
-    }
-  }
+  return cells[k.cells + i[0] + k.size[0] * (i[1] + k.size[1] * i[2])];
+}
+__device__ __forceinline__ void cullPoint(const CullRec& k, float x, float y, float z, float u[3]) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+    u[a] = fmaf(k.m[3 * a], x, fmaf(k.m[3 * a + 1], y, fmaf(k.m[3 * a + 2], z, k.t[a])));
+}
+template <int SET>
+__device__ __forceinline__ bool inSphere(const CullRec& k, const float u[3], float r) {
+  if (SET != FDM_SET_PARTICLE) return true;
+  const float x = u[0] - k.centre[0], y = u[1] - k.centre[1], z = u[2] - k.centre[2], rr = k.radius + r;
+  return fmaf(x, x, fmaf(y, y, z * z)) <= rr * rr;
+}
+// Whether the ball about the point s of A's frame may hold a contact of the
+// pair: a contact point q lies in a cell with code 0, the point p of the SDF
+// box nearest to the ball's centre has |centre - q|^2 >= |centre - p|^2 +
+// |p - q|^2 (the box is convex), and |p - q| is at least the distance that
+// the code of p's cell gives.
+template <int SET>
+__device__ __forceinline__ bool ballMayTouch(const CullRec& k, const unsigned char* cells, float4 s) {
+  float u[3], c[3];
+  cullPoint(k, s.x, s.y, s.z, u);
+  if (SET == FDM_SET_WALL && k.cells < 0) return u[0] - k.scale * s.w <= k.planeSlack;
+  const float r = fmaf(s.w, k.scale, 2.f * k.eps);
+  if (!inSphere<SET>(k, u, r)) return false;
+  int i[3];
+  const float d = (float)max(cellCode(k, cells, u, c, i) - 1, 0) * (1.f / FDM_CELL_UNIT);
+  const float ex = u[0] - c[0], ey = u[1] - c[1], ez = u[2] - c[2];
+  return fmaf(ex, ex, fmaf(ey, ey, fmaf(ez, ez, d * d))) * (1.f - 1e-5f) <= r * r;
+}
+// The same for a node: its cell's code is 0, or it lies within the slack of a
+// face of a cell next to such a cell.
+template <int SET>
+__device__ __forceinline__ bool nodeMayTouch(const CullRec& k, const unsigned char* cells, float4 s) {
+  float u[3], c[3];
+  cullPoint(k, s.x, s.y, s.z, u);
+  if (SET == FDM_SET_WALL && k.cells < 0) return u[0] <= k.planeSlack;
+  if (!inSphere<SET>(k, u, k.eps)) return false;
+  int i[3];
+  const int code = cellCode(k, cells, u, c, i);
+  if (!(fmaxf(fmaxf(fabsf(u[0] - c[0]), fabsf(u[1] - c[1])), fabsf(u[2] - c[2])) <= k.eps)) return false;
+  if (code != 1) return code == 0;
+  float f = 1.f;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) f = fminf(f, fminf(c[a] - (float)i[a], (float)(i[a] + 1) - c[a]));
+  return f <= k.eps;
 }
 
-// Four wall pairs per wave, sixteen lanes each (pair 4q + j on lanes
-// 16j..16j+15): the pre-cull, chunk culls and exact node predicate of
-// sweepPair<FDM_SET_WALL, true>, with the per-pair values held per lane. A
-// group first collects, in node order, the nodes of its surviving chunks
-// that pass the plane test of an affine target (every node of another
-// target) into LDS, then evaluates the predicate on them sixteen at a time,
-// so that the few nodes near a plane wall are fetched in one round for four
-// pairs. Contacts are staged in LDS in node order (past kGroupHits they are
-// recomputed straight into the workspace once the range is reserved).
-constexpr int kGroupHits = 16;
-constexpr int kGroupedWallPairs = 65536;
-constexpr int kGroupCands = 64;
-struct WallGroupSlots {
-  double pc[3][4][kGroupHits];
-  double nrm[3][4][kGroupHits];
-  double ov[4][kGroupHits];
-  int node[4][kGroupHits];
-  int cand[4][kGroupCands];
-};
-
-__device__ void sweepWallGroup(const NarrowCommon& C, const NarrowSet& S, const NarrowScratch& X,
-                               int g0, int nPairs, int q, unsigned gmask, int lane,
-                               WallGroupSlots& ws) {
-  const int grp = lane >> 4, gl = lane & 15, sh = 16 * grp;
-  const int p = 4 * q + grp;
-  const int w = g0 + p;
-  const unsigned below = gl == 0 ? 0u : (0xFFFFu >> (16 - gl));  // lanes of the group below this one
-  auto groupBits = [&](unsigned long long m) __attribute__((always_inline)) {
-    return (unsigned)((m >> sh) & 0xFFFFull);
-  };
-  bool active = p < nPairs && ((gmask >> grp) & 1u);
-  const int A = active ? ldu(S.pairs.pairA + p) : 0;
-  const int T = active ? ldu(S.pairs.pairT + p) : 0;
+// Node sweep of a run of `np` <= kRunMax candidate pairs of one set by one
+// wave: the pairs, their node groups and their nodes are culled in the
+// target's frame, the remaining nodes of all the run's pairs take the
+// reference's exact predicate together, and each pair's contacts are staged
+// in node order for the contact-law kernel, with its record range reserved.
+//
+// A pair is a chain of dependent loads (list, bodies, templates, groups,
+// cell codes, nodes, cell codes, SDF corners) with little arithmetic between
+// them, and each stage leaves a different number of items per pair. So a run
+// goes through the stages together, each stage's items taken from a list in
+// LDS and dealt to all lanes:
+//  - one pair per lane: poses, bounding spheres, and the map from A's
+//    template frame to the target's SDF index coordinates (one 3 x 3 matrix
+//    and a shift);
+//  - one node group (16 nodes) per lane, then one node per lane: placed with
+//    nine multiply-adds and tested against one byte, its SDF cell's code: the
+//    distance to the nearest cell in which phi can be <= 0. (A Lipschitz
+//    bound of phi does not serve here: f / |grad f| is steep to 1e9 at the
+//    centre of a superellipsoid.) Affine walls test the plane instead;
+//  - the exact predicate (two quaternion rotations, eight SDF corners, the
+//    cell stencil: some 300 FP64 instructions) for the few nodes left.
+// Measured against one pair per wave with 64-node chunks culled by Lipschitz
+// bound and swept in FP64 (and wall pairs four per wave): 254K particle pairs
+// of a compressed lattice, 23 % of them in contact, 613 + 22 -> 201 us; the
+// million-particle pour's 11.4K wall, 5.8K particle and 4.1K image pairs 44.3
+// -> 23 us; 44.6K pairs of touching 400-node spheres 79 -> 29 us; one pair
+// alone 10.7 -> 10.1 us.
+// Margins: reaches are widened by kReach (a unit quaternion stored in FP32
+// scales vectors by up to 1 +- 2.4e-7), and index coordinates by eps, which
+// covers the FP32 rounding of the map, of the nodes and of their sums (a few
+// 2^-24 of the largest coordinate) and the exact predicate's own rounding.
+template <int SET, bool MANY>
+__device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const NarrowScratch& X, int w0,
+                         int p0, int np, int lane, SweepSlots& ws) {
+  // (opaque in every run, as the grid in particleGrid)
+  asm volatile("" : "+v"(lane));
+  const int n = C.P.n;
+  const int p = p0 + lane, w = w0 + lane;
+  const fdm_geometry& tgeo = SET == FDM_SET_WALL ? C.wgeo : C.pgeo;
+  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   auto emptyRange = [&]() __attribute__((always_inline)) {
-    if (gl == 0) {
-      S.pairs.recOff[p] = 0;
-      S.pairs.recCnt[p] = 0;
-      *reinterpret_cast<int4*>(X.lawHead + 8 * (size_t)w) = make_int4(0, 0, 0, 0);
-    }
+    S.pairs.recOff[p] = 0;
+    S.pairs.recCnt[p] = 0;
+    if (X.lawHead) *reinterpret_cast<int4*>(X.lawHead + 8 * (size_t)w) = make_int4(0, 0, 0, 0);
   };
-  if (active && A < 0) {  // slot left empty by a capacity overflow
-    emptyRange();
-    active = false;
-  }
-  // the caller gives groups whose pairs share the target (and system)
-  const unsigned long long act = ballot64(active);
-  if (!act) return;
-  const int ref = __builtin_ctzll(act);
-  const int Tu = readlaneI(T, ref), Au = readlaneI(A, ref);
-  const int inst = C.inst.count > 0 ? ldu(C.inst.particleInstance + Au) : 0;
-  // lanes of an inactive group read body Au and use nothing
-  const int Ai = active ? A : Au;
-  const int geoA = ldu(C.P.geo + Ai);
-  const double radiusA = ldu(&C.pgeo.info[geoA].radius);
-  const PairFrame fr = pairFrame<FDM_SET_WALL>(C, S, Au);
-  const Q4 qA = detectQA<FDM_SET_WALL>(C, fr, Ai);
-  const V3 xA = detectPosA<FDM_SET_WALL>(C, fr, Ai);
-  // the wall grid by value (wave-uniform; a pointer that may point into
-  // the kernel arguments would make the compiler copy them to scratch)
-  const fdm_grid tgrid = C.inst.count > 0 ? ldu(C.inst.wgrid + inst) : S.grid;
-  Target tg;
-  V3 armB;
-  resolveTarget<FDM_SET_WALL>(C, S, p, Tu, fr, tg, armB);
-  if (active) {
-    const double RA = radiusA * kReach;
-    const double rs = RA + tg.t.boxReach * kReach;
-    const V3 d = vsub(xA, tg.x);
-    bool keep = vlen2(d) <= rs * rs;
-    if (keep) keep = !outsideBox(toLocal(d, tg), RA, tg.t);
-    if (!keep) {
-      emptyRange();
-      active = false;
+  int units = 0;
+  int A = -1, T = 0;
+  int prevOff = 0, prevCnt = -1;  // previous record range of the pair (-1: not at its index)
+  if (lane < np) {
+    ws.total[lane] = 0;
+    ws.chunks[lane] = 0ull;
+    A = ldu(S.pairs.pairA + p);
+    T = ldu(S.pairs.pairT + p);
+    // (lists kept from the previous step hold the pair at the same index:
+    // these loads go along with the pair's own)
+    if (X.lawHead && p < min(ldu(S.prev.total), S.prev.capacity)) {
+      const int pA = ldu(S.prev.pairA + p), pT = ldu(S.prev.pairT + p);
+      prevOff = ldu(S.prev.recOff + p);
+      prevCnt = ldu(S.prev.recCnt + p);
+      if (pA != A || pT != T) prevCnt = -1;
     }
-  }
-  const double RB = tg.t.radius;
-  const I3 tcell = decodeHash(tg.hash, tgrid);
-  const int nChunks = active ? ldu(&C.pgeo.info[geoA].chunkCount) : 0;
-  const int nodeCount = active ? ldu(&C.pgeo.info[geoA].nodeCount) : 0;
-  const float4* chunks =
-      reinterpret_cast<const float4*>(C.pgeo.chunks) + ldu(&C.pgeo.info[geoA].chunkStart);
-  const fdm_real* nodes = C.pgeo.nodes + 3 * (size_t)ldu(&C.pgeo.info[geoA].nodeStart);
-
-  // chunk culls, sixteen chunks of the group's pair at a time
-  unsigned long long live = 0ull;
-  for (int cb = 0; cb < FDM_MAX_CHUNKS && ballot64(cb < nChunks); cb += 16) {
-    const int c = cb + gl;
-    bool lv = false;
-    if (c < nChunks) {
-      const float4 ch = chunks[c];
-      const V3 cw = vadd(qrotate(qA, {(double)ch.x, (double)ch.y, (double)ch.z}), xA);
-      const double rc = (double)ch.w * kReach;
-      I3 lo, hi;
-      cellRange(cw, rc, tgrid, lo, hi);
-      lv = cellNear(tcell, lo, hi);
-      if (lv) {
-        const V3 lc = toLocal(vsub(cw, tg.x), tg);
-        if (outsideBox(lc, rc, tg.t) || levelClear(lc, rc, tg.t, tg.sdf)) lv = false;
+    if (A >= 0) {  // (below zero: a slot left empty by a capacity overflow)
+      const int inst = MANY ? ldu(C.inst.particleInstance + A) : 0;
+      const fdm_grid pg = particleGrid<MANY>(C, inst);
+      const fdm_periodic per = MANY ? ldu(C.inst.periodic + inst) : C.periodic;
+      // A's and the target's poses as the set's detection sees them
+      V3 xA = ldpR(C.P.x, n, A);
+      Q4 qA = ld4R(C.P.q, n, A);
+      const int geoA = ldu(C.P.geo + A);
+      V3 xT;
+      Q4 qT;
+      int hash, geoT;
+      if (SET == FDM_SET_WALL) {
+        xT = ldpR(C.W.x, C.W.n, T);
+        qT = ld4R(C.W.q, C.W.n, T);
+        geoT = ldu(C.W.geo + T);
+        hash = ldu(S.targetHash + T);
+      } else {
+        xT = ldpR(C.P.x, n, T);
+        qT = ld4R(C.P.q, n, T);
+        geoT = ldu(C.P.geo + T);
+        if (SET == FDM_SET_PARTICLE) hash = ldu(S.targetHash + T);
+      }
+      if (SET == FDM_SET_GHOST) {
+        if (per.sector) {
+          const SectorWrap sw = sectorWrap(xA, pg, per);
+          qA = sectorTurnQ(qA, sw.turns, per);
+          xA = sw.x;
+        } else {
+          xA = wrapStages(xA, pg, per).afterY;
+        }
+        if (S.ghostFromReal) {
+          const WrapStages ww = wrapStages(xT, pg, per);
+          xT = ghostOf(S.ghostMask == 1 ? ww.afterX : ww.afterY, pg, S.ghostMask);
+          hash = ghostCellHash(xT, pg);
+        } else {
+          const int gi = ldu(S.pairs.pairG + p);
+          xT = ldd3R(S.ghostPos + 3 * (size_t)gi);
+          hash = ldu(S.ghostHash + gi);
+          if (S.ghostQ) {
+            const double* gq = S.ghostQ + 4 * (size_t)gi;
+            qT = {gq[0], gq[1], gq[2], gq[3]};
+          }
+        }
+      }
+      // (every template value is loaded before the sphere test, so that the
+      // loads go together)
+      const fdm_template* tA = C.pgeo.info + geoA;
+      const fdm_template* tT = tgeo.info + geoT;
+      const double RA = ldu(&tA->radius), RB = ldu(&tT->radius), reachT = ldu(&tT->boxReach);
+      const int groups = ldu(&tA->groupCount), groupStart = ldu(&tA->groupStart);
+      const double ih = ldu(&tT->invSpacing);
+      const V3 o = {ldu(&tT->origin[0]), ldu(&tT->origin[1]), ldu(&tT->origin[2])};
+      const int nx = ldu(&tT->size[0]), ny = ldu(&tT->size[1]), nz = ldu(&tT->size[2]);
+      const long long cellStart = ldu(&tT->cellStart);
+      const bool plane = SET == FDM_SET_WALL && ldu(&tT->affine);
+      V3 a = {0., 0., 0.};
+      double a3 = 0., slack = 0.;
+      if (SET == FDM_SET_WALL) {
+        a = {ldu(&tT->plane[0]), ldu(&tT->plane[1]), ldu(&tT->plane[2])};
+        a3 = ldu(&tT->plane[3]);
+        slack = ldu(&tT->planeSlack);
+      }
+      const V3 d = vsub(xA, xT);
+      const double rs = (RA + (SET == FDM_SET_PARTICLE ? RB : reachT)) * kReach;
+      if (vlen2(d) <= rs * rs) {
+        units = (groups + kUnitLanes - 1) / kUnitLanes;
+        PairCtx& c = ws.ctx[lane];
+        c.qA[0] = qA.q0; c.qA[1] = qA.q1; c.qA[2] = qA.q2; c.qA[3] = qA.q3;
+        c.xA[0] = xA.x; c.xA[1] = xA.y; c.xA[2] = xA.z;
+        c.qT[0] = qT.q0; c.qT[1] = qT.q1; c.qT[2] = qT.q2; c.qT[3] = qT.q3;
+        c.xT[0] = xT.x; c.xT[1] = xT.y; c.xT[2] = xT.z;
+        c.geoA = geoA;
+        c.geoT = geoT;
+        c.hash = hash;
+        c.inst = inst;
+        CullRec& k = ws.cull[lane];
+        k.groupStart = groupStart;
+        k.groupCount = groups;
+        if (plane) {
+          // the plane's value at s is c0 + u . s (the rotation formula's
+          // transpose is the conjugate's for any quaternion)
+          const V3 ga = qrotate(qT, a);
+          const V3 u = qrotateT(ga, qA);
+          const double c0 = a3 + vdot(ga, d);
+          const double a1 = fabs(a.x) + fabs(a.y) + fabs(a.z);
+          k.m[0] = (float)u.x;
+          k.m[1] = (float)u.y;
+          k.m[2] = (float)u.z;
+          k.t[0] = (float)c0;
+          k.scale = (float)(a1 * kReach);
+          k.planeSlack = (float)((slack + 2e-6 * (fabs(c0) + a1 * RA)) * kReach);
+          k.cells = -1;
+        } else {
+          c.ih = ih;
+          k.centre[0] = (float)(-o.x * ih);
+          k.centre[1] = (float)(-o.y * ih);
+          k.centre[2] = (float)(-o.z * ih);
+          // (the pair's coordinates stay within the two reaches of the centre)
+          const double span = (2. * RA + reachT) * ih;
+          k.eps = (float)(1e-4 + 2e-6 * span);
+          k.radius = (float)(RB * ih * kReach) + k.eps;
+          k.scale = (float)(ih * kReach);
+          k.top[0] = (float)(nx - 1);
+          k.top[1] = (float)(ny - 1);
+          k.top[2] = (float)(nz - 1);
+          k.size[0] = nx - 1;
+          k.size[1] = ny - 1;
+          k.cells = cellStart;
+        }
       }
     }
-    live |= (unsigned long long)groupBits(ballot64(lv)) << cb;
+    if (units == 0) emptyRange();
   }
-  int prevOff = 0;
-  const int prevCnt = active && live ? findPrevPair(S, p, A, T, prevOff) : 0;
-  const bool planeNodes = active && tg.t.affine;
-  V3 pu = {0., 0., 0.};
-  double pc0 = 0.;
-  if (planeNodes && live) {
-    const V3 ga = toWorld({tg.t.plane[0], tg.t.plane[1], tg.t.plane[2]}, tg);
-    pu = qrotateT(ga, qA);
-    pc0 = tg.t.plane[3] + vdot(ga, vsub(xA, tg.x));
-  }
-  auto loadNode = [&](int k) __attribute__((always_inline)) {
-    return V3{(double)nodes[3 * k], (double)nodes[3 * k + 1], (double)nodes[3 * k + 2]};
-  };
-  // a node worth the exact predicate: in range and, on an affine target,
-  // not above the plane by more than its slack (as in sweepPair)
-  auto candidate = [&](int k, V3 sn) __attribute__((always_inline)) {
-    return k < nodeCount &&
-           !(planeNodes && pc0 + pu.x * sn.x + pu.y * sn.y + pu.z * sn.z > tg.t.planeSlack);
-  };
-  auto stageLds = [&](int slot, int k, V3 pn, const Sample& sm) __attribute__((always_inline)) {
-    const double ov = -trilinear(sm.x, sm.y, sm.z, sm.c);
-    const V3 nrm = vnormalize(toWorld(gradientIntX(sm.x, sm.y, sm.z, sm.c), tg));
-    const V3 pc = vadd(pn, vmul(nrm, 0.5 * ov));
-    ws.pc[0][grp][slot] = pc.x;
-    ws.pc[1][grp][slot] = pc.y;
-    ws.pc[2][grp][slot] = pc.z;
-    ws.nrm[0][grp][slot] = nrm.x;
-    ws.nrm[1][grp][slot] = nrm.y;
-    ws.nrm[2][grp][slot] = nrm.z;
-    ws.ov[grp][slot] = ov;
-    ws.node[grp][slot] = k;
-  };
-
-  int ncand = 0, total = 0;
-  // the exact predicate of the collected candidates, sixteen per round, hits
-  // staged in node order
-  auto flush = [&]() __attribute__((always_inline)) {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    for (int r = 0; ballot64(r < ncand); r += 16) {
-      bool hit = false;
-      Sample sm;
-      V3 pn = {0., 0., 0.};
-      int k = 0;
-      if (r + gl < ncand) {
-        k = ws.cand[grp][r + gl];
-        pn = vadd(qrotate(qA, loadNode(k)), xA);
-        hit = nodeHit<FDM_SET_WALL>(pn, tg, tcell, tgrid, RB, sm);
-      }
-      const unsigned m = groupBits(ballot64(hit));
-      if (hit) {
-        const int slot = total + __popc(m & below);
-        if (slot < kGroupHits) stageLds(slot, k, pn, sm);
-      }
-      total += __popc(m);
-    }
-    ncand = 0;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  };
-  // collection: the i-th surviving chunk of every group per iteration, its
-  // 64 nodes four per lane (node 64c + 16u + gl, so u-major is node order)
-  for (unsigned long long rem = live; ballot64(rem != 0ull);) {
-    const int c = rem ? __builtin_ctzll(rem) : -1;
-    if (rem) rem &= rem - 1ull;
-    bool pass[4];
-    unsigned m[4];
-    int add = 0;
+  // units of the group cull, pair by pair
+  int before = units;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int k = c * FDM_CHUNK + 16 * u + gl;
-      pass[u] = c >= 0 && k < nodeCount && candidate(k, loadNode(k));
-      m[u] = groupBits(ballot64(pass[u]));
-      add += __popc(m[u]);
-    }
-    if (ballot64(ncand + add > kGroupCands)) flush();
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (pass[u]) ws.cand[grp][ncand + __popc(m[u] & below)] = c * FDM_CHUNK + 16 * u + gl;
-      ncand += __popc(m[u]);
-    }
+  for (int off = 1; off < kRunMax; off <<= 1) {
+    const int v = __shfl_up(before, off, 64);
+    if (lane >= off) before += v;
   }
-  if (ballot64(ncand > 0)) flush();
+  const int nUnits = __shfl(before, kRunMax - 1);
+  if (nUnits == 0) return;
+  for (int u = 0; u < units; ++u) ws.unit[before - units + u] = (unsigned short)(lane << 8 | u);
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 
-  // record and staging reservations (one lane of each group)
-  const int pool = w % FDM_REC_POOLS;
-  int rb = 0, gb = 0;
-  if (active && gl == 0 && total > 0) {
-    rb = atomicAdd(S.pairs.recTotal + pool * FDM_REC_STRIDE, total);
-    gb = atomicAdd(X.hitCount + pool * FDM_REC_STRIDE, total);
-  }
-  rb = __shfl(rb, sh);
-  gb = __shfl(gb, sh);
-  int base = 0, gbase = 0;
-  if (active && total > 0) {
-    const int rCap = S.pairs.recCapacity / FDM_REC_POOLS, gCap = X.hitCapacity / FDM_REC_POOLS;
-    if (rb + total > rCap || gb + total > gCap) {
-      if (gl == 0)
-        atomicOr(C.status, rb + total > rCap ? FDM_STATUS_RECORD_OVERFLOW : FDM_STATUS_STAGING_OVERFLOW);
-      total = 0;
-    } else {
-      base = pool * rCap + rb;
-      gbase = pool * gCap + gb;
+  auto quat = [](const double* q) __attribute__((always_inline)) { return Q4{q[0], q[1], q[2], q[3]}; };
+  // the maps of the run's pairs, one column per lane (column 3: the shift)
+  {
+    const int j = lane >> 2, col = lane & 3;
+    const bool has = __shfl(units, j) > 0;
+    if (has && (SET != FDM_SET_WALL || ws.cull[j].cells >= 0)) {
+      const PairCtx& c = ws.ctx[j];
+      CullRec& k = ws.cull[j];
+      const V3 e = qrotate(quat(c.qA), {col == 0 ? 1. : 0., col == 1 ? 1. : 0., col == 2 ? 1. : 0.});
+      const V3 d = vsub({c.xA[0], c.xA[1], c.xA[2]}, {c.xT[0], c.xT[1], c.xT[2]});
+      const V3 l = vmul(qrotateT({col < 3 ? e.x : d.x, col < 3 ? e.y : d.y, col < 3 ? e.z : d.z}, quat(c.qT)), c.ih);
+      if (col < 3) {
+        k.m[col] = (float)l.x;
+        k.m[3 + col] = (float)l.y;
+        k.m[6 + col] = (float)l.z;
+      } else {
+        k.t[0] = (float)l.x + k.centre[0];
+        k.t[1] = (float)l.y + k.centre[1];
+        k.t[2] = (float)l.z + k.centre[2];
+      }
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  if (active && total > 0 && total <= kGroupHits)
-    for (int h = gl; h < total; h += 16)
-      stageHit(X.hitGeom + 8 * (size_t)(gbase + h), {ws.pc[0][grp][h], ws.pc[1][grp][h], ws.pc[2][grp][h]},
-               {ws.nrm[0][grp][h], ws.nrm[1][grp][h], ws.nrm[2][grp][h]}, ws.ov[grp][h], ws.node[grp][h]);
-  // more contacts than slots: the group's surviving chunks again, hits
-  // written in node order at the reserved range
-  const bool again = active && total > kGroupHits;
-  if (ballot64(again)) {
-    int running = 0;
-    for (unsigned long long rem = again ? live : 0ull; ballot64(rem != 0ull);) {
-      const int c = rem ? __builtin_ctzll(rem) : -1;
-      if (rem) rem &= rem - 1ull;
-#pragma unroll 1
-      for (int u = 0; u < 4; ++u) {
-        const int k = c * FDM_CHUNK + 16 * u + gl;
-        bool hit = false;
-        Sample sm;
+  auto identity = [](Q4 q) __attribute__((always_inline)) {
+    return q.q0 == 1.0 && q.q1 == 0.0 && q.q2 == 0.0 && q.q3 == 0.0;
+  };
+  // contact point, normal and overlap of a hit
+  auto contactOf = [&](V3 pn, const Sample& sm, int j, V3& pc, V3& nrm, double& ov) __attribute__((always_inline)) {
+    ov = -trilinear(sm.x, sm.y, sm.z, sm.c);
+    const V3 gr = gradientIntX(sm.x, sm.y, sm.z, sm.c);
+    const Q4 q = quat(ws.ctx[j].qT);
+    nrm = vnormalize(identity(q) ? gr : qrotate(q, gr));
+    pc = vadd(pn, vmul(nrm, 0.5 * ov));
+  };
+  // the exact predicate for node `id` of the run's pair j
+  auto exact = [&](int j, int id, V3& pn, Sample& sm) __attribute__((always_inline)) {
+    const PairCtx& c = ws.ctx[j];
+    const fdm_template* tp = tgeo.info + c.geoT;
+    const fdm_real* s = C.pgeo.nodes + 3 * ((size_t)ldu(&C.pgeo.info[c.geoA].nodeStart) + id);
+    pn = vadd(qrotate(quat(c.qA), {(double)s[0], (double)s[1], (double)s[2]}), {c.xA[0], c.xA[1], c.xA[2]});
+    Target tg;
+    tg.x = {c.xT[0], c.xT[1], c.xT[2]};
+    tg.q = quat(c.qT);
+    tg.ident = identity(tg.q);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      tg.t.origin[a] = ldu(&tp->origin[a]);
+      tg.t.size[a] = ldu(&tp->size[a]);
+    }
+    tg.t.invSpacing = ldu(&tp->invSpacing);
+    tg.t.sdfStart = ldu(&tp->sdfStart);
+    tg.t.affine = 0;
+    tg.sdf = tgeo.sdf;
+    tg.hash = c.hash;
+    const fdm_grid tgrid = targetGrid<SET, MANY>(C, S, c.inst);
+    return nodeHit<SET>(pn, tg, decodeHash(c.hash, tgrid), tgrid, ldu(&tp->radius), sm);
+  };
+
+  const float4* groups = reinterpret_cast<const float4*>(C.pgeo.groups);
+  const float4* nodes = reinterpret_cast<const float4*>(C.pgeo.groupNodes);
+  const int sub = lane / kUnitLanes, sl = lane % kUnitLanes;
+  int iu = 0;                          // next unit
+  int nlive = 0, il = 0;               // surviving groups, and the next of them
+  int ncand = 0, nhit = 0;
+  while (true) {
+    // groups, while the list has room
+    while (iu < nUnits && nlive + 64 <= kLiveMax) {
+      bool live = false;
+      int code = 0;
+      if (iu + sub < nUnits) {
+        const int un = ws.unit[iu + sub];
+        const CullRec& k = ws.cull[un >> 8];
+        const int g = (un & 0xFF) * kUnitLanes + sl;
+        code = (un & 0xFF00) | g;
+        if (g < k.groupCount) live = ballMayTouch<SET>(k, tgeo.cells, groups[k.groupStart + g]);
+      }
+      iu += 64 / kUnitLanes;
+      const unsigned long long m = ballot64(live);
+      if (live) ws.live[nlive + __popcll(m & lt)] = (unsigned short)code;
+      nlive += __popcll(m);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    // nodes, until 64 are at hand
+    bool full = false;
+    while (il < nlive) {
+      bool cand = false;
+      int code = 0;
+      if (il + sub < nlive) {
+        const int lv = ws.live[il + sub];
+        const CullRec& k = ws.cull[lv >> 8];
+        const float4 s = nodes[FDM_GROUP * (size_t)(k.groupStart + (lv & 0xFF)) + sl];
+        const int id = __float_as_int(s.w);
+        code = (lv & 0xFF00) << 8 | id;
+        cand = id >= 0 && nodeMayTouch<SET>(k, tgeo.cells, s);
+      }
+      const unsigned long long m = ballot64(cand);
+      if (ncand + __popcll(m) > 64) {  // these groups again after the exact test
+        full = true;
+        break;
+      }
+      il += 64 / kUnitLanes;
+      if (cand) ws.cand[ncand + __popcll(m & lt)] = code;
+      ncand += __popcll(m);
+    }
+    if (!full) {
+      nlive = il = 0;
+      if (iu < nUnits) continue;
+    }
+    if (ncand > 0) {
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      bool hit = false;
+      Sample sm;
+      V3 pn = {0., 0., 0.};
+      int code = 0;
+      if (lane < ncand) {
+        code = ws.cand[lane];
+        hit = exact(code >> 16, code & 0xFFFF, pn, sm);
+      }
+      const unsigned long long m = ballot64(hit);
+      if (hit) {
+        const int slot = nhit + __popcll(m & lt);
+        if (slot < kMaxHits) {
+          V3 pc, nrm;
+          double ov;
+          contactOf(pn, sm, code >> 16, pc, nrm, ov);
+          ws.pc[0][slot] = pc.x;
+          ws.pc[1][slot] = pc.y;
+          ws.pc[2][slot] = pc.z;
+          ws.nrm[0][slot] = nrm.x;
+          ws.nrm[1][slot] = nrm.y;
+          ws.nrm[2][slot] = nrm.z;
+          ws.ov[slot] = ov;
+          ws.hit[slot] = code;
+        }
+        atomicAdd(&ws.total[code >> 16], 1);
+        atomicOr(&ws.chunks[code >> 16], 1ull << ((code & 0xFFFF) / FDM_CHUNK));
+      }
+      nhit += __popcll(m);
+      ncand = 0;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+    if (!full) break;
+  }
+
+  // the record and staging reservations and the mirror slots, one pair per
+  // lane, their atomics issued together (one round trip instead of three)
+  const bool open = units > 0;
+  int total = open ? ws.total[lane] : 0;
+  if (open && total == 0) emptyRange();
+  if (nhit == 0) return;
+  const int pool = w % FDM_REC_POOLS;
+  const bool mirrored = SET != FDM_SET_WALL && total > 0 && T != A;
+  int base = 0, gbase = 0, mpos = 0;
+  const bool has = total > 0;
+  if (has) {
+    base = atomicAdd(S.pairs.recTotal + pool * FDM_REC_STRIDE, total);
+    gbase = atomicAdd(X.hitCount + pool * FDM_REC_STRIDE, total);
+    if (mirrored) mpos = atomicAdd(&S.mirror.count[T], 1);
+    // the previous step's record range of the pair, for the law's header
+    if (X.lawHead && prevCnt < 0) prevCnt = findPrevPair(S, p, A, T, prevOff);
+    const int rCap = S.pairs.recCapacity / FDM_REC_POOLS, gCap = X.hitCapacity / FDM_REC_POOLS;
+    if (base + total > rCap || gbase + total > gCap) {
+      atomicOr(C.status, base + total > rCap ? FDM_STATUS_RECORD_OVERFLOW : FDM_STATUS_STAGING_OVERFLOW);
+      total = base = gbase = 0;
+    } else {
+      base += pool * rCap;
+      gbase += pool * gCap;
+    }
+    ws.gbase[lane] = total > 0 ? gbase : -1;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  if (nhit <= kMaxHits) {
+    // a contact's place: the contacts of its pair at lower nodes come first
+    const int code = lane < nhit ? ws.hit[lane] : INT_MAX;
+    int at = 0;
+    for (int h = 0; h < nhit; ++h) {
+      const int c = readlaneI(code, h);
+      at += (c >> 16) == (code >> 16) && c < code ? 1 : 0;
+    }
+    const int gb = lane < nhit ? ws.gbase[code >> 16] : -1;
+    if (gb >= 0)
+      stageHit(X.hitGeom + 8 * (size_t)(gb + at), {ws.pc[0][lane], ws.pc[1][lane], ws.pc[2][lane]},
+               {ws.nrm[0][lane], ws.nrm[1][lane], ws.nrm[2][lane]}, ws.ov[lane], code & 0xFFFF);
+  } else {
+    // more contacts than slots: each pair's chunks with contacts again, in
+    // node order
+    for (int j = 0; j < np; ++j) {
+      if (readlaneI(total, j) <= 0) continue;
+      int run = readlaneI(gbase, j);
+      const int count = ldu(&C.pgeo.info[ws.ctx[j].geoA].nodeCount);
+      for (unsigned long long cm = ws.chunks[j]; cm; cm &= cm - 1ull) {
+        const int id = __builtin_ctzll(cm) * FDM_CHUNK + lane;
         V3 pn = {0., 0., 0.};
-        if (c >= 0 && k < nodeCount) {
-          const V3 sn = loadNode(k);
-          if (candidate(k, sn)) {
-            pn = vadd(qrotate(qA, sn), xA);
-            hit = nodeHit<FDM_SET_WALL>(pn, tg, tcell, tgrid, RB, sm);
-          }
-        }
-        const unsigned mh = groupBits(ballot64(hit));
+        Sample sm;
+        const bool hit = id < count && exact(j, id, pn, sm);
+        const unsigned long long m = ballot64(hit);
         if (hit) {
-          const double ov = -trilinear(sm.x, sm.y, sm.z, sm.c);
-          const V3 nrm = vnormalize(toWorld(gradientIntX(sm.x, sm.y, sm.z, sm.c), tg));
-          const V3 pc = vadd(pn, vmul(nrm, 0.5 * ov));
-          stageHit(X.hitGeom + 8 * (size_t)(gbase + running + __popc(mh & below)), pc, nrm, ov, k);
+          V3 pc, nrm;
+          double ov;
+          contactOf(pn, sm, j, pc, nrm, ov);
+          stageHit(X.hitGeom + 8 * (size_t)(run + __popcll(m & lt)), pc, nrm, ov, id);
         }
-        running += __popc(mh);
+        run += __popcll(m);
       }
     }
   }
-  if (active && gl == 0) {
-    S.pairs.recOff[p] = base;
-    S.pairs.recCnt[p] = total;
-    X.workHit[w] = gbase;
+  if (!has) return;
+  S.pairs.recOff[p] = base;
+  S.pairs.recCnt[p] = total;
+  X.workHit[w] = gbase;
+  if (X.lawHead) {
     int4* h = reinterpret_cast<int4*>(X.lawHead + 8 * (size_t)w);
     h[0] = make_int4(total, base, gbase, A);
     if (total > 0) h[1] = make_int4(T, prevOff, prevCnt, 0);
+  }
+  // (a pair whose reservation overflowed keeps its mirror slot, with no
+  // records and zero sums: the slot count and the list agree, and the
+  // target's fold adds nothing stale)
+  if (mirrored) {
+    if (mpos < S.mirror.capacity) S.mirror.list[(size_t)T * S.mirror.capacity + mpos] = p;
+    else atomicOr(C.status, FDM_STATUS_BUCKET_OVERFLOW);
+    if (total == 0)
+      for (int c = 0; c < 3; ++c) {
+        S.pairs.sumF[3 * (size_t)p + c] = 0.;
+        S.pairs.sumTB[3 * (size_t)p + c] = 0.;
+      }
   }
 }
 
@@ -1633,119 +1507,61 @@ __device__ __forceinline__ SetStarts setStarts(const NarrowMulti& a) {
   return st;
 }
 
-// The pre-cull and the sweep in one pass: one wave per candidate pair (WAVES
-// waves per workgroup). The wave takes the pre-cull's test itself (its
-// values are wave-uniform) and sweeps the pair only when it is kept; a culled
-// pair gets empty record ranges. No work list: the candidate index is the
-// work item.
-// Four waves per SIMD (at most 128 VGPRs): the sweep waits on memory for
-// most of its life, so the occupancy that hides that wait matters more than
-// the few registers the collecting mode then spills.
-template <int WAVES, int NPL>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4, 4)))
-kCullSweep(NarrowMulti a, NarrowScratch x) {
-  if (gateOff(a.gate)) return;
-  __shared__ HitSlots slots[WAVES];
-  __shared__ CandSlots cands[NPL == 3 ? WAVES : 1];
+// The sweep over the candidate pairs of every set: runs of pairs of one set
+// per wave (sweepRun), persistent waves, no work list. One wave per workgroup
+// (waves share nothing). Runs are as long as still gives every resident wave
+// one (up to 1.5 for pairs of two, 2 for four): a short list is bound by the
+// latency of one run, a long one by the instructions, which a run's pairs
+// share.
+//
+// Work assignment: workgroups are dealt to the eight XCDs in turn (workgroup
+// b runs on XCD b mod 8), each XCD with an L2 of its own, and neighbouring
+// candidates share bodies, templates and list lines: so each XCD takes
+// stretches of 64 consecutive pairs (stretch q on XCD q mod 8), its waves
+// sharing out its runs. Items are taken from the end: the image sets (whose
+// box test lets many pairs through) before the wall and particle sets.
+template <bool MANY>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+kSweep(NarrowMulti a, NarrowScratch x) {
+  __shared__ SweepSlots slots;
   const int lane = laneId();
-  const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int on = gateValue(a.gate, a.s[0].pairs.total);
   const SetStarts st = setStarts(a);
-  const int total = st.v[kMaxSets];
-  // Work assignment. Workgroups are dealt to the eight XCDs in turn
-  // (workgroup b runs on XCD b mod 8), each XCD with an L2 of its own, and
-  // neighbouring candidates share bodies, templates and list lines: so each
-  // XCD takes runs of 64 consecutive candidates (run q on XCD q mod 8), its
-  // waves sharing out its runs. Candidates are taken from the end of the
-  // index space: the ghost sets (image pairs, whose spheres hold many nodes)
-  // before the wall set, so that the cheap wall pairs fill the last round.
-  // (a set swept by kWallGroups is left out of the index space)
-  int ws0 = 0, nWall = 0;
+  asm volatile("" ::"s"(on), "s"(st.v[kMaxSets]));  // (loaded together)
+  if (!on) return;
+  int shift = 0;  // log2 of the pairs of a run
+  while ((1 << shift) < kRunMax &&
+         (st.v[kMaxSets] >> shift) > (int)gridDim.x + ((int)gridDim.x >> 1) * shift)
+    ++shift;
+  const int run = 1 << shift;
+  int item[kMaxSets + 1];  // first item of each set
+  item[0] = 0;
 #pragma unroll
-  for (int q = 0; q < kMaxSets; ++q)
-    if (q == a.wallSet) {
-      ws0 = st.v[q];
-      nWall = st.v[q + 1] - st.v[q];
-    }
-  const int nOther = total - nWall;
-  const bool byXcd = gridDim.x % kXcds == 0;
-  const int xcd = byXcd ? blockIdx.x % kXcds : 0;
-  const int stride = byXcd ? gridDim.x / kXcds * WAVES : gridDim.x * WAVES;
-  for (int i = (byXcd ? blockIdx.x / kXcds : blockIdx.x) * WAVES + wave;; i += stride) {
-    const int r = byXcd ? ((i >> 6) * kXcds + xcd) * 64 + (i & 63) : i;
-    if (r >= nOther) break;
-    const int go = nOther - 1 - r;
-    const int g = go < ws0 ? go : go + nWall;
-    int k = 0, base = 0;
-#pragma unroll
-    for (int q = 1; q < kMaxSets; ++q)  // constant indices: the starts stay scalar
-      if (g >= st.v[q]) {
-        k = q;
-        base = st.v[q];
-      }
-    const NarrowSet& s = a.s[k];
-    const int p = g - base;
-    if (s.pairs.pairA[p] < 0) {  // an empty slot of an overflowing list
-      if (lane == 0) {
-        s.pairs.recOff[p] = 0;
-        s.pairs.recCnt[p] = 0;
-        if (x.lawHead) *reinterpret_cast<int4*>(x.lawHead + 8 * (size_t)g) = make_int4(0, 0, 0, 0);
-      }
-      continue;
-    }
-    const int pool = g % FDM_REC_POOLS;
-    CandSlots* cs = NPL == 3 ? &cands[wave] : nullptr;
-    if (s.kind == FDM_SET_PARTICLE)
-      sweepPair<FDM_SET_PARTICLE, true, NPL>(a.c, s, x, g, p, lane, slots[wave], pool, cs);
-    else if (s.kind == FDM_SET_WALL)
-      sweepPair<FDM_SET_WALL, true, NPL>(a.c, s, x, g, p, lane, slots[wave], pool, cs);
-    else
-      sweepPair<FDM_SET_GHOST, true, NPL>(a.c, s, x, g, p, lane, slots[wave], pool, cs);
-  }
-}
-
-// The wall set's pairs four per wave (sweepWallGroup) for the one-node-per-
-// lane sweep, launched before kCullSweep, which then leaves the wall set
-// out. One wave per workgroup; runs of 16 groups (64 consecutive pairs) per
-// XCD as in kCullSweep. A group of four whose pairs do not share the target
-// and system is swept one pair at a time (the same code with one group of
-// lanes taking part).
-__global__ void __launch_bounds__(64) kWallGroups(NarrowMulti a, NarrowScratch x) {
-  if (gateOff(a.gate)) return;
-  __shared__ WallGroupSlots groups;
-  const int lane = laneId();
-  const SetStarts st = setStarts(a);
-  int k = 0, ws0 = 0, nWall = 0;
-#pragma unroll
-  for (int q = 0; q < kMaxSets; ++q)  // constant indices: the starts stay scalar
-    if (q == a.wallSet) {
-      k = q;
-      ws0 = st.v[q];
-      nWall = st.v[q + 1] - st.v[q];
-    }
-  const NarrowSet& S = a.s[k];
-  const NarrowCommon& C = a.c;
-  const int items = (nWall + 3) / 4;
+  for (int q = 0; q < kMaxSets; ++q) item[q + 1] = item[q] + ((st.v[q + 1] - st.v[q] + run - 1) >> shift);
+  const int items = item[kMaxSets];
   const bool byXcd = gridDim.x % kXcds == 0;
   const int xcd = byXcd ? blockIdx.x % kXcds : 0;
   const int stride = byXcd ? gridDim.x / kXcds : gridDim.x;
+  const int stretch = 6 - shift;  // log2 of the runs of a stretch
   for (int i = byXcd ? blockIdx.x / kXcds : blockIdx.x;; i += stride) {
-    const int r = byXcd ? ((i >> 4) * kXcds + xcd) * 16 + (i & 15) : i;
+    const int r = byXcd ? ((((i >> stretch) * kXcds) + xcd) << stretch) + (i & ((1 << stretch) - 1)) : i;
     if (r >= items) break;
-    const int p = 4 * r + (lane >> 4);
-    const bool in = p < nWall;
-    const int A = in ? ldu(S.pairs.pairA + p) : -1;
-    const int T = in ? ldu(S.pairs.pairT + p) : 0;
-    const bool live = A >= 0;
-    const int inst = live && C.inst.count > 0 ? ldu(C.inst.particleInstance + A) : 0;
-    const unsigned long long act = ballot64(live);
-    bool uniform = true;
-    if (act) {
-      const int ref = __builtin_ctzll(act);
-      uniform = !ballot64(live && (T != readlaneI(T, ref) || inst != readlaneI(inst, ref)));
-    }
-    const int passes = uniform ? 1 : 4;
-    for (int it = 0; it < passes; ++it)
-      sweepWallGroup(C, S, x, ws0, nWall, r, uniform ? 0xFu : (1u << it), lane, groups);
+    const int it = items - 1 - r;
+    int k = 0, i0 = 0, g0 = 0, np = st.v[1];
+#pragma unroll
+    for (int q = 1; q < kMaxSets; ++q)  // constant indices: the starts stay scalar
+      if (it >= item[q]) {
+        k = q;
+        i0 = item[q];
+        g0 = st.v[q];
+        np = st.v[q + 1] - st.v[q];
+      }
+    const NarrowSet& s = a.s[k];
+    const int p0 = (it - i0) << shift;
+    const int len = min(run, np - p0);
+    if (s.kind == FDM_SET_PARTICLE) sweepRun<FDM_SET_PARTICLE, MANY>(a.c, s, x, g0 + p0, p0, len, lane, slots);
+    else if (s.kind == FDM_SET_WALL) sweepRun<FDM_SET_WALL, MANY>(a.c, s, x, g0 + p0, p0, len, lane, slots);
+    else sweepRun<FDM_SET_GHOST, MANY>(a.c, s, x, g0 + p0, p0, len, lane, slots);
   }
 }
 
@@ -1784,9 +1600,11 @@ __global__ void __launch_bounds__(64 * WAVES) kCullSweepLaw(NarrowMulti a) {
 // The contact law over the candidate index space of kCullSweep (one thread
 // per candidate; culled pairs and pairs without contacts return at once).
 __global__ void __launch_bounds__(256) kContactLawAll(NarrowMulti a, NarrowScratch x) {
-  if (gateOff(a.gate)) return;
+  const int on = gateValue(a.gate, a.s[0].pairs.total);
   const SetStarts st = setStarts(a);
   const int total = st.v[kMaxSets];
+  asm volatile("" ::"s"(on), "s"(total));  // (loaded together)
+  if (!on) return;
   for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
     int k = 0, base = 0;
 #pragma unroll
@@ -1811,7 +1629,7 @@ __global__ void kResetCounter(int* c) {
 
 namespace fdm {
 namespace {
-fdm_tuning g_tuning = {1, 32, 256, 256, 1, 1, 0};
+fdm_tuning g_tuning = {1, 16, 256, 256, 1, 1, 0};
 }
 const fdm_tuning& tuning() { return g_tuning; }
 }  // namespace fdm
@@ -2030,26 +1848,11 @@ extern "C" int fdm_launchNarrowPhaseSets(const fdm_narrowphase_args* sets, int n
   x.hitCount = ws->hitCount;
   fdm_tuning tu = tuning();
   if (ws->tuning && !completeTuning(*ws->tuning, tu)) return FDM_EINVAL;
-  // The wall set four pairs per wave (one node per lane, law in its own
-  // kernel): by default for wall sets sized for at least kGroupedWallPairs
-  // pairs, as a small system's step is bound by launch latency, which a
-  // second sweep kernel would add to. The grid covers the set's capacity in
-  // groups.
-  k.wallSet = -1;
-  int wallGroups = 0;
-  if (tu.lawMode == 1 && tu.nodesPerLane == 1 && x.lawHead)
-    for (int i = 0; i < nsets && k.wallSet < 0; ++i)
-      if (sets[i].set == FDM_SET_WALL && tu.wallGroups != 2 &&
-          (tu.wallGroups == 1 || sets[i].pairs.capacity >= kGroupedWallPairs)) {
-        k.wallSet = i;
-        wallGroups = (sets[i].pairs.capacity + 3) / 4;
-      }
+  // geometry without the culling tables of sweepPair: the kernel that culls
+  // by chunk
+  const fdm_geometry& pg = sets[0].pgeo;
+  if (!pg.groups || !pg.groupNodes || !pg.cells || (sets[0].wgeo.num > 0 && !sets[0].wgeo.cells)) tu.lawMode = 2;
   const int sweepBlocks = std::max(1, persistentBlocks(tu.sweepWaves) * tu.sweepWavesPerCU / 32);
-  if (k.wallSet >= 0) {
-    const int blocks = std::min(persistentBlocks(1) * 12 / 32, wallGroups);
-    hipLaunchKernelGGL(kWallGroups, dim3(std::max(kXcds, blocks / kXcds * kXcds)), dim3(64), 0, stream,
-                       k, x);
-  }
   if (tu.lawMode == 2) {
     if (tu.sweepWaves == 4)
       hipLaunchKernelGGL(kCullSweepLaw<4>, dim3(sweepBlocks), dim3(256), 0, stream, k);
@@ -2059,27 +1862,9 @@ extern "C" int fdm_launchNarrowPhaseSets(const fdm_narrowphase_args* sets, int n
       hipLaunchKernelGGL(kCullSweepLaw<1>, dim3(sweepBlocks), dim3(64), 0, stream, k);
     return launchStatus();
   }
-  if (tu.nodesPerLane == 3) {
-    if (tu.sweepWaves == 4)
-      hipLaunchKernelGGL((kCullSweep<4, 3>), dim3(sweepBlocks), dim3(256), 0, stream, k, x);
-    else if (tu.sweepWaves == 2)
-      hipLaunchKernelGGL((kCullSweep<2, 3>), dim3(sweepBlocks), dim3(128), 0, stream, k, x);
-    else
-      hipLaunchKernelGGL((kCullSweep<1, 3>), dim3(sweepBlocks), dim3(64), 0, stream, k, x);
-  } else if (tu.nodesPerLane == 2) {
-    if (tu.sweepWaves == 4)
-      hipLaunchKernelGGL((kCullSweep<4, 2>), dim3(sweepBlocks), dim3(256), 0, stream, k, x);
-    else if (tu.sweepWaves == 2)
-      hipLaunchKernelGGL((kCullSweep<2, 2>), dim3(sweepBlocks), dim3(128), 0, stream, k, x);
-    else
-      hipLaunchKernelGGL((kCullSweep<1, 2>), dim3(sweepBlocks), dim3(64), 0, stream, k, x);
-  } else if (tu.sweepWaves == 4) {
-    hipLaunchKernelGGL((kCullSweep<4, 1>), dim3(sweepBlocks), dim3(256), 0, stream, k, x);
-  } else if (tu.sweepWaves == 2) {
-    hipLaunchKernelGGL((kCullSweep<2, 1>), dim3(sweepBlocks), dim3(128), 0, stream, k, x);
-  } else {
-    hipLaunchKernelGGL((kCullSweep<1, 1>), dim3(sweepBlocks), dim3(64), 0, stream, k, x);
-  }
+  const int waves = std::max(kXcds, persistentBlocks(1) * tu.sweepWavesPerCU / 32 / kXcds * kXcds);
+  if (sets[0].inst.count > 0) hipLaunchKernelGGL(kSweep<true>, dim3(waves), dim3(64), 0, stream, k, x);
+  else hipLaunchKernelGGL(kSweep<false>, dim3(waves), dim3(64), 0, stream, k, x);
   hipLaunchKernelGGL(kContactLawAll, dim3(persistentBlocks(tu.lawBlock / 64)), dim3(tu.lawBlock), 0,
                      stream, k, x);
   return launchStatus();

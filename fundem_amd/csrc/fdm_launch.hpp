@@ -47,6 +47,13 @@ const fdm_tuning& tuning();
 // the flag is null or *flag != 0. Steps captured in a graph launch every
 // kernel; gates let the device skip work it decided is not needed.
 __device__ __forceinline__ bool gateOff(const int* gate) { return gate && *gate == 0; }
+// The flag's value loaded without a branch on the gate (`any`: some readable
+// word, read when there is no gate), so that it goes along with the loads
+// around it; off when the result is zero.
+__device__ __forceinline__ int gateValue(const int* gate, const int* any) {
+  const int v = *(gate ? gate : any);
+  return gate ? v : 1;
+}
 
 // Device-wide scans over ints (sort.hip). out may alias in.
 size_t scanWorkspace(size_t n);

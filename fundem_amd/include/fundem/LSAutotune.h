@@ -22,11 +22,9 @@
 //     each step by their own cell rule), nor for batched systems (their
 //     packings are configured with cells below twice the largest radius: a
 //     coarser candidate changed their contacts and overflowed a mirror list);
-//   - the solver's launch shapes (fdm_tuning): node-sweep waves (kept pairs
-//     in flight) per workgroup and sweep grid size, nodes per lane (64 or
-//     128 nodes in flight per sweep wave), where the contact law runs (a
-//     kernel of its own, or the sweep's wave), contact-law and reduction
-//     workgroup sizes.
+//   - the solver's launch shapes (fdm_tuning): sweep grid size, where the
+//     contact law runs (a kernel of its own, or the sweep's wave),
+//     contact-law and reduction workgroup sizes.
 // Each candidate is timed from the same saved point (LSAdjoint::mark /
 // rollback) one knob at a time, keeping the best value of each knob before
 // the next; the solver is left at the saved point with the best settings.
@@ -101,13 +99,11 @@ class LSAutotuner {
       bestCost = pick(group, window, best, "cell");
     }
     group.clear();
-    for (int w : {1, 2, 4})
-      for (int pc : {16, 32, 64}) {
-        TuneChoice c = best;
-        c.launch.sweepWaves = w;
-        c.launch.sweepWavesPerCU = pc;
-        group.push_back(c);
-      }
+    for (int pc : {8, 16, 32}) {
+      TuneChoice c = best;
+      c.launch.sweepWavesPerCU = pc;
+      group.push_back(c);
+    }
     bestCost = pick(group, trialSteps, best, "sweep");
     group.clear();
     for (int m : {1, 2}) {
@@ -117,15 +113,6 @@ class LSAutotuner {
     }
     bestCost = pick(group, trialSteps, best, "lawMode");
     group.clear();
-    if (best.launch.lawMode == 1) {
-      for (int npl : {1, 2, 3}) {
-        TuneChoice c = best;
-        c.launch.nodesPerLane = npl;
-        group.push_back(c);
-      }
-      bestCost = pick(group, trialSteps, best, "nodesPerLane");
-      group.clear();
-    }
     for (int b : {64, 128, 256}) {
       TuneChoice c = best;
       c.launch.lawBlock = b;

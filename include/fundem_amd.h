@@ -107,7 +107,19 @@ typedef struct {
                             plane[3] + plane[0..2] . l - planeSlack (culling only) */
   double plane[4];
   double planeSlack;
+  long long cellStart;   /* offset into the cell codes (fdm_geometry.cells) */
+  int groupStart;        /* first node group (fdm_geometry.groups) */
+  int groupCount;
 } fdm_template;
+
+/* Node groups: the surface nodes of a template regrouped into compact runs
+ * of FDM_GROUP (culling only; node ids are unchanged). */
+#define FDM_GROUP 16
+/* Cell codes per cell spacing: code c >= 1 of an SDF cell says that every
+ * cell in which the trilinear phi can be <= 0 is at least (c - 1) /
+ * FDM_CELL_UNIT spacings away from every point of the cell; 0 that phi can
+ * be <= 0 in the cell itself. */
+#define FDM_CELL_UNIT 15
 
 /* One material (materialInfo, LSParticle.h:12-51) after the clamps of
  * LSParticle::addMaterial; dissipation = -ln e / sqrtf(ln^2 e + pi^2) as
@@ -140,6 +152,11 @@ typedef struct {
   const float* sdf;
   const fdm_real* nodes; /* xyz triples after the centroid shift */
   const float* chunks;   /* float4 per chunk */
+  /* Culling tables of the several-set sweep; all NULL: the sweep culls by
+   * chunk (fdm_tuning.lawMode 2's kernel). */
+  const float* groups;        /* float4 per node group: centre xyz, enclosing radius */
+  const float* groupNodes;    /* float4 per group slot: node xyz (FP32), node id bits (-1: none) */
+  const unsigned char* cells; /* code of every SDF cell, (size-1) per axis, x fastest */
 } fdm_geometry;
 
 /* Uniform grid parameters (spatialGrid, myUtility/mySpatialGrid.h:162-256). */
@@ -598,14 +615,16 @@ typedef struct {
 } fdm_narrow_workspace;
 /* No counterpart in the reference: the narrow phase of up to five sets at
  * once, in two kernels over the candidate pairs of all sets (set k's pairs
- * follow those of sets 0..k-1). The first (one wave per candidate pair)
- * tests whether the pair's bodies can still touch at this step's positions
- * (the broad-phase tests without the skin), gives a rejected pair empty
- * record ranges, and otherwise sweeps the surface nodes, stages every
- * contact's point, normal and overlap in hitGeom and reserves the pair's
- * records; the second (one thread per candidate pair) applies the contact
- * law to the staged contacts in node order and writes the records and the
- * pair sums. Shared fields (bodies, geometry, materials, pgrid, periodic,
+ * follow those of sets 0..k-1). The first (runs of one to eight pairs per
+ * wave) tests whether the pairs' bodies can still touch at this step's
+ * positions (the broad-phase tests without the skin), gives a rejected pair
+ * empty record ranges, and otherwise culls node groups and nodes against the
+ * target's cell codes, tests the rest exactly, stages every contact's point,
+ * normal and overlap in hitGeom and reserves the pair's records; the second
+ * (one thread per candidate pair) applies the contact law to the staged
+ * contacts in node order and writes the records and the pair sums. Geometry
+ * without the culling tables (fdm_geometry.groups, groupNodes, cells) runs
+ * as lawMode 2. Shared fields (bodies, geometry, materials, pgrid, periodic,
  * dt, updateSprings, status, dbg*) come from sets[0]. Unlike
  * fdm_launchNarrowPhase it clears no counter: the sets' record counters
  * (pairs.recTotal) and the hitCount pools must be zero at launch. Candidate
@@ -663,21 +682,19 @@ int fdm_fillInt(int* ptr, size_t n, int value, hipStream_t stream);
  * default and validates them. Graphs captured before a change keep the shapes
  * they were captured with. */
 typedef struct fdm_tuning_s {
-  int sweepWaves;       /* node-sweep waves (kept pairs in flight) per workgroup: 1, 2 or 4 */
-  int sweepWavesPerCU;  /* node-sweep grid size, in waves per CU: 4..128 (default 32) */
+  int sweepWaves;       /* node-sweep waves per workgroup: 1, 2 or 4 (lawMode 2; lawMode 1's
+                           sweep has one wave per workgroup) */
+  int sweepWavesPerCU;  /* node-sweep grid size, in waves per CU: 4..128 (default 16, as many
+                           as lawMode 1's sweep keeps resident) */
   int lawBlock;         /* contact-law threads per workgroup: 64, 128 or 256 */
   int reduceBlock;      /* reduction threads per workgroup: a multiple of 64 up to 1024 */
   int lawMode;          /* contact law of the narrow phase: 1 in a kernel of its own (one
                            thread per candidate pair, contacts staged in the workspace),
                            2 in the sweep's wave (one contact per lane) */
-  int nodesPerLane;     /* how a sweep wave walks a pair's surviving 64-node chunks: 1 one
-                           chunk per iteration (one node per lane), 2 two chunks per
-                           iteration (128 nodes in flight), 3 the nodes that pass the tests
-                           before the SDF fetch collected first, then up to 64 of their SDF
-                           cells fetched at once; lawMode 1 only */
-  int wallGroups;       /* wall pairs four per wave in a kernel of their own (nodesPerLane 1,
-                           lawMode 1): 0 automatic (wall sets sized for at least 65536
-                           pairs), 1 always, 2 never */
+  int nodesPerLane;     /* 1, 2 or 3: accepted, without effect (every sweep collects the
+                           nodes that pass the cell test before it fetches SDF values) */
+  int wallGroups;       /* 0, 1 or 2: accepted, without effect (every set is swept several
+                           pairs per wave) */
 } fdm_tuning;
 int fdm_setTuning(const fdm_tuning* t);
 void fdm_getTuning(fdm_tuning* t);
