@@ -5,6 +5,7 @@
 
 #include "fdm_device.hpp"
 #include "fdm_launch.hpp"
+#include "step_device.hpp"
 
 namespace fdm {
 
@@ -126,168 +127,63 @@ __global__ void kCommitStateInstances(const double* x, int n, fdm_instances I, i
   }
 }
 
-// Rebuild decision of one step (one thread). The displacement bound grows by
-// dt times the largest motion rate, plus 1e-6 rho per step for the rounding
-// of orientations to FP32 (a relative 2^-24 per component moves a point at
-// distance rho by well under 1e-6 rho). Ghost lists are also rebuilt after
-// a visibility change or a wrap; a wrap (positions jump by a period)
-// rebuilds the next step's lists as well. One thread of one workgroup runs
-// it, after every other writer of the control words has finished (earlier
-// kernels of the stream); `rate` and `flags` (bit 0 grid state changed, 1
-// visibility changed, 2 wrapped) add this kernel's own findings. The control
-// words are read together (plain loads: the cache is fresh at kernel start),
-// and the host's copy of the decision is one word, (number << 2) | rebuild
-// << 1 | ghost rebuild, so it needs no ordering fence.
-__device__ void decideStep(const fdm_skin& s, float rateIn, int flagsIn) {
-  int* c = s.ctl;
-  int w[FDM_CTL_WORDS];
-#pragma unroll
-  for (int k = 0; k < FDM_CTL_WORDS; ++k) w[k] = c[k];
-  const double disp = *s.disp;
-  const float rate = fmaxf(__int_as_float(w[FDM_CTL_MAX_RATE]), rateIn);
-  double d = disp + s.dt * (double)rate * (1.0 + 1e-6) + 1e-6 * s.rhoMax;
-  const bool rebuild = w[FDM_CTL_FORCE] != 0 || w[FDM_CTL_PENDING] != 0 ||
-                       w[FDM_CTL_VALID_CHANGED] != 0 || (flagsIn & 1) || !(2.0 * d <= s.skin);
-  const bool wrapped = w[FDM_CTL_WRAPPED] != 0 || (flagsIn & 4);
-  const bool ghost = rebuild || wrapped || w[FDM_CTL_GHOST_CHANGED] != 0 || (flagsIn & 2);
-  if (rebuild) {
-    d = 0.0;
-    c[FDM_CTL_COUNT] = w[FDM_CTL_COUNT] + 1;
-  }
-  if (ghost) c[FDM_CTL_GHOST_COUNT] = w[FDM_CTL_GHOST_COUNT] + 1;
-  *s.disp = d;
-  c[FDM_CTL_REBUILD] = rebuild ? 1 : 0;
-  c[FDM_CTL_REBUILD_GHOST] = ghost ? 1 : 0;
-  c[FDM_CTL_KEEP] = (rebuild || ghost) ? 0 : 1;
-  c[FDM_CTL_PENDING] = wrapped ? 1 : 0;
-  c[FDM_CTL_MAX_RATE] = 0;
-  c[FDM_CTL_FORCE] = 0;
-  c[FDM_CTL_VALID_CHANGED] = 0;
-  c[FDM_CTL_WRAPPED] = 0;
-  c[FDM_CTL_GHOST_CHANGED] = 0;
-  const int seq = w[FDM_CTL_SEQ] + 1;
-  c[FDM_CTL_SEQ] = seq;
-  if (s.hostDecision)
-    *(volatile int*)(s.hostDecision + (seq & (FDM_DECISION_RING - 1))) =
-        (int)(((unsigned)seq << 2) | (rebuild ? 2u : 0u) | (ghost ? 1u : 0u));
-}
-
 __global__ void kSkinDecide(fdm_skin s) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   decideStep(s, 0.f, 0);
 }
 
-struct StepBeginK {
-  fdm_step_begin_args a;
-  fdm_skin s;
-  float* blockRate;  // [gridDim.x] largest motion rate of each workgroup
-  int* blockFlags;   // [gridDim.x] bit 0 grid state changed, 1 visibility changed, 2 wrapped
-};
-
-// Phase A of a step (one thread per particle, then per wall). Each workgroup
-// leaves its largest motion rate and its change flags in a slot of its own
-// (no atomics on shared words); kStepDecide folds the slots.
-// One body of phase A. Everything it reads from the launch arguments is
-// copied into registers first (selecting between argument structs by
-// reference would make the compiler copy them to per-lane scratch).
-// MANY: bodies of several systems (per-body grids and periodic flags); the
-// single-system kernel holds its grid in scalar registers.
-template <bool WALL, bool MANY>
-__device__ __forceinline__ void stepBeginBody(const fdm_step_begin_args& a, int j, float& rate,
-                                              int& flags) {
-  const fdm_bodies b = WALL ? a.walls : a.particles;
-  const fdm_template* tmpl = WALL ? a.wgeo.info : a.pgeo.info;
-  const fdm_hash_table t = WALL ? a.wtable : a.ptable;
-  const bool many = MANY;
-  const int in = !many ? 0 : (WALL ? a.inst.wallInstance[j] : a.inst.particleInstance[j]);
-  const fdm_grid grid =
-      !many ? (WALL ? a.wgrid : a.pgrid) : (WALL ? a.inst.wgrid[in] : a.inst.pgrid[in]);
-  const fdm_periodic perI = many ? a.inst.periodic[in] : a.periodic;
-  const bool ghosts = !WALL && anyPeriodic(a.periodic);
-  const bool kick = !WALL && a.kick;
-  const int n = b.n;
-  // Every input is loaded before anything is stored: the arrays may alias as
-  // far as the compiler knows, so a load placed after a store could not be
-  // issued before it. One round of loads (the torque only where the spin
-  // changes), then the half-kick and the drift in registers with the
-  // roundings of the stored state (kickOne, driftOne), then the stores.
-  // (the stored FP32 values are held as loaded and widened where used)
-  const int geo = b.geo[j];
-  const V3 x0 = ldp(b.x, n, j);
-  R3 v = ld3s(b.v, n, j), w = ld3s(b.w, n, j);
-  const R4 q0 = ld4s(b.q, n, j);
-  R3 F = {0, 0, 0};
-  if (kick) F = ld3s(b.F, n, j);
-  const int atBuild = t.validAtBuild[j];
-  const int ghostAtBuild = ghosts ? a.ghostAtBuild[j] : 0;
-  const fdm_template& tp = tmpl[geo];
-  bool vNew = false, wNew = false;
-  if (kick && !nearZero(tp.invMass)) {
-    // particleVelocityAngularVelocityIntegrationKernel (particleIntegrationKernel.cu:3-32)
-    const double h = 0.5 * a.dt;
-    v = narrow3(vadd(wide(v), vmul(vadd(vmul(wide(F), tp.invMass), fromD3(a.gravity)), h)));
-    vNew = true;
-    if (!spinFixed(tp)) {
-      const V3 wd = wide(w);
-      const Q4 qd = wide(q0);
-      const V3 Iw = smul(srotate(qd, lds6(tp.inertia)), wd);
-      const V3 T = ld3(b.T, n, j);
-      w = narrow3(vadd(wd, vmul(smul(srotate(qd, lds6(tp.invInertia)), vsub(T, vcross(wd, Iw))), h)));
-      wNew = true;
-    }
-  }
-  V3 x = x0;
-  if (vNew) st3s(b.v, n, j, v);
-  if (wNew) st3s(b.w, n, j, w);
-  if (a.drift) {
-    // particlePositionOrientationIntegrationKernel (particleIntegrationKernel.cu:34-48)
-    x = vadd(x0, vmul(wide(v), a.dt));
-    stp(b.x, n, j, x);
-    st4(b.q, n, j, qintegrate(wide(q0), wide(w), a.dt));
-  }
-  t.hashValue[j] = cellHash(x, grid);
-  if (a.drift) {
-    const double rho = fmax(tp.radius, tp.boxReach);
-    const double r = vlen(wide(v)) + vlen(wide(w)) * rho;
-    rate = (float)r * (1.0f + 1e-6f);
-  }
-  const int st = bodyState(x, grid);
-  if (st == 2 || st != atBuild) flags |= 1;
-  if (ghosts) {
-    // sets exist where any instance is periodic; an instance contributes
-    // only to the sets of its own periodic axes
-    const int vb = visibilityBits(x, grid, a.periodic, perI);
-    const int bits = vb & 7;
-    for (int k = 0; k < 3; ++k)
-      if (a.ghostFlag[k]) a.ghostFlag[k][j] = (bits >> k) & 1;
-    if (bits != ghostAtBuild) flags |= 2;
-    if (vb & 8) flags |= 4;
-  }
-}
-
-template <bool MANY>
+// Phase A of a step (one thread per particle, then per wall). DECIDE: the
+// last workgroup takes the list decision (decideLast); otherwise each leaves
+// its largest motion rate and its change flags in a slot of its own for
+// kStepDecide.
+template <bool MANY, bool DECIDE>
 __global__ void __launch_bounds__(256) kStepBegin(StepBeginK k) {
   if (gateOff(k.a.gate)) return;
   const fdm_step_begin_args& a = k.a;
-  __shared__ float waveMax[4];
   const int nP = a.particles.n, nW = a.walls.n;
   float rate = 0.f;
   int flags = 0;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nP) stepBeginBody<false, MANY>(a, i, rate, flags);
   else if (i < nP + nW) stepBeginBody<true, MANY>(a, i - nP, rate, flags);
-  const int f1 = __syncthreads_or(flags & 1), f2 = __syncthreads_or(flags & 2),
-            f4 = __syncthreads_or(flags & 4);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) rate = fmaxf(rate, __shfl_xor(rate, off, 64));
-  if (laneId() == 0) waveMax[threadIdx.x >> 6] = rate;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float m = waveMax[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) m = fmaxf(m, waveMax[w]);
-    k.blockRate[blockIdx.x] = m;
-    k.blockFlags[blockIdx.x] = (f1 ? 1 : 0) | (f2 ? 2 : 0) | (f4 ? 4 : 0);
+  if (DECIDE) {
+    decideLast(k, rate, flags);
+  } else {
+    foldBlock(rate, flags);
+    if (threadIdx.x == 0) {
+      k.blockRate[blockIdx.x] = rate;
+      k.blockFlags[blockIdx.x] = flags;
+    }
   }
+}
+
+// The end of one step and the first phase of the next in one pass over the
+// bodies: fold, second half-kick, then first half-kick, drift, cell id, flags
+// and the next step's list decision. A body's state is read and written once
+// instead of twice, and its force and torque, which only the half-kicks use
+// between two steps, are not stored. Bound by the body state's bytes (some 210
+// read and written per particle) on many bodies and by its chain of loads on
+// few. Measured against a fold kernel, a step-begin kernel and a decision
+// kernel: 1e6 particles 23.5 + 38.9 + 5.7 -> 48.4 us, a whole step of one
+// particle 34.5 -> 30.7 us, of 64 packings (523K bodies) 146 -> 73 us, of 8192
+// bonded spheres 141 -> 82 us (the last two with the sweep in runs).
+template <bool MANY>
+__global__ void __launch_bounds__(256) kReduceStep(ReduceK r, StepBeginK k) {
+  if (gateOff(k.a.gate)) return;
+  const fdm_step_begin_args& a = k.a;
+  const int nP = a.particles.n, nW = a.walls.n;
+  float rate = 0.f;
+  int flags = 0;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0 && r.stepCounter) *r.stepCounter += 1;
+  if (i < nP) {
+    V3 F, T;
+    foldForces(r, i, F, T);
+    stepBeginBody<false, MANY, true>(a, i, rate, flags, narrow3(F), narrow3(T));
+  } else if (i < nP + nW) {
+    stepBeginBody<true, MANY>(a, i - nP, rate, flags);
+  }
+  decideLast(k, rate, flags);
 }
 
 // Clears the given counter arrays, folds the workgroup slots of kStepBegin
@@ -460,11 +356,14 @@ int stepBeginSetup(const fdm_step_begin_args* args, const fdm_skin* skin, void* 
     if (a.periodic.sector && (a.periodic.x || a.periodic.y || a.inst.count > 0)) return FDM_EINVAL;
   }
   const long long total = (long long)a.particles.n + a.walls.n;
-  if (workspaceBytes < fdm_stepBeginWorkspaceBytes((size_t)total)) return FDM_EINVAL;
   nb = std::max<unsigned>(1, blocksFor(total, 256));
-  Carve cv(workspace, workspaceBytes);
   k.a = a;
   k.s = *skin;
+  k.blockRate = nullptr;
+  k.blockFlags = nullptr;
+  if (!workspace) return skin->fold ? FDM_OK : FDM_EINVAL;  // (decided by the last workgroup)
+  if (workspaceBytes < fdm_stepBeginWorkspaceBytes((size_t)total)) return FDM_EINVAL;
+  Carve cv(workspace, workspaceBytes);
   k.blockRate = cv.take<float>(nb);
   k.blockFlags = cv.take<int>(nb);
   return cv.ok ? FDM_OK : FDM_EINVAL;
@@ -474,22 +373,54 @@ int stepBeginSetup(const fdm_step_begin_args* args, const fdm_skin* skin, void* 
 
 extern "C" int fdm_launchStepBegin(const fdm_step_begin_args* args, const fdm_skin* skin,
                                    void* workspace, size_t workspaceBytes, hipStream_t stream) {
+  if (!workspace) return FDM_EINVAL;
   StepBeginK k;
   unsigned nb = 0;
   const int r = stepBeginSetup(args, skin, workspace, workspaceBytes, k, nb);
   if (r != FDM_OK) return r;
-  if (args->inst.count > 0) hipLaunchKernelGGL(kStepBegin<true>, dim3(nb), dim3(256), 0, stream, k);
-  else hipLaunchKernelGGL(kStepBegin<false>, dim3(nb), dim3(256), 0, stream, k);
+  if (args->inst.count > 0) hipLaunchKernelGGL((kStepBegin<true, false>), dim3(nb), dim3(256), 0, stream, k);
+  else hipLaunchKernelGGL((kStepBegin<false, false>), dim3(nb), dim3(256), 0, stream, k);
   return launchStatus();
 }
 
 extern "C" int fdm_launchStepDecide(const fdm_step_begin_args* args, const fdm_skin* skin,
                                     void* workspace, size_t workspaceBytes, hipStream_t stream) {
+  if (!workspace) return FDM_EINVAL;
   StepBeginK k;
   unsigned nb = 0;
   const int r = stepBeginSetup(args, skin, workspace, workspaceBytes, k, nb);
   if (r != FDM_OK) return r;
   hipLaunchKernelGGL(kStepDecide, dim3(1), dim3(1024), 0, stream, k, (int)nb);
+  return launchStatus();
+}
+
+extern "C" int fdm_launchStepBeginDecide(const fdm_step_begin_args* args, const fdm_skin* skin,
+                                         hipStream_t stream) {
+  StepBeginK k;
+  unsigned nb = 0;
+  const int r = stepBeginSetup(args, skin, nullptr, 0, k, nb);
+  if (r != FDM_OK) return r;
+  if (args->inst.count > 0) hipLaunchKernelGGL((kStepBegin<true, true>), dim3(nb), dim3(256), 0, stream, k);
+  else hipLaunchKernelGGL((kStepBegin<false, true>), dim3(nb), dim3(256), 0, stream, k);
+  return launchStatus();
+}
+
+extern "C" int fdm_launchReduceStep(const fdm_reduce_args* reduce, const fdm_step_begin_args* args,
+                                    const fdm_skin* skin, hipStream_t stream) {
+  if (!reduce || !args) return FDM_EINVAL;
+  // one pass: the same bodies, a full step on either side
+  if (reduce->particles.n != args->particles.n || reduce->particles.x != args->particles.x || !args->kick ||
+      !args->drift || reduce->gate != args->gate)
+    return FDM_EINVAL;
+  StepBeginK k;
+  unsigned nb = 0;
+  int r = stepBeginSetup(args, skin, nullptr, 0, k, nb);
+  if (r != FDM_OK) return r;
+  ReduceK rk;
+  r = fillReduce(*reduce, rk);
+  if (r != FDM_OK) return r;
+  if (args->inst.count > 0) hipLaunchKernelGGL(kReduceStep<true>, dim3(nb), dim3(256), 0, stream, rk, k);
+  else hipLaunchKernelGGL(kReduceStep<false>, dim3(nb), dim3(256), 0, stream, rk, k);
   return launchStatus();
 }
 

@@ -8,8 +8,11 @@
 // (owned before mirrored on a tie), bonds by bond id. Each record is a
 // per-pair sum that the narrow phase accumulated in node order. The second
 // half-kick follows in the same thread.
+#include <algorithm>
+
 #include "fdm_device.hpp"
 #include "fdm_launch.hpp"
+#include "step_device.hpp"
 
 namespace fdm {
 
@@ -83,107 +86,14 @@ __global__ void kBonds(fdm_bodies P, fdm_bonds b) {
   oj[0] = Tj.x; oj[1] = Tj.y; oj[2] = Tj.z;
 }
 
-struct ReduceK {
-  fdm_bodies P;
-  fdm_geometry pgeo;
-  fdm_pairs pp, pw, g[3];
-  fdm_mirror ppm, gm[3];
-  int havePW, haveG[3];
-  fdm_bonds bonds;
-  int haveBonds;
-  V3 gravity;
-  double h;
-  int kick;
-  int* stepCounter;
-  const int* gate;
-};
-
-__device__ __forceinline__ void addRec(V3& F, V3& T, const double* f, const double* t, bool negF) {
-  const V3 fv = {f[0], f[1], f[2]};
-  F = vadd(F, negF ? vneg(fv) : fv);
-  T = vadd(T, {t[0], t[1], t[2]});
-}
-
-// Smallest mirror entry greater than `last` (mirror lists are short and
-// unordered; selection keeps the fold order independent of append order).
-__device__ __forceinline__ int nextMirror(const int* list, int m, int last) {
-  int best = INT_MAX;
-  for (int t = 0; t < m; ++t) {
-    const int v = list[t];
-    if (v > last && v < best) best = v;
-  }
-  return best;
-}
-
-__device__ __forceinline__ int segBegin(const fdm_pairs& s, int i) {
-  return min(s.count[i], s.capacity);
-}
-__device__ __forceinline__ int segEnd(const fdm_pairs& s, int i) {
-  return min(s.count[i + 1], s.capacity);
-}
-
 __global__ void kReduce(ReduceK a) {
   if (gateOff(a.gate)) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int n = a.P.n;
   if (i == 0 && a.stepCounter) *a.stepCounter += 1;  // read by the bond stage before this launch
   if (i >= n) return;
-  V3 F = {0., 0., 0.}, T = {0., 0., 0.};
-  // particle pairs: as target (partners below i), then owned (partners above)
-  {
-    const int m = min(a.ppm.count[i], a.ppm.capacity);
-    const int* list = a.ppm.list + (size_t)i * a.ppm.capacity;
-    int last = -1;
-    for (int r = 0; r < m; ++r) {
-      const int p = nextMirror(list, m, last);
-      last = p;
-      addRec(F, T, a.pp.sumF + 3 * (size_t)p, a.pp.sumTB + 3 * (size_t)p, true);
-    }
-    if (m > 0) a.ppm.count[i] = 0;
-    for (int p = segBegin(a.pp, i); p < segEnd(a.pp, i); ++p)
-      if (a.pp.recCnt[p] > 0) addRec(F, T, a.pp.sumF + 3 * (size_t)p, a.pp.sumTA + 3 * (size_t)p, false);
-  }
-  if (a.havePW)
-    for (int p = segBegin(a.pw, i); p < segEnd(a.pw, i); ++p)
-      if (a.pw.recCnt[p] > 0) addRec(F, T, a.pw.sumF + 3 * (size_t)p, a.pw.sumTA + 3 * (size_t)p, false);
-  for (int s = 0; s < 3; ++s) {
-    if (!a.haveG[s]) continue;
-    const fdm_pairs& G = a.g[s];
-    const fdm_mirror& M = a.gm[s];
-    const int m = min(M.count[i], M.capacity);
-    const int* list = M.list + (size_t)i * M.capacity;
-    int own = segBegin(G, i);
-    const int ownEnd = segEnd(G, i);
-    int mp = m > 0 ? nextMirror(list, m, -1) : INT_MAX;
-    int used = 0;
-    while (true) {
-      while (own < ownEnd && G.recCnt[own] == 0) ++own;
-      const bool haveOwn = own < ownEnd;
-      const bool haveMir = used < m;
-      if (!haveOwn && !haveMir) break;
-      const int partnerOwn = haveOwn ? G.pairT[own] : INT_MAX;
-      const int partnerMir = haveMir ? G.pairA[mp] : INT_MAX;
-      if (haveOwn && partnerOwn <= partnerMir) {
-        addRec(F, T, G.sumF + 3 * (size_t)own, G.sumTA + 3 * (size_t)own, false);
-        ++own;
-      } else {
-        addRec(F, T, G.sumF + 3 * (size_t)mp, G.sumTB + 3 * (size_t)mp, true);
-        ++used;
-        mp = used < m ? nextMirror(list, m, mp) : INT_MAX;
-      }
-    }
-    if (m > 0) M.count[i] = 0;
-  }
-  if (a.haveBonds) {
-    const fdm_bonds& b = a.bonds;
-    for (int e = b.partStart[i]; e < b.partStart[i + 1]; ++e) {
-      const int code = b.partList[e];
-      const int k = code >> 1;
-      if (!b.applied[k]) continue;
-      if ((code & 1) == 0) addRec(F, T, b.outF + 3 * (size_t)k, b.outTi + 3 * (size_t)k, false);
-      else addRec(F, T, b.outF + 3 * (size_t)k, b.outTj + 3 * (size_t)k, true);
-    }
-  }
+  V3 F, T;
+  foldForces(a, i, F, T);
   st3(a.P.F, n, i, F);
   st3(a.P.T, n, i, T);
   if (!a.kick) return;
@@ -213,6 +123,59 @@ extern "C" int fdm_launchBondForces(fdm_bodies particles, fdm_bonds bonds, hipSt
   return launchStatus();
 }
 
+namespace fdm {
+// Which sets each particle has candidate pairs in: as A from the lists'
+// counts, as target (mirrored sets) from the pairs.
+struct TouchK {
+  int n, haveBonds;
+  const int* bondStart;
+  const int* count[5];  // NULL: no such set
+  const int* total[5];
+  const int* pairT[5];
+  int capacity[5];
+};
+__global__ void kTouchOwn(TouchK k, int* touch) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= k.n) return;
+  int t = 0;
+#pragma unroll
+  for (int s = 0; s < 5; ++s)
+    if (k.count[s] && k.count[s][i + 1] > k.count[s][i]) t |= FDM_TOUCH_A(s);
+  if (k.haveBonds && k.bondStart[i + 1] > k.bondStart[i]) t |= FDM_TOUCH_BOND;
+  touch[i] = t;
+}
+__global__ void kTouchTargets(TouchK k, int* touch) {
+  const int s = blockIdx.y;
+  if (s == 1 || !k.count[s]) return;  // walls are not mirrored
+  const int total = min(*k.total[s], k.capacity[s]);
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < total; p += gridDim.x * blockDim.x) {
+    const int t = k.pairT[s][p];
+    if (t >= 0 && t < k.n) atomicOr(&touch[t], FDM_TOUCH_T(s));
+  }
+}
+}  // namespace fdm
+
+extern "C" int fdm_launchTouch(const fdm_pairs* const sets[5], const fdm_bonds* bonds, int n, int* touch,
+                               hipStream_t stream) {
+  if (!sets || n < 0 || (n > 0 && !touch)) return FDM_EINVAL;
+  if (n == 0) return FDM_OK;
+  TouchK k{};
+  k.n = n;
+  k.haveBonds = bonds && bonds->n > 0;
+  k.bondStart = k.haveBonds ? bonds->partStart : nullptr;
+  for (int s = 0; s < 5; ++s)
+    if (sets[s]) {
+      k.count[s] = sets[s]->count;
+      k.total[s] = sets[s]->total;
+      k.pairT[s] = sets[s]->pairT;
+      k.capacity[s] = sets[s]->capacity;
+    }
+  hipLaunchKernelGGL(kTouchOwn, dim3(blocksFor(n, 256)), dim3(256), 0, stream, k, touch);
+  hipLaunchKernelGGL(kTouchTargets, dim3(std::min<unsigned>(blocksFor(n, 256), 256), 5), dim3(256), 0, stream,
+                     k, touch);
+  return launchStatus();
+}
+
 __global__ void kIncrement(int* c) {
   if (threadIdx.x == 0) *c += 1;
 }
@@ -223,10 +186,9 @@ extern "C" int fdm_incrementCounter(int* counter, hipStream_t stream) {
   return launchStatus();
 }
 
-extern "C" int fdm_launchReduceForceTorque(const fdm_reduce_args* args, hipStream_t stream) {
-  if (!args || !args->pp || !args->ppMirror) return FDM_EINVAL;
-  const fdm_reduce_args& g = *args;
-  ReduceK k{};
+int fdm::fillReduce(const fdm_reduce_args& g, ReduceK& k) {
+  if (!g.pp || !g.ppMirror) return FDM_EINVAL;
+  k = ReduceK{};
   k.P = g.particles;
   k.pgeo = g.pgeo;
   k.pp = *g.pp;
@@ -247,6 +209,15 @@ extern "C" int fdm_launchReduceForceTorque(const fdm_reduce_args* args, hipStrea
   k.kick = g.kick;
   k.stepCounter = g.stepCounter;
   k.gate = g.gate;
+  k.touch = g.touch;
+  return FDM_OK;
+}
+
+extern "C" int fdm_launchReduceForceTorque(const fdm_reduce_args* args, hipStream_t stream) {
+  if (!args) return FDM_EINVAL;
+  const fdm_reduce_args& g = *args;
+  ReduceK k;
+  if (fillReduce(g, k) != FDM_OK) return FDM_EINVAL;
   if (g.particles.n <= 0) {
     if (g.stepCounter) hipLaunchKernelGGL(kIncrement, dim3(1), dim3(64), 0, stream, g.stepCounter);
     return launchStatus();

@@ -308,6 +308,8 @@ class LSSolver {
     if (periodic_.isSector()) skin_ = 0.0;  // images are rebuilt every step
     ctl_.allocate(FDM_CTL_WORDS);
     disp_.allocate(1);
+    fold_.allocate(FDM_FOLD_WORDS);
+    touch_.allocate(std::max<size_t>(N, 1));
     {
       const int one = 1;  // the first step builds every list
       hipCheck(hipMemcpy(ctl_.get() + FDM_CTL_FORCE, &one, sizeof(int), hipMemcpyHostToDevice),
@@ -1084,6 +1086,7 @@ class LSSolver {
     k.ctl = ctl_.get();
     k.disp = disp_.get();
     k.hostDecision = hostDecisionDev_;
+    k.fold = fold_.get();
     return k;
   }
 
@@ -1146,6 +1149,12 @@ class LSSolver {
   // needs: list builds when decided, then the narrow phase of every set in
   // one launch, bonds and the reduction with the second kick.
   void phaseA(bool prime, const int* gate = nullptr) {
+    const fdm_step_begin_args a = beginArgs(prime, gate);
+    const fdm_skin sk = skinView();
+    Timer t(this, "step_begin");
+    fdmCheck(fdm_launchStepBeginDecide(&a, &sk, stream_), "step begin");
+  }
+  fdm_step_begin_args beginArgs(bool prime, const int* gate) {
     fdm_step_begin_args a{};
     a.gate = gate;
     a.particles = particles_.bodies();
@@ -1174,14 +1183,7 @@ class LSSolver {
     for (int s = 0; s < 3; ++s)
       if (periodic_.active(s)) a.clearCounters[q++] = periodic_.set(s).interaction.nextRecordCounter();
     a.clearCounters[q++] = hitCount_.get();
-    const fdm_skin sk = skinView();
-    const size_t wsBytes = workspace_.size() * sizeof(double);
-    {
-      Timer t(this, "step_begin");
-      fdmCheck(fdm_launchStepBegin(&a, &sk, workspace_.get(), wsBytes, stream_), "step begin");
-    }
-    Timer t(this, "decide");
-    fdmCheck(fdm_launchStepDecide(&a, &sk, workspace_.get(), wsBytes, stream_), "step decision");
+    return a;
   }
 
   struct Decision {
@@ -1277,12 +1279,28 @@ class LSSolver {
           broadPhase(FDM_SET_GHOST, periodic_.set(s).interaction, &gv[s], particles_.grid(),
                      periodic_.set(s).table.view());
     }
+    fdm_pairs cur[5];
+    const fdm_pairs* sets[5] = {};
+    cur[0] = pp_.current();
+    sets[0] = &cur[0];
+    if (W) {
+      cur[1] = pw_.current();
+      sets[1] = &cur[1];
+    }
+    for (int s = 0; s < 3; ++s)
+      if (periodic_.active(s)) {
+        cur[2 + s] = periodic_.set(s).interaction.current();
+        sets[2 + s] = &cur[2 + s];
+      }
+    const fdm_bonds bv = bonds_.view();
+    fdmCheck(fdm_launchTouch(sets, &bv, (int)N, touch_.get(), stream_), "pair sets of particles");
   }
 
   // The part of phase B every step runs: the narrow phase of all sets, bonds
   // and the reduction with the second kick. With `gate` each kernel runs
-  // only if *gate != 0 (queued before the decision is known).
-  void phaseBCommon(bool prime, double time, Decision d, const int* gate) {
+  // only if *gate != 0 (queued before the decision is known). chain: the
+  // next step follows at once, so its phase A runs in the reduction's pass.
+  void phaseBCommon(bool prime, double time, Decision d, const int* gate, bool chain = false) {
     fdm_bodies P = particles_.bodies();
     fdm_geometry pgeo = particles_.geometry();
     const fdm_double3 g = {gravity_.x, gravity_.y, gravity_.z};
@@ -1364,6 +1382,14 @@ class LSSolver {
     r.stepCounter = stepCounter_.get();
     r.gate = gate;
     r.tuning = &tuning_;
+    r.touch = touch_.get();
+    if (chain) {
+      r.kick = 1;
+      const fdm_step_begin_args a = beginArgs(false, gate);
+      const fdm_skin sk = skinView();
+      fdmCheck(fdm_launchReduceStep(&r, &a, &sk, stream_), "reduce and step begin");
+      return;
+    }
     {
       Timer t(this, "reduce_kick");
       if (hookMode_ == HookNone) {
@@ -1431,6 +1457,8 @@ class LSSolver {
   }
 
   // ---------------------------------------------------------- lookahead
+  // (within one advance() a step's reduction and the next step's phase A are
+  // one kernel: both run under the same word, the first step's decision)
   // advance() queues each step before the decisions of the steps ahead of
   // it are known: phase A runs only when the control word FDM_CTL_KEEP is
   // set, i.e. when the previous step kept its lists (its own decision sets
@@ -1448,23 +1476,26 @@ class LSSolver {
     double time;
   };
   // Queues `count` steps (1, or kGraphSteps from a captured graph of that
-  // many steps when graphs are on).
-  void queueSteps(int count, double time, std::vector<Queued>& q) {
+  // many steps when graphs are on). `begun`: the first one's phase A was
+  // queued with the step before it; `more`: another step follows these, whose
+  // phase A is queued with the last of them (begun on return).
+  void queueSteps(int count, double time, std::vector<Queued>& q, bool& begun, bool more) {
     const int* keep = ctl_.get() + FDM_CTL_KEEP;
     const Decision kd = {false, false};
     GenState before[kGraphSteps];
+    auto body = [&] {
+      for (int j = 0; j < count; ++j) {
+        if (j == 0 && !begun) phaseA(false, keep);
+        before[j] = saveGenerations();
+        beginSets(kd);
+        phaseBCommon(false, time + dt_ * double(j), kd, keep, more || j + 1 < count);
+      }
+    };
     if (useGraph_) {
       const int stepNext = pp_.nextStepIndex();
-      hipGraphExec_t& ge = (count == 1 ? graphsQueued1_ : graphsQueuedK_)[stepNext][pp_.listIndex()]
+      hipGraphExec_t& ge = (count == 1 ? graphsQueued1_ : graphsQueuedK_)[begun ? 1 : 0][more ? 1 : 0]
+                                                                        [stepNext][pp_.listIndex()]
                                                                         [ghostListIndex()];
-      auto body = [&] {
-        for (int j = 0; j < count; ++j) {
-          phaseA(false, keep);
-          before[j] = saveGenerations();
-          beginSets(kd);
-          phaseBCommon(false, 0.0, kd, keep);
-        }
-      };
       if (!ge) {
         ge = capture(body);
       } else {
@@ -1475,13 +1506,9 @@ class LSSolver {
       }
       hipCheck(hipGraphLaunch(ge, stream_), "graph launch");
     } else {
-      for (int j = 0; j < count; ++j) {
-        phaseA(false, keep);
-        before[j] = saveGenerations();
-        beginSets(kd);
-        phaseBCommon(false, time + dt_ * double(j), kd, keep);
-      }
+      body();
     }
+    begun = more;
     for (int j = 0; j < count; ++j) {
       Queued e;
       e.time = time + dt_ * double(j);
@@ -1522,20 +1549,24 @@ class LSSolver {
     std::vector<Queued> q;
     size_t next = 0;       // next step to queue
     size_t completed = 0;  // steps whose decision has been read
+    bool begun = false;    // phase A of step `next` is queued
     while (completed < nSteps) {
       // with graphs, kGraphSteps steps per launch where they fit
       if (useGraph_ && next + kGraphSteps <= nSteps && (int)q.size() + kGraphSteps <= lookahead_) {
-        queueSteps(kGraphSteps, time + dt_ * double(next), q);
+        queueSteps(kGraphSteps, time + dt_ * double(next), q, begun, next + kGraphSteps < nSteps);
         next += kGraphSteps;
         continue;
       }
       if (next < nSteps && (int)q.size() < lookahead_) {
-        queueSteps(1, time + dt_ * double(next), q);
+        queueSteps(1, time + dt_ * double(next), q, begun, next + 1 < nSteps);
         ++next;
         continue;
       }
       const size_t first = completed;
-      if (!resolveOldest(q)) next = first + 1;  // queue the skipped steps again
+      if (!resolveOldest(q)) {  // queue the skipped steps again
+        next = first + 1;
+        begun = false;
+      }
       completed = first + 1;
     }
   }
@@ -1588,8 +1619,8 @@ class LSSolver {
       if (g) (void)hipGraphExecDestroy(g);
       g = nullptr;
     }
-    for (auto* set : {&graphsQueued1_[0][0][0], &graphsQueuedK_[0][0][0]})
-      for (int k = 0; k < 8; ++k) {
+    for (auto* set : {&graphsQueued1_[0][0][0][0][0], &graphsQueuedK_[0][0][0][0][0]})
+      for (int k = 0; k < 32; ++k) {
         if (set[k]) (void)hipGraphExecDestroy(set[k]);
         set[k] = nullptr;
       }
@@ -1623,7 +1654,7 @@ class LSSolver {
   DeviceBuffer<double> workspace_;
   DeviceBuffer<unsigned> status_;
   DeviceBuffer<int> stepCounter_;
-  DeviceBuffer<int> ctl_;
+  DeviceBuffer<int> ctl_, fold_, touch_;
   std::vector<SystemDesc> systems_;
   std::vector<fdm_grid> sysGrid_;  // particle grid of each system (host copy)
   fdm_instances inst_{};
@@ -1644,11 +1675,12 @@ class LSSolver {
   HookMode hookMode_ = HookUnknown;
   hipGraphExec_t graphsA_[2] = {};
   // queued steps as graphs: one step, or kGraphSteps steps (an even number,
-  // so a graph starts and ends at the same generation parity), keyed by the
-  // result generation, list generation and ghost list generation
+  // so a graph starts and ends at the same generation parity), keyed by
+  // whether the first step's phase A is in the graph and the next step's is,
+  // by the result generation, list generation and ghost list generation
   static constexpr int kGraphSteps = 4;
-  hipGraphExec_t graphsQueued1_[2][2][2] = {};
-  hipGraphExec_t graphsQueuedK_[2][2][2] = {};
+  hipGraphExec_t graphsQueued1_[2][2][2][2][2] = {};
+  hipGraphExec_t graphsQueuedK_[2][2][2][2][2] = {};
   int lookahead_ = 2 * kGraphSteps;
   hipGraphExec_t graphsB_[2][2][2][2][2] = {};
   hipGraphExec_t graphsKeep_[2][2][2] = {};

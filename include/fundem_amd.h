@@ -203,6 +203,7 @@ typedef struct {
 #define FDM_CTL_SEQ 10           /* decisions taken so far */
 #define FDM_CTL_KEEP 11          /* 1 when this step keeps every list (no rebuild at all) */
 #define FDM_CTL_WORDS 16
+#define FDM_FOLD_WORDS (16 * 64 + 16)  /* fdm_skin.fold */
 #define FDM_DECISION_RING 16     /* words of the host-visible decision ring */
 typedef struct {
   double skin;         /* extra reach of the candidate lists (0: rebuild every step) */
@@ -216,6 +217,9 @@ typedef struct {
                           launches only the work a step needs, and may queue up to
                           FDM_DECISION_RING - 1 steps ahead of the decisions it has read);
                           NULL to skip */
+  int* fold;           /* [FDM_FOLD_WORDS], zero before the first use: where the workgroups of
+                          fdm_launchStepBeginDecide and fdm_launchReduceStep meet (NULL: those
+                          two are refused); left zero by each launch. One step at a time. */
 } fdm_skin;
 
 /* Candidate pairs and tangential history of one interaction set. */
@@ -409,6 +413,8 @@ int fdm_launchStepBegin(const fdm_step_begin_args* args, const fdm_skin* skin, v
                         size_t workspaceBytes, hipStream_t stream);
 int fdm_launchStepDecide(const fdm_step_begin_args* args, const fdm_skin* skin, void* workspace,
                          size_t workspaceBytes, hipStream_t stream);
+/* Both in one launch: the last workgroup to finish takes the decision. */
+int fdm_launchStepBeginDecide(const fdm_step_begin_args* args, const fdm_skin* skin, hipStream_t stream);
 /* No counterpart in the reference. When ctl[FDM_CTL_REBUILD] is set, records
  * every body's grid state in table.validAtBuild and writes the table's
  * unsorted lists for the build (sortKey = cell id + 1, sortIndex = body
@@ -666,8 +672,26 @@ typedef struct {
   int* stepCounter;    /* incremented by one after the reduction (NULL: skip) */
   const int* gate;     /* run only when *gate != 0 (NULL: always) */
   const struct fdm_tuning_s* tuning; /* launch shapes (NULL: the process default) */
+  const int* touch;    /* [n] sets a particle has candidate pairs in, of fdm_launchTouch for
+                          the lists in use (NULL: every set's counts are read) */
 } fdm_reduce_args;
 int fdm_launchReduceForceTorque(const fdm_reduce_args* args, hipStream_t stream);
+
+/* No counterpart in the reference. touch[i] tells the sets in which particle
+ * i has candidate pairs, as A or as target, and whether it has bonds; sets in
+ * the order particle, wall, ghost X, Y, XY (NULL: no such set). */
+#define FDM_TOUCH_A(set) (1 << (set))
+#define FDM_TOUCH_T(set) (1 << (8 + (set)))
+#define FDM_TOUCH_BOND (1 << 16)
+int fdm_launchTouch(const fdm_pairs* const sets[5], const fdm_bonds* bonds, int n, int* touch,
+                    hipStream_t stream);
+
+/* No counterpart in the reference: fdm_launchReduceForceTorque with kick = 1,
+ * followed by fdm_launchStepBeginDecide of the next step (kick and drift set,
+ * the same bodies and gate), in one pass over the bodies. The force and
+ * torque are used, but not stored. */
+int fdm_launchReduceStep(const fdm_reduce_args* reduce, const fdm_step_begin_args* begin,
+                         const fdm_skin* skin, hipStream_t stream);
 
 /* Fill n ints with a value (a kernel, not a memset node, so it replays
  * correctly inside captured graphs). */
