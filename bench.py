@@ -91,7 +91,8 @@ def log(*a):
 
 # Algorithmic HBM bytes per launch of the timed stages (FP64 positions, FP32
 # v, w, q, F, T, 32-bit ids; template tables stay in cache):
-#   step_begin   (kStepBegin alone; the decision kernel is timed as "decide")
+#   step_begin   (with the list decision; steps timed one by one run it apart
+#                from the reduction)
 #                per particle: read x 24, v 12, w 12, q 16, F 12, T 12,
 #                template id 4, grid state at build 4, visibility at build 4
 #                (= 100); write x 24, v 12, w 12, q 16, cell id 4 (= 68);
@@ -475,7 +476,7 @@ def log_stages(stages, steps):
             f"{ms / steps * 1e3:8.1f} us/step (stage-timed pass)")
 
 
-REBUILD_STAGES = ("sort_cells", "broad_pp", "broad_pw", "broad_ghost", "periodic_build")
+REBUILD_STAGES = ("list_build", "sort_cells", "broad_pp", "broad_pw", "broad_ghost", "periodic_build")
 
 
 def rebuild_cost(stages, steps, builds):

@@ -36,12 +36,11 @@
 // they never remove a contact that the exact test would accept.
 #include <algorithm>
 
+#include "cull_device.hpp"
 #include "fdm_device.hpp"
 #include "fdm_launch.hpp"
 
 namespace fdm {
-
-constexpr double kReach = 1.0 + 1e-5;
 
 struct Target {
   V3 x;       // detection position
@@ -79,18 +78,6 @@ __device__ __forceinline__ Q4 ld4R(const fdm_real* p, int n, int i) {
 }
 __device__ __forceinline__ V3 ldd3R(const double* p) { return {ldu(p), ldu(p + 1), ldu(p + 2)}; }
 
-// True when no point within `reach` of `local` (target frame) can have
-// phi <= 0: the point is inside the SDF box and phi - Lip*reach is positive
-// beyond a relative margin.
-__device__ __forceinline__ bool lipschitzClear(V3 local, double reach, const fdm_template& t,
-                                               const float* sdf) {
-  Sample s;
-  if (!sampleSDF(local, t, sdf, s)) return false;
-  const double phi = trilinear(s.x, s.y, s.z, s.c);
-  const double lr = t.lipschitz * reach;
-  return phi - lr > 1e-6 * (fabs(phi) + lr);
-}
-
 // True when phi > 0 at `local` for certain on an affine (plane-wall) SDF:
 // the plane's value exceeds the fit's bound on the residual and rounding.
 // Such a node cannot touch, so its SDF fetch is skipped.
@@ -113,30 +100,6 @@ __device__ __forceinline__ bool levelClear(V3 local, double reach, const fdm_tem
   return t.affine ? planeClearBall(local, reach, t) : lipschitzClear(local, reach, t, sdf);
 }
 
-// True when the ball (local, reach) misses the SDF box of t (target frame).
-__device__ __forceinline__ bool outsideBox(V3 local, double reach, const fdm_template& t) {
-  const double h = 1.0 / t.invSpacing;
-  double d2 = 0.0;
-  const double lo[3] = {t.origin[0], t.origin[1], t.origin[2]};
-  const double p[3] = {local.x, local.y, local.z};
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const double hi = lo[a] + h * (double)(t.size[a] - 1);
-    const double m = 1e-6 * (hi - lo[a]);
-    double e = 0.0;
-    if (p[a] < lo[a] - m) e = lo[a] - m - p[a];
-    else if (p[a] > hi + m) e = p[a] - hi - m;
-    d2 += e * e;
-  }
-  const double r = reach * kReach;
-  return d2 > r * r;
-}
-
-// Clamped cell range of the box [c - r, c + r] (monotone in each coordinate).
-__device__ __forceinline__ void cellRange(V3 c, double r, const fdm_grid& g, I3& lo, I3& hi) {
-  lo = clampedCell(vsub(c, {r, r, r}), g);
-  hi = clampedCell(vadd(c, {r, r, r}), g);
-}
 __device__ __forceinline__ bool cellNear(I3 t, I3 lo, I3 hi) {
   return t.x >= lo.x - 1 && t.x <= hi.x + 1 && t.y >= lo.y - 1 && t.y <= hi.y + 1 &&
          t.z >= lo.z - 1 && t.z <= hi.z + 1;

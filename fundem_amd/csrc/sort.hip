@@ -118,6 +118,32 @@ __global__ void __launch_bounds__(kScanThreads) kScanApply(const int* in, int* o
   }
 }
 
+// Exclusive scan of up to kScanOne ints in place by one workgroup: for the
+// histograms of small sorts, where two more launches cost more than the
+// parallelism gives (110592 keys: one launch of 5.6 us, three of 2.4 to 5).
+constexpr int kScanOne = 16384;
+__global__ void __launch_bounds__(1024) kScanOneBlock(int* data, int n, const int* gate) {
+  if (gateOff(gate)) return;
+  __shared__ int lds[1024 / 64 + 1];
+  int carry = 0;
+  for (int base = 0; base < n; base += 4096) {
+    const int i = base + 4 * (int)threadIdx.x;
+    int v[4], s = 0, t;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = i + k < n ? data[i + k] : 0;
+      s += v[k];
+    }
+    int run = carry + blockExclusiveScan(s, lds, t);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (i + k < n) data[i + k] = run;
+      run += v[k];
+    }
+    carry += t;
+  }
+}
+
 size_t scanWorkspace(size_t n) { return alignUp((blocksFor((long long)n, kScanTile) + 1) * sizeof(int)); }
 
 int scanInts(const int* in, int* out, size_t n, bool inclusive, int* total, void* ws, size_t wsBytes,
@@ -286,9 +312,12 @@ int radixSort(unsigned* keys, int* vals, size_t n, const int* nDev, int keyBits,
     const int shift = p * kRadixBits;
     hipLaunchKernelGGL(kRadixUpsweep, dim3(nb), dim3(kSortThreads), 0, stream, ki, n, nDev, shift,
                        hist, (int)nb, gate);
-    int r = scanInts(hist, hist, (size_t)nb * kRadixBins, false, nullptr, sws, swsBytes, stream,
-                     gate);
-    if (r != FDM_OK) return r;
+    if (nb * kRadixBins <= kScanOne) {
+      hipLaunchKernelGGL(kScanOneBlock, dim3(1), dim3(1024), 0, stream, hist, (int)(nb * kRadixBins), gate);
+    } else {
+      const int r = scanInts(hist, hist, (size_t)nb * kRadixBins, false, nullptr, sws, swsBytes, stream, gate);
+      if (r != FDM_OK) return r;
+    }
     hipLaunchKernelGGL(kRadixDownsweep, dim3(nb), dim3(kSortThreads), 0, stream, ki, vi, ko, vo, n,
                        nDev, shift, hist, (int)nb, gate);
     unsigned* tk = ki;

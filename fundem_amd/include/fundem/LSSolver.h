@@ -310,6 +310,7 @@ class LSSolver {
     disp_.allocate(1);
     fold_.allocate(FDM_FOLD_WORDS);
     touch_.allocate(std::max<size_t>(N, 1));
+    buildOff_.allocate(5 * std::max<size_t>(N, 1), false);
     {
       const int one = 1;  // the first step builds every list
       hipCheck(hipMemcpy(ctl_.get() + FDM_CTL_FORCE, &one, sizeof(int), hipMemcpyHostToDevice),
@@ -361,7 +362,7 @@ class LSSolver {
     bonds_.initialize(N, stepCounter_.get(), stream_);
     size_t ws = fdm_radixSortWorkspaceBytes(std::max<size_t>({N, W, size_t(64)}));
     ws = std::max(ws, fdm_scanWorkspaceBytes(N + 1));
-    ws = std::max(ws, fdm_stepBeginWorkspaceBytes(N + W));
+    ws = std::max(ws, fdm_buildListsWorkspaceBytes(std::max<size_t>(N, 64)));
     workspace_.allocate(ws / sizeof(double) + 1, false);
     destroyGraphs();
     if (!hostDecision_) {
@@ -1224,6 +1225,56 @@ class LSSolver {
   // List builds of a step (the part of phase B that runs only when the
   // decision asks for it).
   void phaseBRebuild(Decision d) {
+    // images with poses of their own, or more walls than one workgroup sorts
+    if (periodic_.isSector() || walls_.num() > 1024) {
+      phaseBRebuildStaged(d);
+      return;
+    }
+    const size_t W = walls_.num();
+    fdm_build_args b{};
+    b.particles = particles_.bodies();
+    b.pgeo = particles_.geometry();
+    b.pgrid = particles_.grid();
+    b.ptable = particles_.table().view();
+    b.walls = walls_.bodies();
+    b.walls.n = (int)W;
+    b.wgeo = walls_.geometry();
+    b.wgrid = walls_.grid();
+    b.wtable = walls_.table().view();
+    b.periodic = periodic_.flags();
+    b.inst = inst_;
+    fdm_pairs cur[5];
+    fdm_ghosts gv[3];
+    cur[0] = pp_.current();
+    b.sets[0] = &cur[0];
+    if (W) {
+      cur[1] = pw_.current();
+      b.sets[1] = &cur[1];
+    }
+    for (int s = 0; s < 3; ++s) {
+      if (!periodic_.active(s)) continue;
+      gv[s] = periodic_.view(s);
+      b.ghosts[s] = &gv[s];
+      cur[2 + s] = periodic_.set(s).interaction.current();
+      b.sets[2 + s] = &cur[2 + s];
+    }
+    const fdm_bonds bv = bonds_.view();
+    b.bonds = &bv;
+    b.skin = skin_;
+    b.maxRadius = maxRadius_;
+    b.maxBoxReach = maxBoxReach_;
+    b.full = d.rebuild ? 1 : 0;
+    b.touch = touch_.get();
+    // (the law's headers are written by the sweep that follows)
+    b.tmp = lawHead_.get();
+    b.tmpWords = (long long)lawHead_.size();
+    b.tmpOff = buildOff_.get();
+    b.status = status_.get();
+    Timer t(this, "list_build");
+    fdmCheck(fdm_launchBuildLists(&b, workspace_.get(), workspace_.size() * sizeof(double), stream_),
+             "list build");
+  }
+  void phaseBRebuildStaged(Decision d) {
     fdm_bodies P = particles_.bodies();
     const size_t N = particles_.num(), W = walls_.num();
     void* ws = workspace_.get();
@@ -1551,21 +1602,29 @@ class LSSolver {
     size_t completed = 0;  // steps whose decision has been read
     bool begun = false;    // phase A of step `next` is queued
     while (completed < nSteps) {
+      // Steps in flight: a rebuild costs the launches of the steps queued
+      // behind it, so the queue is short after one and doubles with every
+      // step that keeps its lists (a flowing periodic system rebuilds every
+      // other step; a settled one not for hundreds).
+      const int depth = std::min(lookahead_, depth_);
       // with graphs, kGraphSteps steps per launch where they fit
-      if (useGraph_ && next + kGraphSteps <= nSteps && (int)q.size() + kGraphSteps <= lookahead_) {
+      if (useGraph_ && next + kGraphSteps <= nSteps && (int)q.size() + kGraphSteps <= depth) {
         queueSteps(kGraphSteps, time + dt_ * double(next), q, begun, next + kGraphSteps < nSteps);
         next += kGraphSteps;
         continue;
       }
-      if (next < nSteps && (int)q.size() < lookahead_) {
+      if (next < nSteps && (int)q.size() < depth) {
         queueSteps(1, time + dt_ * double(next), q, begun, next + 1 < nSteps);
         ++next;
         continue;
       }
       const size_t first = completed;
-      if (!resolveOldest(q)) {  // queue the skipped steps again
+      if (resolveOldest(q)) {
+        depth_ = std::min(2 * depth_, FDM_DECISION_RING);
+      } else {  // queue the skipped steps again
         next = first + 1;
         begun = false;
+        depth_ = 2;
       }
       completed = first + 1;
     }
@@ -1654,7 +1713,7 @@ class LSSolver {
   DeviceBuffer<double> workspace_;
   DeviceBuffer<unsigned> status_;
   DeviceBuffer<int> stepCounter_;
-  DeviceBuffer<int> ctl_, fold_, touch_;
+  DeviceBuffer<int> ctl_, fold_, touch_, buildOff_;
   std::vector<SystemDesc> systems_;
   std::vector<fdm_grid> sysGrid_;  // particle grid of each system (host copy)
   fdm_instances inst_{};
@@ -1682,6 +1741,7 @@ class LSSolver {
   hipGraphExec_t graphsQueued1_[2][2][2][2][2] = {};
   hipGraphExec_t graphsQueuedK_[2][2][2][2][2] = {};
   int lookahead_ = 2 * kGraphSteps;
+  int depth_ = FDM_DECISION_RING;  // steps in flight now, at most lookahead_
   hipGraphExec_t graphsB_[2][2][2][2][2] = {};
   hipGraphExec_t graphsKeep_[2][2][2] = {};
   int* hostDecision_ = nullptr;     // pinned, host view

@@ -647,6 +647,41 @@ int fdm_launchBondForces(fdm_bodies particles, fdm_bonds bonds, hipStream_t stre
 int fdm_launchBroadPhaseWrite(const fdm_broadphase_args* args, unsigned* status,
                               hipStream_t stream);
 
+/* No counterpart in the reference: the list builds of a step (planar or no
+ * periodicity, at most 1024 walls): with `full` every set, otherwise the
+ * ghost sets only. Replaces, in one call, fdm_launchCommitBodyState and
+ * fdm_buildHashStartEnd of particles and walls, fdm_launchPeriodicBuild,
+ * fdm_launchBroadPhase and fdm_launchBroadPhaseWrite of every set, and
+ * fdm_launchTouch. Lists and the particle and wall tables are the same; the
+ * ghost sets' tables hold linked lists instead of sorted ranges (cellStart:
+ * first ghost of the clamped geometric cell or -1; sortIndex: the next one),
+ * with the ghosts in no order. */
+typedef struct {
+  fdm_bodies particles;
+  fdm_geometry pgeo;
+  fdm_grid pgrid;
+  fdm_hash_table ptable;
+  fdm_bodies walls;
+  fdm_geometry wgeo;
+  fdm_grid wgrid;
+  fdm_hash_table wtable;
+  fdm_periodic periodic;
+  fdm_instances inst;
+  const fdm_ghosts* ghosts[3]; /* X, Y, XY where active, sharing one atBuild */
+  const fdm_pairs* sets[5];    /* particle, wall (NULL: no walls), ghost X, Y, XY */
+  const fdm_bonds* bonds;      /* NULL when there are none */
+  double skin, maxRadius, maxBoxReach; /* over the particle templates */
+  int full;
+  int* touch;                  /* [n] as fdm_launchTouch */
+  int* tmp;                    /* [tmpWords >= 2 * the capacities of the built sets] */
+  long long tmpWords;
+  int* tmpOff;                 /* [5 * n] */
+  unsigned* status;
+} fdm_build_args;
+size_t fdm_buildListsWorkspaceBytes(size_t n);
+int fdm_launchBuildLists(const fdm_build_args* args, void* workspace, size_t workspaceBytes,
+                         hipStream_t stream);
+
 /* Add one to a device counter (the step index a captured graph replays). */
 int fdm_incrementCounter(int* counter, hipStream_t stream);
 
