@@ -22,8 +22,8 @@
 //               reference's predicate exactly in FP64: stencil membership of
 //               the target's cell, bounding sphere (particle targets, lower
 //               index only), SDF box and -phi >= 0. The contacts' normals and
-//               points are staged in node order and history records reserved;
-//               then one thread per pair takes each contact's previous spring
+//               points stay in LDS and history records are reserved; then
+//               one lane per contact takes the contact's previous spring
 //               (keyed by (A, target, node)), applies the linear
 //               spring-dashpot law and writes the updated spring. Forces and
 //               torques are summed per pair in node order, serially, so the
@@ -788,27 +788,10 @@ __global__ void __launch_bounds__(256) kNarrow(NarrowK a) {
 // that walks its contacts in node order.
 
 struct NarrowScratch {
-  int* workHit;      // [work item] first staged contact
-  // [8 * work item] or null: what the law kernel needs first, written by the
-  // sweep so that the law's thread starts with one load instead of a chain:
-  // record count, first record, first staged contact, A, target, and the
-  // previous step's record range of the pair
-  int* lawHead;
   double* hitGeom;   // [8 * hitCapacity]: contact point, normal, overlap, node id
   int hitCapacity;
   int* hitCount;     // [FDM_REC_COUNTERS] pool counters of the staged contacts
 };
-
-__device__ __forceinline__ void stageHit(double* g, V3 pc, V3 nrm, double ov, int k) {
-  g[0] = pc.x;
-  g[1] = pc.y;
-  g[2] = pc.z;
-  g[3] = nrm.x;
-  g[4] = nrm.y;
-  g[5] = nrm.z;
-  g[6] = ov;
-  g[7] = (double)k;
-}
 
 // ------------------------------------------------------------------- sweep
 // What the culls need of one pair, in FP32 (margins below). With SDF grids:
@@ -826,7 +809,14 @@ struct alignas(16) CullRec {
 // What the exact predicate needs of one pair.
 struct PairCtx {
   double qA[4], xA[3], qT[4], xT[3], ih;
-  int geoA, geoT, hash, inst;
+  int geoA, geoT, hash, inst, ghost;
+};
+// What the contact law needs of one pair of a run.
+struct LawRec {
+  int base, first;        // first record (-1: none), first of the run's contacts
+  int prevOff, prevCnt;   // the pair's records of the previous step
+  int A, T;
+  int staged;             // first staged contact (contacts in memory)
 };
 constexpr int kRunMax = 8;                  // pairs of one wave and item
 constexpr int kUnitLanes = FDM_GROUP;       // groups per unit of the group cull, nodes per group
@@ -836,11 +826,14 @@ constexpr int kLiveMax = 256;
 struct SweepSlots {
   CullRec cull[kRunMax];
   PairCtx ctx[kRunMax];
-  double pc[3][kMaxHits], nrm[3][kMaxHits], ov[kMaxHits];  // the run's hits in the order found
-  unsigned long long chunks[kRunMax];                      // chunks of the pair holding hits
+  // rows 0-6: point, normal and overlap of the run's hits in the order found;
+  // then force and torques of its contacts in the order of their sums
+  double c[9][kMaxHits];
+  unsigned long long chunks[kRunMax];  // chunks of the pair holding hits
+  LawRec law[kRunMax];
   int hit[kMaxHits];                                       // pair of the run << 16 | node
   int cand[64];  // nodes that passed the cell test, not yet tested exactly (same coding)
-  int total[kRunMax], gbase[kRunMax];
+  int total[kRunMax];
   unsigned short unit[kRunMax * kMaxBlocks];  // pair << 8 | block of groups
   unsigned short live[kLiveMax];              // pair << 8 | surviving group
 };
@@ -853,10 +846,29 @@ __device__ __forceinline__ fdm_grid particleGrid(const NarrowCommon& C, int inst
   asm volatile("" : "+s"(g.min.x), "+s"(g.min.y), "+s"(g.max.x), "+s"(g.max.y));
   return g;
 }
+// (images of a sector boundary in a kernel of their own: what turns them
+// costs registers)
+template <bool MANY, bool SECTOR>
+__device__ __forceinline__ fdm_periodic particlePeriodic(const NarrowCommon& C, int inst) {
+  fdm_periodic p = MANY ? ldu(C.inst.periodic + inst) : C.periodic;
+  if (!SECTOR) p.sector = 0;
+  return p;
+}
 template <int SET, bool MANY>
 __device__ __forceinline__ fdm_grid targetGrid(const NarrowCommon& C, const NarrowSet& S, int inst) {
   if (MANY) return SET == FDM_SET_WALL ? ldu(C.inst.wgrid + inst) : ldu(C.inst.pgrid + inst);
   return S.grid;
+}
+__device__ __forceinline__ int lanesBelow(unsigned long long m) {  // set bits of lanes below this one
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+// Inclusive sum over lanes 0 to kRunMax - 1 (lanes of one row: a row shift
+// fills with zero, and no lane index is kept over the wave's loop).
+__device__ __forceinline__ int runScan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+  return v;
 }
 __device__ __forceinline__ float clampTo(float u, float hi) { return __builtin_amdgcn_fmed3f(u, 0.f, hi); }
 // The code of the SDF cell nearest to index coordinates u (their clamped
@@ -916,11 +928,76 @@ __device__ __forceinline__ bool nodeMayTouch(const CullRec& k, const unsigned ch
   return f <= k.eps;
 }
 
+// The linear spring-dashpot law of one contact of a run, contact `at` of its
+// pair in node order: its spring is updated and left as its record, its force
+// and torques in `slot`.
+template <int SET, bool MANY, bool SECTOR>
+__device__ __forceinline__ void lawContact(const NarrowCommon& C, const NarrowSet& S, const PairCtx& c, const LawRec& lr,
+                                           int node, int at, V3 pc, V3 nrm, double ov, SweepSlots& ws, int slot) {
+  // the pair's previous contact at this place, nearly always of the same node
+  fdm_record pr{};
+  if (lr.prevCnt > 0) pr = ldu(S.prev.rec + lr.prevOff + min(at, lr.prevCnt - 1));
+  const int n = C.P.n;
+  const fdm_grid pg = particleGrid<MANY>(C, c.inst);
+  const PairFrame fr = {&pg, &pg, particlePeriodic<MANY, SECTOR>(C, c.inst)};
+  // material constants of the pair (contactKernel.cu:79-110,167-193,243-274)
+  const fdm_material Mi = matOf(C.pmat, ldu(C.P.mat + lr.A));
+  const double invMi = ldu(&C.pgeo.info[c.geoA].invMass);
+  double kn = 0., ks = 0., effM = 0., mu, diss;
+  V3 vB, wB;
+  if (SET == FDM_SET_WALL) {
+    const fdm_material Mw = matOf(C.wmat, ldu(C.W.mat + lr.T));
+    if (invMi > 0.) effM = 1. / invMi;
+    mu = fmin(Mi.mu, Mw.mu);
+    diss = Mi.e <= Mw.e ? Mi.dissipation : Mw.dissipation;
+    kn = Mi.kn;
+    ks = Mi.ks;
+    vB = ld3R(C.W.v, C.W.n, lr.T);
+    wB = ld3R(C.W.w, C.W.n, lr.T);
+  } else {
+    const fdm_material Mj = matOf(C.pmat, ldu(C.P.mat + lr.T));
+    const double invMj = ldu(&C.pgeo.info[c.geoT].invMass);
+    if (Mi.kn > 0. && Mj.kn > 0.) kn = Mi.kn * Mj.kn / (Mi.kn + Mj.kn);
+    if (Mi.ks > 0. && Mj.ks > 0.) ks = Mi.ks * Mj.ks / (Mi.ks + Mj.ks);
+    if (invMi > 0. || invMj > 0.) effM = 1. / (invMi + invMj);
+    diss = Mi.e <= Mj.e ? Mi.dissipation : Mj.dissipation;
+    mu = fmin(Mi.mu, Mj.mu);
+    vB = SECTOR && SET == FDM_SET_GHOST && S.ghostVel ? ldd3R(S.ghostVel + 3 * (size_t)c.ghost) : forceVel(C, fr, lr.T);
+    wB = ld3R(C.P.w, n, lr.T);  // a sector image keeps the real spin (contactKernel.cu:258)
+  }
+  const V3 vA = forceVel(C, fr, lr.A);
+  const V3 wA = ld3R(C.P.w, n, lr.A);
+  const V3 xA = {c.xA[0], c.xA[1], c.xA[2]}, xT = {c.xT[0], c.xT[1], c.xT[2]};
+  const V3 armA = SET == FDM_SET_GHOST ? xA : wrappedArm(xA, pg, fr.periodic);
+  const V3 armB = SET == FDM_SET_PARTICLE ? wrappedArm(xT, pg, fr.periodic) : xT;
+  V3 F = {0., 0., 0.}, spring = {0., 0., 0.};
+  if (lr.prevCnt > 0) spring = pr.node == node ? recordSpring(pr) : findPrevSpring(S, lr.prevOff, lr.prevCnt, node);
+  if (C.updateSprings) {
+    const V3 vc = vsub(vadd(vA, vcross(wA, vsub(pc, armA))), vadd(vB, vcross(wB, vsub(pc, armB))));
+    linearContact(F, spring, vc, nrm, ov, C.dt, kn, ks, mu, diss, effM);
+  }
+  const V3 TA = vcross(vsub(pc, armA), F), TB = vcross(vsub(pc, armB), vneg(F));
+  const double v[9] = {F.x, F.y, F.z, TA.x, TA.y, TA.z, TB.x, TB.y, TB.z};
+#pragma unroll
+  for (int c = 0; c < 9; ++c) ws.c[c][slot] = v[c];
+  const int r = lr.base + at;
+  S.pairs.rec[r] = makeRecord(spring, node);
+  if (C.dbgPoint) {
+    C.dbgPoint[3 * r] = pc.x;
+    C.dbgPoint[3 * r + 1] = pc.y;
+    C.dbgPoint[3 * r + 2] = pc.z;
+    C.dbgNormal[3 * r] = nrm.x;
+    C.dbgNormal[3 * r + 1] = nrm.y;
+    C.dbgNormal[3 * r + 2] = nrm.z;
+    C.dbgOverlap[r] = ov;
+  }
+}
+
 // Node sweep of a run of `np` <= kRunMax candidate pairs of one set by one
 // wave: the pairs, their node groups and their nodes are culled in the
 // target's frame, the remaining nodes of all the run's pairs take the
-// reference's exact predicate together, and each pair's contacts are staged
-// in node order for the contact-law kernel, with its record range reserved.
+// reference's exact predicate together, and the contact law runs with one
+// contact per lane, each pair's forces and torques added in node order.
 //
 // A pair is a chain of dependent loads (list, bodies, templates, groups,
 // cell codes, nodes, cell codes, SDF corners) with little arithmetic between
@@ -936,51 +1013,56 @@ __device__ __forceinline__ bool nodeMayTouch(const CullRec& k, const unsigned ch
 //    bound of phi does not serve here: f / |grad f| is steep to 1e9 at the
 //    centre of a superellipsoid.) Affine walls test the plane instead;
 //  - the exact predicate (two quaternion rotations, eight SDF corners, the
-//    cell stencil: some 300 FP64 instructions) for the few nodes left.
+//    cell stencil: some 300 FP64 instructions) for the few nodes left;
+//  - the contact law from the contacts in LDS: the records are reserved by one
+//    pair per lane (their atomics issued together), then one contact per lane,
+//    then one component of a pair's sums per lane. As a kernel of its own with
+//    a thread per pair the law was a serial chain over the pair's contacts,
+//    with their geometry passed through memory. A run with more contacts than
+//    the 64 slots recomputes them chunk by chunk and stages them in memory.
 // Measured against one pair per wave with 64-node chunks culled by Lipschitz
 // bound and swept in FP64 (and wall pairs four per wave): 254K particle pairs
 // of a compressed lattice, 23 % of them in contact, 613 + 22 -> 201 us; the
 // million-particle pour's 11.4K wall, 5.8K particle and 4.1K image pairs 44.3
 // -> 23 us; 44.6K pairs of touching 400-node spheres 79 -> 29 us; one pair
-// alone 10.7 -> 10.1 us.
+// alone 10.7 -> 10.1 us. With the law, against the sweep and the law kernel:
+// 201 + 46 -> 220 us; 23.1 + 11.7 -> 24.5 us; 216 particles, up to 20 contacts
+// a pair, 11.8 + 19.5 -> 13.3 us; one pair 10.0 + 5.1 -> 11.8 us.
 // Margins: reaches are widened by kReach (a unit quaternion stored in FP32
 // scales vectors by up to 1 +- 2.4e-7), and index coordinates by eps, which
 // covers the FP32 rounding of the map, of the nodes and of their sums (a few
 // 2^-24 of the largest coordinate) and the exact predicate's own rounding.
-template <int SET, bool MANY>
-__device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const NarrowScratch& X, int w0,
-                         int p0, int np, int lane, SweepSlots& ws) {
+template <int SET, bool MANY, bool SECTOR>
+__device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const NarrowScratch& X, int w0, int p0, int np,
+                         int lane, SweepSlots& ws) {
   // (opaque in every run, as the grid in particleGrid)
   asm volatile("" : "+v"(lane));
   const int n = C.P.n;
   const int p = p0 + lane, w = w0 + lane;
   const fdm_geometry& tgeo = SET == FDM_SET_WALL ? C.wgeo : C.pgeo;
-  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   auto emptyRange = [&]() __attribute__((always_inline)) {
     S.pairs.recOff[p] = 0;
     S.pairs.recCnt[p] = 0;
-    if (X.lawHead) *reinterpret_cast<int4*>(X.lawHead + 8 * (size_t)w) = make_int4(0, 0, 0, 0);
   };
   int units = 0;
-  int A = -1, T = 0;
-  int prevOff = 0, prevCnt = -1;  // previous record range of the pair (-1: not at its index)
   if (lane < np) {
+    int prevOff = 0, prevCnt = -1;  // previous record range of the pair (-1: not at its index)
     ws.total[lane] = 0;
     ws.chunks[lane] = 0ull;
-    A = ldu(S.pairs.pairA + p);
-    T = ldu(S.pairs.pairT + p);
+    const int A = ldu(S.pairs.pairA + p), T = ldu(S.pairs.pairT + p);
     // (lists kept from the previous step hold the pair at the same index:
     // these loads go along with the pair's own)
-    if (X.lawHead && p < min(ldu(S.prev.total), S.prev.capacity)) {
+    if (p < min(ldu(S.prev.total), S.prev.capacity)) {
       const int pA = ldu(S.prev.pairA + p), pT = ldu(S.prev.pairT + p);
       prevOff = ldu(S.prev.recOff + p);
       prevCnt = ldu(S.prev.recCnt + p);
       if (pA != A || pT != T) prevCnt = -1;
     }
+    ws.law[lane] = {-1, 0, prevOff, prevCnt, A, T, 0};
     if (A >= 0) {  // (below zero: a slot left empty by a capacity overflow)
       const int inst = MANY ? ldu(C.inst.particleInstance + A) : 0;
       const fdm_grid pg = particleGrid<MANY>(C, inst);
-      const fdm_periodic per = MANY ? ldu(C.inst.periodic + inst) : C.periodic;
+      const fdm_periodic per = particlePeriodic<MANY, SECTOR>(C, inst);
       // A's and the target's poses as the set's detection sees them
       V3 xA = ldpR(C.P.x, n, A);
       Q4 qA = ld4R(C.P.q, n, A);
@@ -1013,9 +1095,10 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
           hash = ghostCellHash(xT, pg);
         } else {
           const int gi = ldu(S.pairs.pairG + p);
+          ws.ctx[lane].ghost = gi;
           xT = ldd3R(S.ghostPos + 3 * (size_t)gi);
           hash = ldu(S.ghostHash + gi);
-          if (S.ghostQ) {
+          if (SECTOR && S.ghostQ) {
             const double* gq = S.ghostQ + 4 * (size_t)gi;
             qT = {gq[0], gq[1], gq[2], gq[3]};
           }
@@ -1091,13 +1174,8 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
     if (units == 0) emptyRange();
   }
   // units of the group cull, pair by pair
-  int before = units;
-#pragma unroll
-  for (int off = 1; off < kRunMax; off <<= 1) {
-    const int v = __shfl_up(before, off, 64);
-    if (lane >= off) before += v;
-  }
-  const int nUnits = __shfl(before, kRunMax - 1);
+  const int before = runScan(units);
+  const int nUnits = readlaneI(before, kRunMax - 1);
   if (nUnits == 0) return;
   for (int u = 0; u < units; ++u) ws.unit[before - units + u] = (unsigned short)(lane << 8 | u);
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1106,7 +1184,7 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
   // the maps of the run's pairs, one column per lane (column 3: the shift)
   {
     const int j = lane >> 2, col = lane & 3;
-    const bool has = __shfl(units, j) > 0;
+    const bool has = __builtin_amdgcn_ds_bpermute(4 * j, units) > 0;
     if (has && (SET != FDM_SET_WALL || ws.cull[j].cells >= 0)) {
       const PairCtx& c = ws.ctx[j];
       CullRec& k = ws.cull[j];
@@ -1180,7 +1258,7 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
       }
       iu += 64 / kUnitLanes;
       const unsigned long long m = ballot64(live);
-      if (live) ws.live[nlive + __popcll(m & lt)] = (unsigned short)code;
+      if (live) ws.live[nlive + lanesBelow(m)] = (unsigned short)code;
       nlive += __popcll(m);
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1203,7 +1281,7 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
         break;
       }
       il += 64 / kUnitLanes;
-      if (cand) ws.cand[ncand + __popcll(m & lt)] = code;
+      if (cand) ws.cand[ncand + lanesBelow(m)] = code;
       ncand += __popcll(m);
     }
     if (!full) {
@@ -1222,18 +1300,14 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
       }
       const unsigned long long m = ballot64(hit);
       if (hit) {
-        const int slot = nhit + __popcll(m & lt);
+        const int slot = nhit + lanesBelow(m);
         if (slot < kMaxHits) {
           V3 pc, nrm;
           double ov;
           contactOf(pn, sm, code >> 16, pc, nrm, ov);
-          ws.pc[0][slot] = pc.x;
-          ws.pc[1][slot] = pc.y;
-          ws.pc[2][slot] = pc.z;
-          ws.nrm[0][slot] = nrm.x;
-          ws.nrm[1][slot] = nrm.y;
-          ws.nrm[2][slot] = nrm.z;
-          ws.ov[slot] = ov;
+          const double v[7] = {pc.x, pc.y, pc.z, nrm.x, nrm.y, nrm.z, ov};
+#pragma unroll
+          for (int c = 0; c < 7; ++c) ws.c[c][slot] = v[c];
           ws.hit[slot] = code;
         }
         atomicAdd(&ws.total[code >> 16], 1);
@@ -1246,51 +1320,56 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
     if (!full) break;
   }
 
-  // the record and staging reservations and the mirror slots, one pair per
-  // lane, their atomics issued together (one round trip instead of three)
+  // the record reservations and the mirror slots, one pair per lane, their
+  // atomics issued together
   const bool open = units > 0;
   int total = open ? ws.total[lane] : 0;
   if (open && total == 0) emptyRange();
   if (nhit == 0) return;
-  const int pool = w % FDM_REC_POOLS;
-  const bool mirrored = SET != FDM_SET_WALL && total > 0 && T != A;
-  int base = 0, gbase = 0, mpos = 0;
-  const bool has = total > 0;
+  const bool has = total > 0, all = nhit <= kMaxHits;
+  int base = -1, gbase = 0, mpos = 0;
+  const int first = runScan(total) - total;  // first of the pair's contacts among the run's
   if (has) {
+    const LawRec lr = ws.law[lane];
+    const int A = lr.A, T = lr.T;
+    const bool mirrored = SET != FDM_SET_WALL && T != A;
+    int prevOff = lr.prevOff, prevCnt = lr.prevCnt;
+    const int pool = w % FDM_REC_POOLS;
     base = atomicAdd(S.pairs.recTotal + pool * FDM_REC_STRIDE, total);
-    gbase = atomicAdd(X.hitCount + pool * FDM_REC_STRIDE, total);
+    if (!all) gbase = atomicAdd(X.hitCount + pool * FDM_REC_STRIDE, total);
     if (mirrored) mpos = atomicAdd(&S.mirror.count[T], 1);
-    // the previous step's record range of the pair, for the law's header
-    if (X.lawHead && prevCnt < 0) prevCnt = findPrevPair(S, p, A, T, prevOff);
-    const int rCap = S.pairs.recCapacity / FDM_REC_POOLS, gCap = X.hitCapacity / FDM_REC_POOLS;
-    if (base + total > rCap || gbase + total > gCap) {
-      atomicOr(C.status, base + total > rCap ? FDM_STATUS_RECORD_OVERFLOW : FDM_STATUS_STAGING_OVERFLOW);
-      total = base = gbase = 0;
-    } else {
-      base += pool * rCap;
-      gbase += pool * gCap;
+    if (prevCnt < 0) prevCnt = findPrevPair(S, p, A, T, prevOff);
+    const int cap = S.pairs.recCapacity / FDM_REC_POOLS, gcap = X.hitCapacity / FDM_REC_POOLS;
+    if (base + total > cap || gbase + total > gcap) {
+      atomicOr(C.status, base + total > cap ? FDM_STATUS_RECORD_OVERFLOW : FDM_STATUS_STAGING_OVERFLOW);
+      total = 0;
     }
-    ws.gbase[lane] = total > 0 ? gbase : -1;
+    gbase += pool * gcap;
+    S.pairs.recOff[p] = total > 0 ? base + pool * cap : 0;
+    S.pairs.recCnt[p] = total;
+    base = total > 0 ? base + pool * cap : -1;
+    // (a pair whose reservation overflowed keeps its mirror slot, with no
+    // records and zero sums: the slot count and the list agree, and the
+    // target's fold adds nothing stale)
+    if (mirrored) {
+      if (mpos < S.mirror.capacity) S.mirror.list[(size_t)T * S.mirror.capacity + mpos] = p;
+      else atomicOr(C.status, FDM_STATUS_BUCKET_OVERFLOW);
+      if (total == 0)
+        for (int c = 0; c < 3; ++c) {
+          S.pairs.sumF[3 * (size_t)p + c] = 0.;
+          S.pairs.sumTB[3 * (size_t)p + c] = 0.;
+        }
+    }
+    ws.law[lane] = {base, first, prevOff, prevCnt, A, T, gbase};
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  if (nhit <= kMaxHits) {
-    // a contact's place: the contacts of its pair at lower nodes come first
-    const int code = lane < nhit ? ws.hit[lane] : INT_MAX;
-    int at = 0;
-    for (int h = 0; h < nhit; ++h) {
-      const int c = readlaneI(code, h);
-      at += (c >> 16) == (code >> 16) && c < code ? 1 : 0;
-    }
-    const int gb = lane < nhit ? ws.gbase[code >> 16] : -1;
-    if (gb >= 0)
-      stageHit(X.hitGeom + 8 * (size_t)(gb + at), {ws.pc[0][lane], ws.pc[1][lane], ws.pc[2][lane]},
-               {ws.nrm[0][lane], ws.nrm[1][lane], ws.nrm[2][lane]}, ws.ov[lane], code & 0xFFFF);
-  } else {
-    // more contacts than slots: each pair's chunks with contacts again, in
-    // node order
+
+  // more contacts than slots: each pair's chunks with contacts again, staged
+  // in node order
+  if (!all) {
     for (int j = 0; j < np; ++j) {
-      if (readlaneI(total, j) <= 0) continue;
-      int run = readlaneI(gbase, j);
+      if (ws.law[j].base < 0) continue;
+      int at = ws.law[j].staged;
       const int count = ldu(&C.pgeo.info[ws.ctx[j].geoA].nodeCount);
       for (unsigned long long cm = ws.chunks[j]; cm; cm &= cm - 1ull) {
         const int id = __builtin_ctzll(cm) * FDM_CHUNK + lane;
@@ -1302,160 +1381,70 @@ __device__ void sweepRun(const NarrowCommon& C, const NarrowSet& S, const Narrow
           V3 pc, nrm;
           double ov;
           contactOf(pn, sm, j, pc, nrm, ov);
-          stageHit(X.hitGeom + 8 * (size_t)(run + __popcll(m & lt)), pc, nrm, ov, id);
+          double* g = X.hitGeom + 8 * (size_t)(at + lanesBelow(m));
+          const double v[8] = {pc.x, pc.y, pc.z, nrm.x, nrm.y, nrm.z, ov, (double)id};
+#pragma unroll
+          for (int c = 0; c < 8; ++c) g[c] = v[c];
         }
-        run += __popcll(m);
+        at += __popcll(m);
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   }
-  if (!has) return;
-  S.pairs.recOff[p] = base;
-  S.pairs.recCnt[p] = total;
-  X.workHit[w] = gbase;
-  if (X.lawHead) {
-    int4* h = reinterpret_cast<int4*>(X.lawHead + 8 * (size_t)w);
-    h[0] = make_int4(total, base, gbase, A);
-    if (total > 0) h[1] = make_int4(T, prevOff, prevCnt, 0);
-  }
-  // (a pair whose reservation overflowed keeps its mirror slot, with no
-  // records and zero sums: the slot count and the list agree, and the
-  // target's fold adds nothing stale)
-  if (mirrored) {
-    if (mpos < S.mirror.capacity) S.mirror.list[(size_t)T * S.mirror.capacity + mpos] = p;
-    else atomicOr(C.status, FDM_STATUS_BUCKET_OVERFLOW);
-    if (total == 0)
-      for (int c = 0; c < 3; ++c) {
-        S.pairs.sumF[3 * (size_t)p + c] = 0.;
-        S.pairs.sumTB[3 * (size_t)p + c] = 0.;
+  // the contact law, one contact per lane, and the pairs' sums in node order
+  for (int b = 0; b < nhit; b += 64) {
+    asm volatile("" : "+v"(lane));  // (as above)
+    const int m = min(nhit - b, 64);
+    int code = INT_MAX, at = 0;
+    V3 pc = {0., 0., 0.}, nrm = {0., 0., 0.};
+    double ov = 0.;
+    if (all) {
+      // a contact's place: the contacts of its pair at lower nodes come first
+      if (lane < m) code = ws.hit[lane];
+      for (int h = 0; h < m; ++h) {
+        const int c = readlaneI(code, h);
+        at += (c >> 16) == (code >> 16) && c < code ? 1 : 0;
       }
+      pc = {ws.c[0][lane], ws.c[1][lane], ws.c[2][lane]};
+      nrm = {ws.c[3][lane], ws.c[4][lane], ws.c[5][lane]};
+      ov = ws.c[6][lane];
+    } else if (lane < m) {
+      int j = 0;
+      for (int q = 1; q < np; ++q)
+        if (ws.total[q] > 0 && ws.law[q].first <= b + lane) j = q;
+      at = b + lane - ws.law[j].first;
+      code = j << 16;
+      if (ws.law[j].base >= 0) {
+        const double* g = X.hitGeom + 8 * (size_t)(ws.law[j].staged + at);
+        pc = {g[0], g[1], g[2]};
+        nrm = {g[3], g[4], g[5]};
+        ov = g[6];
+        code |= (int)g[7];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (lane < m) {
+      const LawRec& lr = ws.law[code >> 16];
+      const int to = lr.first + at - b;
+      if (lr.base >= 0) lawContact<SET, MANY, SECTOR>(C, S, ws.ctx[code >> 16], lr, code & 0xFFFF, at, pc, nrm, ov, ws, to);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    for (int t = lane; t < 9 * np; t += 64) {
+      const int q = t / 9, c = t % 9;
+      const LawRec lr = ws.law[q];
+      if (lr.base < 0) continue;
+      const int end = lr.first + ws.total[q];
+      double* out = c < 3 ? S.pairs.sumF : c < 6 ? S.pairs.sumTA : S.pairs.sumTB;
+      out += 3 * (size_t)(p0 + q) + c % 3;
+      // (a pair's sum goes on from batch to batch)
+      double acc = lr.first < b && b < end ? *out : 0.;
+      for (int i = max(lr.first - b, 0); i < min(end - b, 64); ++i) acc += ws.c[c][i];
+      if (end > b && lr.first < b + 64) *out = acc;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
 }
 
-// Contact law of one kept pair with contacts (one thread): the previous
-// springs by (A, target, node), the linear spring-dashpot law per contact in
-// node order, and the pair's force and torque sums in that order.
-template <int SET>
-__device__ void lawPair(const NarrowCommon& C, const NarrowSet& S, const NarrowScratch& X, int w,
-                        int p) {
-  int cnt, base, gbase, A, T, prevOff = 0, prevCnt;
-  if (X.lawHead) {
-    const int4 h0 = ldu(reinterpret_cast<const int4*>(X.lawHead + 8 * (size_t)w));
-    cnt = h0.x;
-    if (cnt <= 0) return;
-    const int4 h1 = ldu(reinterpret_cast<const int4*>(X.lawHead + 8 * (size_t)w + 4));
-    base = h0.y;
-    gbase = h0.z;
-    A = h0.w;
-    T = h1.x;
-    prevOff = h1.y;
-    prevCnt = h1.z;
-  } else {
-    cnt = S.pairs.recCnt[p];
-    if (cnt <= 0) return;
-    base = S.pairs.recOff[p];
-    gbase = X.workHit[w];
-    A = ldu(S.pairs.pairA + p);
-    T = ldu(S.pairs.pairT + p);
-    prevCnt = findPrevPair(S, p, A, T, prevOff);
-  }
-  const int n = C.P.n;
-  const fdm_template& tA = tmplOf(C.pgeo, ldu(C.P.geo + A));
-  const PairFrame fr = pairFrame<SET>(C, S, A);
-  const V3 xA = detectPosA<SET>(C, fr, A);
-  Target tg;
-  V3 armB;
-  resolveTarget<SET>(C, S, p, T, fr, tg, armB);
-  const V3 armA = SET == FDM_SET_GHOST ? xA : wrappedArm(xA, *fr.pgrid, fr.periodic);
-  // material constants of the pair (contactKernel.cu:79-110,167-193,243-274)
-  const fdm_material Mi = matOf(C.pmat, ldu(C.P.mat + A));
-  const double invMi = tA.invMass;
-  double kn = 0., ks = 0., effM = 0., mu, diss;
-  V3 vB, wB;
-  if (SET == FDM_SET_WALL) {
-    const fdm_material Mw = matOf(C.wmat, ldu(C.W.mat + T));
-    if (invMi > 0.) effM = 1. / invMi;
-    mu = fmin(Mi.mu, Mw.mu);
-    diss = Mi.e <= Mw.e ? Mi.dissipation : Mw.dissipation;
-    kn = Mi.kn;
-    ks = Mi.ks;
-    vB = ld3R(C.W.v, C.W.n, T);
-    wB = ld3R(C.W.w, C.W.n, T);
-  } else {
-    const fdm_material Mj = matOf(C.pmat, ldu(C.P.mat + T));
-    const double invMj = tg.t.invMass;
-    if (Mi.kn > 0. && Mj.kn > 0.) kn = Mi.kn * Mj.kn / (Mi.kn + Mj.kn);
-    if (Mi.ks > 0. && Mj.ks > 0.) ks = Mi.ks * Mj.ks / (Mi.ks + Mj.ks);
-    if (invMi > 0. || invMj > 0.) effM = 1. / (invMi + invMj);
-    diss = Mi.e <= Mj.e ? Mi.dissipation : Mj.dissipation;
-    mu = fmin(Mi.mu, Mj.mu);
-    vB = SET == FDM_SET_GHOST && S.ghostVel ? ldd3R(S.ghostVel + 3 * (size_t)S.pairs.pairG[p])
-                                            : forceVel(C, fr, T);
-    wB = ld3R(C.P.w, n, T);  // a sector image keeps the real spin (contactKernel.cu:258)
-  }
-  const V3 vA = forceVel(C, fr, A);
-  const V3 wA = ld3R(C.P.w, n, A);
-  V3 SF = {0., 0., 0.}, STA = {0., 0., 0.}, STB = {0., 0., 0.};
-  // The pair's previous records are in node order, as its staged contacts
-  // are: walk both in step rather than search per contact; and load the next
-  // contact's staged geometry one iteration ahead.
-  int j = prevOff;
-  const int jEnd = prevOff + prevCnt;
-  fdm_record pr{};
-  if (j < jEnd) pr = ldu(S.prev.rec + j);
-  double gn[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) gn[c] = ldu(X.hitGeom + 8 * (size_t)gbase + c);
-  for (int h = 0; h < cnt; ++h) {
-    double g[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) g[c] = gn[c];
-    if (h + 1 < cnt) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) gn[c] = ldu(X.hitGeom + 8 * (size_t)(gbase + h + 1) + c);
-    }
-    const V3 pc = {g[0], g[1], g[2]};
-    const V3 nrm = {g[3], g[4], g[5]};
-    const double ov = g[6];
-    const int k = (int)g[7];
-    V3 F = {0., 0., 0.};
-    while (j < jEnd && pr.node < k) {
-      ++j;
-      if (j < jEnd) pr = ldu(S.prev.rec + j);
-    }
-    V3 spring = j < jEnd && pr.node == k ? recordSpring(pr) : V3{0., 0., 0.};
-    if (C.updateSprings) {
-      const V3 vc = vsub(vadd(vA, vcross(wA, vsub(pc, armA))), vadd(vB, vcross(wB, vsub(pc, armB))));
-      linearContact(F, spring, vc, nrm, ov, C.dt, kn, ks, mu, diss, effM);
-    }
-    const V3 TA = vcross(vsub(pc, armA), F);
-    const V3 TB = vcross(vsub(pc, armB), vneg(F));
-    SF = vadd(SF, F);
-    STA = vadd(STA, TA);
-    STB = vadd(STB, TB);
-    const int r = base + h;
-    S.pairs.rec[r] = makeRecord(spring, k);
-    if (C.dbgPoint) {
-      C.dbgPoint[3 * r] = pc.x;
-      C.dbgPoint[3 * r + 1] = pc.y;
-      C.dbgPoint[3 * r + 2] = pc.z;
-      C.dbgNormal[3 * r] = nrm.x;
-      C.dbgNormal[3 * r + 1] = nrm.y;
-      C.dbgNormal[3 * r + 2] = nrm.z;
-      C.dbgOverlap[r] = ov;
-    }
-  }
-  double* f = S.pairs.sumF + 3 * (size_t)p;
-  double* ta = S.pairs.sumTA + 3 * (size_t)p;
-  double* tb = S.pairs.sumTB + 3 * (size_t)p;
-  f[0] = SF.x; f[1] = SF.y; f[2] = SF.z;
-  ta[0] = STA.x; ta[1] = STA.y; ta[2] = STA.z;
-  tb[0] = STB.x; tb[1] = STB.y; tb[2] = STB.z;
-}
-
-// Pair-level cull of every set's candidates at this step's positions (one
-// thread per pair): the pair is kept only if a node of A can still reach
-// the target (the broad-phase tests without the skin). Culled pairs get
-// empty record ranges; kept pairs go to the work list as (p << 3 | set).
 // Candidate pairs of all sets in one index space: set k holds the indices
 // [start[k], start[k + 1]).
 struct SetStarts {
@@ -1483,7 +1472,7 @@ __device__ __forceinline__ SetStarts setStarts(const NarrowMulti& a) {
 // stretches of 64 consecutive pairs (stretch q on XCD q mod 8), its waves
 // sharing out its runs. Items are taken from the end: the image sets (whose
 // box test lets many pairs through) before the wall and particle sets.
-template <bool MANY>
+template <bool MANY, bool SECTOR>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 kSweep(NarrowMulti a, NarrowScratch x) {
   __shared__ SweepSlots slots;
@@ -1522,14 +1511,14 @@ kSweep(NarrowMulti a, NarrowScratch x) {
     const NarrowSet& s = a.s[k];
     const int p0 = (it - i0) << shift;
     const int len = min(run, np - p0);
-    if (s.kind == FDM_SET_PARTICLE) sweepRun<FDM_SET_PARTICLE, MANY>(a.c, s, x, g0 + p0, p0, len, lane, slots);
-    else if (s.kind == FDM_SET_WALL) sweepRun<FDM_SET_WALL, MANY>(a.c, s, x, g0 + p0, p0, len, lane, slots);
-    else sweepRun<FDM_SET_GHOST, MANY>(a.c, s, x, g0 + p0, p0, len, lane, slots);
+    if (s.kind == FDM_SET_PARTICLE) sweepRun<FDM_SET_PARTICLE, MANY, SECTOR>(a.c, s, x, g0 + p0, p0, len, lane, slots);
+    else if (s.kind == FDM_SET_WALL) sweepRun<FDM_SET_WALL, MANY, SECTOR>(a.c, s, x, g0 + p0, p0, len, lane, slots);
+    else sweepRun<FDM_SET_GHOST, MANY, SECTOR>(a.c, s, x, g0 + p0, p0, len, lane, slots);
   }
 }
 
 // The pre-cull, the sweep and the contact law in one pass: one wave per
-// candidate pair (WAVES waves per workgroup) as kCullSweep, whose wave then
+// candidate pair (WAVES waves per workgroup) whose wave then
 // applies the law to its pair's contacts (one contact per lane) and folds
 // the pair sums in node order (processPair); no staging, no second kernel.
 template <int WAVES>
@@ -1557,30 +1546,6 @@ __global__ void __launch_bounds__(64 * WAVES) kCullSweepLaw(NarrowMulti a) {
       processPair<FDM_SET_WALL, true>(a.c, s, p, lane, slots[wave], pool);
     else
       processPair<FDM_SET_GHOST, true>(a.c, s, p, lane, slots[wave], pool);
-  }
-}
-
-// The contact law over the candidate index space of kCullSweep (one thread
-// per candidate; culled pairs and pairs without contacts return at once).
-__global__ void __launch_bounds__(256) kContactLawAll(NarrowMulti a, NarrowScratch x) {
-  const int on = gateValue(a.gate, a.s[0].pairs.total);
-  const SetStarts st = setStarts(a);
-  const int total = st.v[kMaxSets];
-  asm volatile("" ::"s"(on), "s"(total));  // (loaded together)
-  if (!on) return;
-  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
-    int k = 0, base = 0;
-#pragma unroll
-    for (int q = 1; q < kMaxSets; ++q)  // constant indices: the starts stay scalar
-      if (g >= st.v[q]) {
-        k = q;
-        base = st.v[q];
-      }
-    const NarrowSet& s = a.s[k];
-    const int p = g - base;
-    if (s.kind == FDM_SET_PARTICLE) lawPair<FDM_SET_PARTICLE>(a.c, s, x, g, p);
-    else if (s.kind == FDM_SET_WALL) lawPair<FDM_SET_WALL>(a.c, s, x, g, p);
-    else lawPair<FDM_SET_GHOST>(a.c, s, x, g, p);
   }
 }
 
@@ -1803,12 +1768,7 @@ extern "C" int fdm_launchNarrowPhaseSets(const fdm_narrowphase_args* sets, int n
   }
   if (cap > ws->workCapacity || cap >= (1ll << 28)) return FDM_EINVAL;
   for (int i = nsets; i < kMaxSets; ++i) k.s[i] = k.s[0];
-  NarrowScratch x;
-  x.workHit = ws->workHit;
-  x.lawHead = ws->workList;
-  x.hitGeom = ws->hitGeom;
-  x.hitCapacity = ws->hitCapacity;
-  x.hitCount = ws->hitCount;
+  const NarrowScratch x = {ws->hitGeom, ws->hitCapacity, ws->hitCount};
   fdm_tuning tu = tuning();
   if (ws->tuning && !completeTuning(*ws->tuning, tu)) return FDM_EINVAL;
   // geometry without the culling tables of sweepPair: the kernel that culls
@@ -1826,10 +1786,9 @@ extern "C" int fdm_launchNarrowPhaseSets(const fdm_narrowphase_args* sets, int n
     return launchStatus();
   }
   const int waves = std::max(kXcds, persistentBlocks(1) * tu.sweepWavesPerCU / 32 / kXcds * kXcds);
-  if (sets[0].inst.count > 0) hipLaunchKernelGGL(kSweep<true>, dim3(waves), dim3(64), 0, stream, k, x);
-  else hipLaunchKernelGGL(kSweep<false>, dim3(waves), dim3(64), 0, stream, k, x);
-  hipLaunchKernelGGL(kContactLawAll, dim3(persistentBlocks(tu.lawBlock / 64)), dim3(tu.lawBlock), 0,
-                     stream, k, x);
+  if (sets[0].inst.count > 0) hipLaunchKernelGGL((kSweep<true, false>), dim3(waves), dim3(64), 0, stream, k, x);
+  else if (sets[0].periodic.sector) hipLaunchKernelGGL((kSweep<false, true>), dim3(waves), dim3(64), 0, stream, k, x);
+  else hipLaunchKernelGGL((kSweep<false, false>), dim3(waves), dim3(64), 0, stream, k, x);
   return launchStatus();
 }
 

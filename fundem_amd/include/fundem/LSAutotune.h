@@ -113,13 +113,6 @@ class LSAutotuner {
     }
     bestCost = pick(group, trialSteps, best, "lawMode");
     group.clear();
-    for (int b : {64, 128, 256}) {
-      TuneChoice c = best;
-      c.launch.lawBlock = b;
-      group.push_back(c);
-    }
-    bestCost = pick(group, trialSteps, best, "lawBlock");
-    group.clear();
     for (int b : {128, 256, 512}) {
       TuneChoice c = best;
       c.launch.reduceBlock = b;

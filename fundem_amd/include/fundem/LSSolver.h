@@ -344,8 +344,8 @@ class LSSolver {
       for (int s = 0; s < 3; ++s)
         if (periodic_.active(s)) cap += std::max<long long>(4 * (long long)N, 1024);
       if (cap >= (1ll << 28)) throw std::invalid_argument("contact capacities too large");
-      workHit_.allocate((size_t)cap, false);
-      lawHead_.allocate(8 * (size_t)cap, false);
+      workCapacity_ = (int)cap;
+      listTmp_.allocate(2 * (size_t)cap, false);
       // staged contacts of one step, all sets together: room for every
       // active set's records
       int activeSets = 1 + (W ? 1 : 0);
@@ -1265,9 +1265,8 @@ class LSSolver {
     b.maxBoxReach = maxBoxReach_;
     b.full = d.rebuild ? 1 : 0;
     b.touch = touch_.get();
-    // (the law's headers are written by the sweep that follows)
-    b.tmp = lawHead_.get();
-    b.tmpWords = (long long)lawHead_.size();
+    b.tmp = listTmp_.get();
+    b.tmpWords = (long long)listTmp_.size();
     b.tmpOff = buildOff_.get();
     b.status = status_.get();
     Timer t(this, "list_build");
@@ -1383,10 +1382,9 @@ class LSSolver {
     {
       Timer t(this, "narrow");
       fdm_narrow_workspace w;
-      w.workList = lawHead_.get();
-      w.workCapacity = (int)workHit_.size();
+      w.workCapacity = workCapacity_;
       w.workCount = nullptr;
-      w.workHit = workHit_.get();
+      w.workHit = listTmp_.get();
       w.hitGeom = hitGeom_.get();
       w.hitCapacity = hitCapacity_;
       w.hitCount = hitCount_.get();
@@ -1721,7 +1719,8 @@ class LSSolver {
   DeviceBuffer<fdm_grid> instPGrid_, instWGrid_;
   DeviceBuffer<long long> instPOff_, instWOff_;
   DeviceBuffer<fdm_periodic> instPeriodic_;
-  DeviceBuffer<int> workHit_, hitCount_, lawHead_;
+  DeviceBuffer<int> hitCount_, listTmp_;
+  int workCapacity_ = 0;
   DeviceBuffer<double> hitGeom_;
   int hitCapacity_ = 0;
   fdm_tuning tuning_{};

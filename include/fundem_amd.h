@@ -607,34 +607,32 @@ typedef struct {
 int fdm_launchNarrowPhase(const fdm_narrowphase_args* args, hipStream_t stream);
 /* Scratch of fdm_launchNarrowPhaseSets. */
 typedef struct {
-  int* workList;               /* [8 * workCapacity] or NULL: per candidate pair, the header
-                                  the sweep writes for the contact law (record count, first
-                                  record, first staged contact, A, target, previous record
-                                  range), so that the law starts from one load */
+  int* workList;               /* unused (may be NULL); kept for the layout */
   int workCapacity;            /* at least the sum of the sets' pair capacities */
   int* workCount;              /* unused (may be NULL); kept for the layout */
-  int* workHit;                /* [workCapacity] first staged contact of each candidate pair */
-  double* hitGeom;             /* [8 * hitCapacity] staged contacts */
+  int* workHit;                /* not NULL; unused, kept for the layout */
+  double* hitGeom;             /* [8 * hitCapacity] staged contacts (runs of pairs with more
+                                  contacts than one wave holds, 64) */
   int hitCapacity;             /* staged contacts, split into FDM_REC_POOLS pools */
   int* hitCount;               /* [FDM_REC_COUNTERS] staged contacts per pool */
   const struct fdm_tuning_s* tuning; /* launch shapes (NULL: the process default) */
 } fdm_narrow_workspace;
 /* No counterpart in the reference: the narrow phase of up to five sets at
- * once, in two kernels over the candidate pairs of all sets (set k's pairs
- * follow those of sets 0..k-1). The first (runs of one to eight pairs per
- * wave) tests whether the pairs' bodies can still touch at this step's
- * positions (the broad-phase tests without the skin), gives a rejected pair
- * empty record ranges, and otherwise culls node groups and nodes against the
- * target's cell codes, tests the rest exactly, stages every contact's point,
- * normal and overlap in hitGeom and reserves the pair's records; the second
- * (one thread per candidate pair) applies the contact law to the staged
- * contacts in node order and writes the records and the pair sums. Geometry
- * without the culling tables (fdm_geometry.groups, groupNodes, cells) runs
- * as lawMode 2. Shared fields (bodies, geometry, materials, pgrid, periodic,
- * dt, updateSprings, status, dbg*) come from sets[0]. Unlike
- * fdm_launchNarrowPhase it clears no counter: the sets' record counters
- * (pairs.recTotal) and the hitCount pools must be zero at launch. Candidate
- * g reserves its records and staged contacts from pool g % FDM_REC_POOLS. */
+ * once, in one kernel over the candidate pairs of all sets (set k's pairs
+ * follow those of sets 0..k-1). A wave takes a run of one to eight pairs. It
+ * tests whether their bodies can still touch at this step's positions (the
+ * broad-phase tests without the skin) and gives a rejected pair empty record
+ * ranges; otherwise it culls node groups and nodes against the target's cell
+ * codes, tests the rest exactly, reserves the pairs' records, applies the
+ * contact law with one contact per lane and adds each pair's forces and
+ * torques in node order. A run with more than 64 contacts stages them in
+ * hitGeom first. Geometry without the culling tables (fdm_geometry.groups,
+ * groupNodes, cells) runs as lawMode 2. Shared fields (bodies, geometry,
+ * materials, pgrid, periodic, dt, updateSprings, status, dbg*) come from
+ * sets[0]. Unlike fdm_launchNarrowPhase it clears no counter: the sets' record
+ * counters (pairs.recTotal) and the hitCount pools must be zero at launch.
+ * Candidate g reserves its records and staged contacts from pool
+ * g % FDM_REC_POOLS. */
 int fdm_launchNarrowPhaseSets(const fdm_narrowphase_args* sets, int nsets,
                               const fdm_narrow_workspace* ws, hipStream_t stream);
 
@@ -745,11 +743,11 @@ typedef struct fdm_tuning_s {
                            sweep has one wave per workgroup) */
   int sweepWavesPerCU;  /* node-sweep grid size, in waves per CU: 4..128 (default 16, as many
                            as lawMode 1's sweep keeps resident) */
-  int lawBlock;         /* contact-law threads per workgroup: 64, 128 or 256 */
+  int lawBlock;         /* 64, 128 or 256: accepted, without effect (the sweep's wave takes
+                           the contact law) */
   int reduceBlock;      /* reduction threads per workgroup: a multiple of 64 up to 1024 */
-  int lawMode;          /* contact law of the narrow phase: 1 in a kernel of its own (one
-                           thread per candidate pair, contacts staged in the workspace),
-                           2 in the sweep's wave (one contact per lane) */
+  int lawMode;          /* narrow phase: 1 runs of one to eight pairs per wave, culled by node
+                           groups and SDF cell codes; 2 one pair per wave, culled by chunk */
   int nodesPerLane;     /* 1, 2 or 3: accepted, without effect (every sweep collects the
                            nodes that pass the cell test before it fetches SDF values) */
   int wallGroups;       /* 0, 1 or 2: accepted, without effect (every set is swept several

@@ -102,3 +102,31 @@ def test_run_lengths_equal_the_chunk_sweep(counts):
     for u, v in zip(ca, cb):
         for key in ("A", "B", "k", "spring"):
             assert np.array_equal(u[key], v[key]), key
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("n,nodes,steps", [(2, 1500, 60), (2, 4000, 60), (12, 900, 60), (40, 1500, 40)])
+def test_contacts_of_a_run_around_one_wave_bitexact(n, nodes, steps, precision):
+    """Blunt bodies pressed into each other and the floor: contacts of a run
+    from a few (one per lane) to several batches of 64 staged in memory, pairs
+    that cross a batch's edge, new and kept springs."""
+    from fundem_amd import Solver
+    tm = [gen.superellipsoid_template(1e-3, 0.9e-3, 1.1e-3, 8.0, 8.0, n_grid=16, n_nodes=nodes)]
+    scn = squeezed(n=n, templates=tm, kn=20.0)
+    scn = dataclasses.replace(scn, x=scn.x.mean(0) + 0.76 * (scn.x - scn.x.mean(0)), v=0.02 * scn.v)
+    g = Solver(precision=precision)
+    g.set_capacity(24, 400)
+    W.apply(scn, g)
+    o = po.OracleSim(precision == "fp32", True)
+    W.apply(scn, o)
+    most = []
+    for i in range(1, steps + 1, 4):
+        g.step(4)
+        o.step(4)
+        assert_states_equal(g.state(), o.state(), f"step {i}")
+        assert_contacts_equal(g, o, f"step {i}")
+        c = o.contacts(po.SET_PP)
+        most.append(int(np.unique(np.stack([c["A"], c["B"]]), axis=1, return_counts=True)[1].max()) if c["A"].size else 0)
+    print(f"{n} {nodes}: contacts of the fullest pair {min(most)}..{max(most)}", flush=True)
+    assert g.status() == 0 and max(most) > 0
+    g.close()
