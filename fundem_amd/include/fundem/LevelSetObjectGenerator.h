@@ -2,8 +2,8 @@
 // (LevelSetObject::TriangleMeshParticle, LevelSetObjectGenerator.h:382-951,
 // with Base::buildGrid / buildGridByResolution / outputGridVTU,
 // LevelSetObjectGenerator.h:56-379). Same class, method names, arguments and
-// results; the grid is sampled on the GPU by fdm_launchMeshSignedDistanceGrid
-// (one thread per grid node over all triangles) instead of a host loop over
+// results; the grid is sampled on the GPU by
+// fdm_launchMeshSignedDistanceGridWith instead of a host loop over
 // a SAH-BVH. Grid placement (padding, snapping to multiples of the spacing,
 // node counts) is computed on the host exactly as the reference does.
 #pragma once
@@ -134,9 +134,11 @@ class TriangleMeshParticle {
     sdf.allocate(N, false);
     const double origin[3] = {lo.x, lo.y, lo.z};
     const int size[3] = {nx, ny, nz};
-    fundem::fdmCheck(fdm_launchMeshSignedDistanceGrid(tri.get(), (int)triangleVertexIndex_.size(),
-                                                      origin, h, size,
-                                                      levelSetPositiveInside_ ? 1 : 0, sdf.get(), s),
+    const int nt = (int)triangleVertexIndex_.size();
+    fundem::DeviceBuffer<char> work;
+    work.allocate(std::max<size_t>(fdm_meshGridWorkspaceBytes(nt, size), 1), false);
+    fundem::fdmCheck(fdm_launchMeshSignedDistanceGridWith(tri.get(), nt, origin, h, size, levelSetPositiveInside_ ? 1 : 0,
+                                                          sdf.get(), work.get(), work.size(), s),
                      "mesh signed distance grid");
     g.gridNodeSignedDistance = sdf.toHost(s, N);
     gridInfo_ = std::move(g);

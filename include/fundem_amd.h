@@ -858,6 +858,15 @@ int fdm_launchAdjointStep(const fdm_adjoint_step_args* args, void* ws, size_t ws
 int fdm_launchMeshSignedDistanceGrid(const double* triangles, int numTriangles,
                                      const double* origin, double spacing, const int* size,
                                      int positiveInside, double* sdf, hipStream_t stream);
+/* The same with a workspace of fdm_meshGridWorkspaceBytes (0: none is needed):
+ * signs by ray crossings and nearest triangles by boxes instead of every
+ * triangle's solid angle and distance at every node. The values are the
+ * same. */
+size_t fdm_meshGridWorkspaceBytes(int numTriangles, const int* size);
+int fdm_launchMeshSignedDistanceGridWith(const double* triangles, int numTriangles,
+                                         const double* origin, double spacing, const int* size,
+                                         int positiveInside, double* sdf, void* workspace,
+                                         size_t workspaceBytes, hipStream_t stream);
 /* TriangleMeshParticle::evaluateImplicitFunctionValueAndGradient
  * (LevelSetObjectGenerator.h:888-914) at numPoints device points [3*numPoints]:
  * value [numPoints] and gradient [3*numPoints]. */
