@@ -20,8 +20,9 @@
 // target (one pair per A, target and set), so the lists are deterministic.
 // Measured against a sort, a scan and two searches (count, write; one thread
 // per particle) per set, 118 launches: a step of 110592 periodic particles
-// that builds lists every 1.6 steps 473 -> 240 us, of 216 particles (a build
-// every 24 steps) 90.7 -> 69.8 us.
+// that builds lists every 1.6 steps 473 -> 240 us (195 with the sweep's law
+// and kBuildBodies as they are), of 216 particles (a build every 24 steps)
+// 90.7 -> 69.8 us.
 #include <algorithm>
 
 #include "cull_device.hpp"
@@ -132,8 +133,13 @@ __global__ void __launch_bounds__(kBodyThreads) kBuildBodies(BuildK k, int parti
     markCells(sorted, W, k.wtable, k.wgrid.num);
     return;
   }
-  __shared__ int cnt[3], base[3];
+  // the workgroup's images of each set: their number and first slot, and the
+  // box of their cells (one global atomic each per workgroup: taken per image,
+  // in turn, they made up most of this kernel's time: 110592 particles 49.9 ->
+  // 18.7 us, 216 particles 28.7 -> 13.7 us)
+  __shared__ int cnt[3], base[3], box[3][6];
   if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
+  if (threadIdx.x < 18) box[threadIdx.x / 6][threadIdx.x % 6] = threadIdx.x % 6 < 3 ? INT_MAX : INT_MIN;
   __syncthreads();
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int n = k.P.n;
@@ -171,40 +177,55 @@ __global__ void __launch_bounds__(kBodyThreads) kBuildBodies(BuildK k, int parti
     k.touch[i] = keep | (k.full && k.bondStart && k.bondStart[i + 1] > k.bondStart[i] ? FDM_TOUCH_BOND : 0);
   }
   if (!(k.periodic.x || k.periodic.y)) return;
+  // lists are built by the clamped geometric cell (monotone in the position);
+  // the reference's ghost cell id decides the stencil rule
+  long long cell[3] = {0, 0, 0};
 #pragma unroll
-  for (int s = 0; s < 3; ++s)
-    if (bits >> s & 1) mine[s] = atomicAdd(&cnt[s], 1);
+  for (int s = 0; s < 3; ++s) {
+    if (!(bits >> s & 1)) continue;
+    mine[s] = atomicAdd(&cnt[s], 1);
+    const I3 c = clampedCell(gp[s], g);
+    cell[s] = off + lin3(c, gsize(g));
+    const int v[3] = {c.x, c.y, c.z};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      atomicMin(&box[s][a], v[a]);
+      atomicMax(&box[s][3 + a], v[a]);
+    }
+  }
   __syncthreads();
   if (threadIdx.x < 3 && cnt[threadIdx.x] > 0) base[threadIdx.x] = atomicAdd(k.ghosts[threadIdx.x].count, cnt[threadIdx.x]);
+  if (threadIdx.x >= 64 && threadIdx.x < 64 + 18) {
+    const int s = (threadIdx.x - 64) / 6, a = (threadIdx.x - 64) % 6;
+    if (cnt[s] > 0) {
+      if (a < 3) atomicMin(&k.ghosts[s].cellBox[a], box[s][a]);
+      else atomicMax(&k.ghosts[s].cellBox[a], box[s][a]);
+    }
+  }
   __syncthreads();
+  int slot[3], next[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    if (!(bits >> s & 1)) continue;
+    slot[s] = base[s] + mine[s];
+    if (slot[s] >= k.ghosts[s].capacity) {
+      atomicOr(k.status, FDM_STATUS_GHOST_OVERFLOW);
+      bits &= ~(1 << s);
+    } else {
+      next[s] = atomicExch(&k.ghosts[s].table.cellStart[cell[s]], slot[s]);
+    }
+  }
 #pragma unroll
   for (int s = 0; s < 3; ++s) {
     if (!(bits >> s & 1)) continue;
     const fdm_ghosts& G = k.ghosts[s];
-    const int slot = base[s] + mine[s];
-    if (slot >= G.capacity) {
-      atomicOr(k.status, FDM_STATUS_GHOST_OVERFLOW);
-      continue;
-    }
-    G.realId[slot] = i;
-    G.pos[3 * slot] = gp[s].x;
-    G.pos[3 * slot + 1] = gp[s].y;
-    G.pos[3 * slot + 2] = gp[s].z;
-    G.table.hashValue[slot] = ghostCellHash(gp[s], g);
-    // lists are built by the clamped geometric cell (monotone in the
-    // position); the reference's ghost cell id above decides the stencil rule
-    const I3 c = clampedCell(gp[s], g);
-    const long long cell = off + lin3(c, gsize(g));
-    G.table.prevKey[slot] = (int)(cell + 1);
-    G.table.sortIndex[slot] = atomicExch(&G.table.cellStart[cell], slot);
-    const int b[3] = {c.x, c.y, c.z};
-    for (int a = 0; a < 3; ++a) {
-      // (bounds only widen, so a bound read late costs an atomic, no more)
-      if (b[a] < __hip_atomic_load(&G.cellBox[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMin(&G.cellBox[a], b[a]);
-      if (b[a] > __hip_atomic_load(&G.cellBox[3 + a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&G.cellBox[3 + a], b[a]);
-    }
+    G.realId[slot[s]] = i;
+    G.pos[3 * slot[s]] = gp[s].x;
+    G.pos[3 * slot[s] + 1] = gp[s].y;
+    G.pos[3 * slot[s] + 2] = gp[s].z;
+    G.table.hashValue[slot[s]] = ghostCellHash(gp[s], g);
+    G.table.prevKey[slot[s]] = (int)(cell[s] + 1);
+    G.table.sortIndex[slot[s]] = next[s];
   }
 }
 
