@@ -409,21 +409,7 @@ int fdmx_status(void* s, unsigned* out) {
 int fdmx_get_state(void* s, double* x, double* v, double* w, double* q, double* f, double* t) {
   return guarded([&] {
     auto* S = static_cast<BoundSolver*>(s);
-    S->downloadState();
-    auto& P = S->getLSParticle();
-    const size_t n = P.num();
-    for (size_t i = 0; i < n; ++i) {
-      const double3 a = P.positionHostRef()[i], b = P.velocityHostRef()[i],
-                    c = P.angularVelocityHostRef()[i], d = P.forceHostRef()[i],
-                    e = P.torqueHostRef()[i];
-      const quaternion r = P.orientationHostRef()[i];
-      if (x) { x[3 * i] = a.x; x[3 * i + 1] = a.y; x[3 * i + 2] = a.z; }
-      if (v) { v[3 * i] = b.x; v[3 * i + 1] = b.y; v[3 * i + 2] = b.z; }
-      if (w) { w[3 * i] = c.x; w[3 * i + 1] = c.y; w[3 * i + 2] = c.z; }
-      if (f) { f[3 * i] = d.x; f[3 * i + 1] = d.y; f[3 * i + 2] = d.z; }
-      if (t) { t[3 * i] = e.x; t[3 * i + 1] = e.y; t[3 * i + 2] = e.z; }
-      if (q) { q[4 * i] = r.q0; q[4 * i + 1] = r.q1; q[4 * i + 2] = r.q2; q[4 * i + 3] = r.q3; }
-    }
+    S->downloadState({x, v, w, q, f, t});
   });
 }
 long long fdmx_num_particles(void* s) {

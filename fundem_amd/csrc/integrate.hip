@@ -127,6 +127,21 @@ __global__ void kCommitStateInstances(const double* x, int n, fdm_instances I, i
   }
 }
 
+// State planes to rows of FP64, one value per thread in the order of `out`,
+// so that the writes, which go to host memory over the bus, are whole lines.
+__global__ void __launch_bounds__(256) kPackState(fdm_bodies b, int first, int count, double* out) {
+  const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x, three = 3 * (size_t)count;
+  if (e >= 19 * (size_t)count) return;
+  const int which = e < 5 * three ? (int)(e / three) : 5;
+  const size_t r = e - which * three;
+  const int width = which < 5 ? 3 : 4;
+  const size_t at = r % width * b.n + first + r / width;
+  double v;
+  if (which == 0) v = b.x[at];
+  else v = (double)(which == 1 ? b.v : which == 2 ? b.w : which == 3 ? b.F : which == 4 ? b.T : b.q)[at];
+  out[e] = v;
+}
+
 __global__ void kSkinDecide(fdm_skin s) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   decideStep(s, 0.f, 0);
@@ -370,6 +385,14 @@ int stepBeginSetup(const fdm_step_begin_args* args, const fdm_skin* skin, void* 
 }
 
 }  // namespace
+
+extern "C" int fdm_launchPackState(fdm_bodies bodies, int first, int count, double* out, hipStream_t stream) {
+  if (first < 0 || count < 0 || first > bodies.n - count) return FDM_EINVAL;
+  if (count == 0) return FDM_OK;
+  if (!out || !bodies.x || !bodies.v || !bodies.w || !bodies.q || !bodies.F || !bodies.T) return FDM_EINVAL;
+  hipLaunchKernelGGL(kPackState, dim3(blocksFor(19ll * count, 256)), dim3(256), 0, stream, bodies, first, count, out);
+  return launchStatus();
+}
 
 extern "C" int fdm_launchStepBegin(const fdm_step_begin_args* args, const fdm_skin* skin,
                                    void* workspace, size_t workspaceBytes, hipStream_t stream) {

@@ -426,8 +426,8 @@ class LSSolver {
     }
   }
   // Bodies and bonds only.
-  void downloadState() {
-    particles_.finalize(stream_);
+  void downloadState(const StateArrays& out = {}) {
+    particles_.finalize(stream_, out);
     walls_.finalize(stream_);
     bonds_.finalize(stream_);
     hipCheck(hipStreamSynchronize(stream_), "download");

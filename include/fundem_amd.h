@@ -680,6 +680,11 @@ size_t fdm_buildListsWorkspaceBytes(size_t n);
 int fdm_launchBuildLists(const fdm_build_args* args, void* workspace, size_t workspaceBytes,
                          hipStream_t stream);
 
+/* State of bodies first to first + count - 1 as rows for the host, FP64: x v w
+ * F T (3 each) and q (4), all rows of one quantity before the next, into
+ * out [19 * count] (device or mapped host memory). */
+int fdm_launchPackState(fdm_bodies bodies, int first, int count, double* out, hipStream_t stream);
+
 /* Add one to a device counter (the step index a captured graph replays). */
 int fdm_incrementCounter(int* counter, hipStream_t stream);
 

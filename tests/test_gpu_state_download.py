@@ -1,0 +1,33 @@
+"""Body state to the host in blocks of 8192 bodies through up to eight pinned
+slots, one thread each (LSParticle::finalize): every body's values in its row,
+for one block, its edges, two blocks, and more blocks than slots."""
+import numpy as np
+import pytest
+
+from fundem_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("n", [1, 2, 8191, 8192, 8193, 65536, 73729])
+def test_every_value_in_its_place(n, precision):
+    from fundem_amd import Solver
+    scn = W.cluster(n=n, seed=3, templates=W.superellipsoid_family(2, 5, n_grid=8, n_nodes=20))
+    real = np.float32 if precision == "fp32" else np.float64
+    g = Solver(precision=precision)
+    W.apply(scn, g)
+    a = g.state()
+    assert np.array_equal(a["x"], scn.x)
+    for key in ("v", "w"):
+        assert np.array_equal(a[key], getattr(scn, key).astype(real).astype(float)), key
+    # (orientations are normalised first: a few roundings of components up to 1)
+    assert np.abs(a["q"] - scn.q).max() <= 4 * np.finfo(real).eps
+    g.step(3)
+    b, c = g.state(), g.state()
+    for key in b:
+        assert np.array_equal(b[key], c[key]), key
+    # weight and velocity agree: no body of another row
+    assert np.isfinite(b["F"]).all() and np.isfinite(b["T"]).all()
+    assert not np.array_equal(b["x"], a["x"])
+    g.close()
