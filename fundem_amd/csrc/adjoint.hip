@@ -62,23 +62,87 @@ __device__ __forceinline__ int setTotal(const TapeSets& S, int p) {
   return S.capOff[p + 1] > S.capOff[p] ? min(*S.s[p].total, S.s[p].capacity) : 0;
 }
 
-// per-pair contact counts of all sets, set after set
-__global__ void kTapeCount(TapeSets S, int* cnt) {
-  int tot[kParts];
+// A step's contacts go to the tape in three launches over tiles of 256 pairs
+// (a tile holds pairs of one set): the tiles' contact counts, their scan by one
+// workgroup, and the contacts, one per thread. Bound by the chain of loads.
+// Measured for 4352 particles against a count and scan over the pair
+// capacities and one thread per pair: six launches of 41 -> three of 17 us.
+constexpr int kTapeTile = 256;
+struct TapeTiles {
+  int tot[kParts], first[kParts + 1];  // pairs of each set, its first tile
+};
+__device__ __forceinline__ TapeTiles tapeTiles(const TapeSets& S) {
+  TapeTiles t;
+  t.first[0] = 0;
 #pragma unroll
-  for (int p = 0; p < kParts; ++p) tot[p] = setTotal(S, p);
-  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < S.capOff[kParts]; g += gridDim.x * blockDim.x) {
-    int p = 0;
-    while (g >= S.capOff[p + 1]) ++p;
-    const int q = g - S.capOff[p];
-    cnt[g] = q < tot[p] ? S.s[p].recCnt[q] : 0;
+  for (int p = 0; p < kParts; ++p) t.tot[p] = setTotal(S, p);
+#pragma unroll
+  for (int p = 0; p < kParts; ++p) t.first[p + 1] = t.first[p] + (t.tot[p] + kTapeTile - 1) / kTapeTile;
+  return t;
+}
+// a tile's set, the set's pairs and its first tile (constant indices: the
+// arrays stay in registers)
+__device__ __forceinline__ int tileSet(const TapeTiles& t, int tile, int& tot, int& first) {
+  int set = 0;
+  tot = t.tot[0];
+  first = 0;
+#pragma unroll
+  for (int p = 1; p < kParts; ++p)
+    if (tile >= t.first[p]) {
+      set = p;
+      tot = t.tot[p];
+      first = t.first[p];
+    }
+  return set;
+}
+// Exclusive scan over a workgroup of up to 1024 threads (lds: 16 ints).
+__device__ __forceinline__ int groupScan(int v, int* lds, int& total) {
+  int inc = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(inc, off, 64);
+    if (laneId() >= off) inc += u;
+  }
+  if (laneId() == 63) lds[threadIdx.x >> 6] = inc;
+  __syncthreads();
+  int before = 0;
+  total = 0;
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
+    if (w < (int)(threadIdx.x >> 6)) before += lds[w];
+    total += lds[w];
+  }
+  __syncthreads();
+  return before + inc - v;
+}
+
+__global__ void __launch_bounds__(kTapeTile) kTapeCount(TapeSets S, int* sums) {
+  __shared__ int lds[16];
+  const TapeTiles t = tapeTiles(S);
+  for (int tile = blockIdx.x; tile < t.first[kParts]; tile += gridDim.x) {
+    int tot, t0;
+    const int set = tileSet(t, tile, tot, t0), p = (tile - t0) * kTapeTile + threadIdx.x;
+    int total;
+    groupScan(p < tot ? S.s[set].recCnt[p] : 0, lds, total);
+    if (threadIdx.x == 0) sums[tile] = total;
   }
 }
 
-__global__ void kTapeBlock(fdm_contact_tape t, int block, TapeSets S, const int* total, const int* off,
-                           int maxBlock) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const int all = *total;
+__global__ void __launch_bounds__(1024) kTapeBlock(fdm_contact_tape t, int block, TapeSets S, const int* sums, int* off,
+                                                   int* total, int maxBlock) {
+  __shared__ int lds[16];
+  const TapeTiles ti = tapeTiles(S);
+  const int tiles = ti.first[kParts];
+  int all = 0;
+  for (int b = 0; b < tiles; b += 1024) {
+    const int i = b + threadIdx.x;
+    int sum;
+    const int ex = groupScan(i < tiles ? sums[i] : 0, lds, sum);
+    if (i < tiles) off[i] = all + ex;
+    all += sum;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  *total = all;
   int* part = t.blockPart + (size_t)(kParts + 1) * block;
   t.blockStart[block] = block * maxBlock;
   if (all > maxBlock) {
@@ -87,7 +151,8 @@ __global__ void kTapeBlock(fdm_contact_tape t, int block, TapeSets S, const int*
     t.blockCount[block] = 0;
     return;
   }
-  for (int p = 0; p < kParts; ++p) part[p] = S.capOff[p] < S.capOff[kParts] ? off[S.capOff[p]] : all;
+#pragma unroll
+  for (int p = 0; p < kParts; ++p) part[p] = ti.first[p] < tiles ? off[ti.first[p]] : all;
   part[kParts] = all;
   t.blockCount[block] = all;
 }
@@ -98,15 +163,35 @@ __device__ __forceinline__ bool keyLess(const fdm_contact_tape& t, int c, int A,
   return t.node[c] < k;
 }
 
-// the same (A, target, node) in the previous block's part of the same set
+// The same (A, target, node) in the previous block's part of the same set.
+// `rel` is the contact's place in its own part: few contacts come or go in a
+// step, so the search starts there and widens in doubling steps.
 __device__ __forceinline__ int prevOf(const fdm_contact_tape& t, int prevBlock, int set, int A, int T,
-                                      int k) {
+                                      int k, int rel) {
   if (prevBlock < 0) return -1;
   const int ps = t.blockStart[prevBlock];
   const int* part = t.blockPart + (size_t)(kParts + 1) * prevBlock;
-  int lo = ps + part[set];
-  const int end = ps + part[set + 1];
-  int hi = end;
+  const int begin = ps + part[set], end = ps + part[set + 1];
+  if (begin >= end) return -1;
+  const int at = min(begin + rel, end - 1);
+  int lo, hi;
+  if (keyLess(t, at, A, T, k)) {
+    lo = hi = at + 1;
+    for (int step = 1; hi < end && keyLess(t, hi, A, T, k); step *= 2) {
+      lo = hi + 1;
+      hi = min(end, lo + step);
+    }
+  } else {
+    lo = hi = at;
+    for (int step = 1; lo > begin; step *= 2) {
+      lo = max(begin, hi - step);
+      if (keyLess(t, lo, A, T, k)) {
+        ++lo;
+        break;
+      }
+      hi = lo;
+    }
+  }
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
     if (keyLess(t, mid, A, T, k)) lo = mid + 1;
@@ -115,37 +200,45 @@ __device__ __forceinline__ int prevOf(const fdm_contact_tape& t, int prevBlock, 
   return (lo < end && t.A[lo] == A && t.T[lo] == T && t.node[lo] == k) ? lo : -1;
 }
 
-// contacts and their history links (thread per pair)
-__global__ void kTapeScatter(TapeSets S, const int* off, const int* total, fdm_contact_tape t, int block,
-                             int prevBlock) {
+// contacts and their history links (thread per contact)
+__global__ void __launch_bounds__(kTapeTile) kTapeScatter(TapeSets S, const int* off, const int* total,
+                                                          fdm_contact_tape t, int block, int prevBlock) {
+  __shared__ int lds[16], first[kTapeTile + 1], pairA[kTapeTile], pairT[kTapeTile], rec0[kTapeTile];
   if (t.blockCount[block] != *total) return;  // block did not fit
+  const TapeTiles ti = tapeTiles(S);
   const int start = t.blockStart[block];
-  int tot[kParts], pre[kParts + 1];
-  pre[0] = 0;
-#pragma unroll
-  for (int p = 0; p < kParts; ++p) {
-    tot[p] = setTotal(S, p);
-    pre[p + 1] = pre[p] + tot[p];
-  }
-  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < pre[kParts]; g += gridDim.x * blockDim.x) {
-    int set = 0;
-    while (g >= pre[set + 1]) ++set;
+  for (int tile = blockIdx.x; tile < ti.first[kParts]; tile += gridDim.x) {
+    int tot, t0;
+    const int set = tileSet(ti, tile, tot, t0), p = (tile - t0) * kTapeTile + threadIdx.x;
     const fdm_pairs& s = S.s[set];
-    const int p = g - pre[set];
-    const int n = s.recCnt[p];
-    if (n <= 0) continue;
-    const int i0 = off[S.capOff[set] + p], A = s.pairA[p], T = s.pairT[p], r0 = s.recOff[p];
-    for (int r = 0; r < n; ++r) {
-      const fdm_record rec = s.rec[r0 + r];
-      const int c = start + i0 + r, k = rec.node;
-      t.A[c] = A;
-      t.T[c] = T;
-      t.node[c] = k;
-      t.spring[3 * (size_t)c] = rec.x;
-      t.spring[3 * (size_t)c + 1] = rec.y;
-      t.spring[3 * (size_t)c + 2] = rec.z;
-      t.prev[c] = prevOf(t, prevBlock, set, A, T, k);
+    const bool on = p < tot;
+    const int n = on ? max(s.recCnt[p], 0) : 0;
+    pairA[threadIdx.x] = on ? s.pairA[p] : 0;
+    pairT[threadIdx.x] = on ? s.pairT[p] : 0;
+    rec0[threadIdx.x] = on ? s.recOff[p] : 0;
+    int m;
+    first[threadIdx.x] = groupScan(n, lds, m);
+    if (threadIdx.x == 0) first[kTapeTile] = m;
+    const int base = off[tile], rel0 = base - t.blockPart[(size_t)(kParts + 1) * block + set];
+    __syncthreads();
+    for (int c = threadIdx.x; c < m; c += kTapeTile) {
+      int lo = 0, hi = kTapeTile - 1;  // the last pair that begins at or before c
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (first[mid] <= c) lo = mid;
+        else hi = mid - 1;
+      }
+      const fdm_record rec = s.rec[rec0[lo] + c - first[lo]];
+      const int to = start + base + c, A = pairA[lo], T = pairT[lo], k = rec.node;
+      t.A[to] = A;
+      t.T[to] = T;
+      t.node[to] = k;
+      t.spring[3 * (size_t)to] = rec.x;
+      t.spring[3 * (size_t)to + 1] = rec.y;
+      t.spring[3 * (size_t)to + 2] = rec.z;
+      t.prev[to] = prevOf(t, prevBlock, set, A, T, k, rel0 + c);
     }
+    __syncthreads();
   }
 }
 
@@ -422,39 +515,57 @@ __global__ void __launch_bounds__(256) kAdjContacts(fdm_adjoint_step_args a, Adj
   }
 }
 
-__device__ __forceinline__ void addShare(double* acc, const double* s) {
-#pragma unroll
-  for (int j = 0; j < kShare; ++j) acc[j] += s[j];
-}
-
+// A workgroup takes kGatherBodies bodies: first 32 lanes per body add its
+// shares, one component per lane (rows of 17 values, whole lines), then one
+// thread per body does the rest. The sums' order is that of one thread's.
+// Measured for 4352 bodies against a thread per body: 17.3 -> 9.9 us.
+constexpr int kGatherBodies = 16;
 __global__ void __launch_bounds__(256) kAdjGather(fdm_adjoint_step_args a, AdjWork k) {
+  __shared__ double sums[kGatherBodies][kShare];
+  __shared__ int targets[8][kBucket];
   const fdm_contact_tape& tp = a.tape;
   const int start = tp.blockStart[a.block];
   const int n = a.before.n;
   const double dt = a.dt, h = 0.5 * a.dt;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+  const int group = threadIdx.x / 32, lane = threadIdx.x % 32;
+  for (int i0 = blockIdx.x * kGatherBodies; i0 < n; i0 += gridDim.x * kGatherBodies) {
+    __syncthreads();
+    for (int body = group; body < kGatherBodies; body += 8) {
+      const int i = i0 + body;
+      if (i >= n) continue;
+      const int m = min(k.bucketCount[i], kBucket);
+      // as target: ascending contact order, from the bucket
+      const int* bk = k.bucket + (size_t)i * kBucket;
+      for (int u = lane; u < m; u += 32) {
+        const int c = bk[u];
+        int rank = 0;
+        for (int q = 0; q < m; ++q) rank += bk[q] < c ? 1 : 0;
+        targets[group][rank] = c;
+      }
+      int r0[kParts], r1[kParts];
+#pragma unroll
+      for (int set = 0; set < kParts; ++set) {
+        r0[set] = k.run[(size_t)set * 2 * n + 2 * i];
+        r1[set] = k.run[(size_t)set * 2 * n + 2 * i + 1];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      if (lane < kShare) {
+        double s = 0.;
+        for (int set = 0; set < kParts; ++set)
+#pragma unroll 4
+          for (int c = r0[set]; c < r1[set]; ++c) s += k.shareA[(size_t)kShare * c + lane];
+#pragma unroll 4
+        for (int r = 0; r < m; ++r) s += k.shareB[(size_t)kShare * targets[group][r] + lane];
+        sums[body][lane] = s;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+    __syncthreads();
+    const int i = i0 + (int)threadIdx.x;
+    if (threadIdx.x >= kGatherBodies || i >= n) continue;
     double s[kShare];
 #pragma unroll
-    for (int j = 0; j < kShare; ++j) s[j] = 0.;
-    for (int set = 0; set < kParts; ++set) {
-      const int* run = k.run + (size_t)set * 2 * n + 2 * i;
-      for (int c = run[0]; c < run[1]; ++c) addShare(s, k.shareA + (size_t)kShare * c);
-    }
-    {
-      // as target: ascending contact order, selected from the bucket
-      const int m = min(k.bucketCount[i], kBucket);
-      const int* bk = k.bucket + (size_t)i * kBucket;
-      int last = -1;
-      for (int r = 0; r < m; ++r) {
-        int next = INT_MAX;
-        for (int u = 0; u < m; ++u) {
-          const int c = bk[u];
-          if (c > last && c < next) next = c;
-        }
-        last = next;
-        addShare(s, k.shareB + (size_t)kShare * next);
-      }
-    }
+    for (int j = 0; j < kShare; ++j) s[j] = sums[threadIdx.x][j];
     // wall-material shares of the wall contacts, per wall material
     const int* wrun = k.run + (size_t)FDM_SET_WALL * 2 * n + 2 * i;
     for (int c = wrun[0]; c < wrun[1]; ++c) {
@@ -589,13 +700,11 @@ extern "C" int fdm_launchTapeAppend(const fdm_pairs* const* sets, fdm_contact_ta
     return FDM_EINVAL;
   TapeWs w;
   if (wsBytes < tapeBytes(maxBlockContacts, cap, &w, (char*)ws)) return FDM_EINVAL;
-  hipLaunchKernelGGL(kTapeCount, dim3(std::max(1u, std::min(blocksFor(cap, 256), 4096u))), dim3(256), 0,
-                     stream, S, w.cnt);
-  int r = scanInts(w.cnt, w.off, (size_t)std::max(cap, 1ll), false, w.total, w.sub, w.subBytes, stream);
-  if (r != FDM_OK) return r;
-  hipLaunchKernelGGL(kTapeBlock, dim3(1), dim3(64), 0, stream, tape, block, S, (const int*)w.total,
-                     (const int*)w.off, maxBlockContacts);
-  hipLaunchKernelGGL(kTapeScatter, dim3(kStride), dim3(256), 0, stream, S, (const int*)w.off,
+  const unsigned tiles = std::min(blocksFor(cap, kTapeTile) + (unsigned)kParts, (unsigned)kStride);
+  hipLaunchKernelGGL(kTapeCount, dim3(tiles), dim3(kTapeTile), 0, stream, S, w.cnt);
+  hipLaunchKernelGGL(kTapeBlock, dim3(1), dim3(1024), 0, stream, tape, block, S, (const int*)w.cnt, w.off, w.total,
+                     maxBlockContacts);
+  hipLaunchKernelGGL(kTapeScatter, dim3(tiles), dim3(kTapeTile), 0, stream, S, (const int*)w.off,
                      (const int*)w.total, tape, block, prevBlock);
   return launchStatus();
 }
@@ -662,7 +771,7 @@ extern "C" int fdm_launchAdjointStep(const fdm_adjoint_step_args* args, void* ws
   const unsigned pb = std::max(1u, std::min(blocksFor(n, 256), 4096u));
   hipLaunchKernelGGL(kAdjKick, dim3(std::max(pb, 64u)), dim3(256), 0, stream, a, k);
   hipLaunchKernelGGL(kAdjContacts, dim3(kStride), dim3(256), 0, stream, a, k);
-  hipLaunchKernelGGL(kAdjGather, dim3(pb), dim3(256), 0, stream, a, k);
+  hipLaunchKernelGGL(kAdjGather, dim3(std::max(1u, std::min(blocksFor(n, kGatherBodies), 65536u))), dim3(256), 0, stream, a, k);
   return launchStatus();
 }
 
