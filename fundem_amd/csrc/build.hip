@@ -288,6 +288,16 @@ __device__ __forceinline__ bool acceptPair(const fdm_bodies& B, const fdm_geomet
   return e2 + dist * dist <= rr * rr;
 }
 
+// A's grid. (Opaque at each use: what is computed from a launch's one grid, as
+// the periods, would otherwise be kept in registers over the loop of the sets.)
+template <bool MANY>
+__device__ __forceinline__ fdm_grid gridOf(const BuildK& k, int in) {
+  if (MANY) return k.inst.pgrid[in];
+  fdm_grid g = k.pgrid;
+  asm volatile("" : "+s"(g.min.x), "+s"(g.min.y), "+s"(g.min.z), "+s"(g.max.x), "+s"(g.max.y));
+  return g;
+}
+
 // Candidates of particle A in one set, by `lanes` lanes of which this is
 // number `gl`: emit(target, ghost index) for each, in no order.
 template <int SET, bool MANY, class Emit>
@@ -304,7 +314,7 @@ __device__ __forceinline__ void findPairs(const BuildK& k, int s, int A, V3 x, d
     }
     return;
   }
-  const fdm_grid grid = MANY ? k.inst.pgrid[in] : k.pgrid;
+  const fdm_grid grid = gridOf<MANY>(k, in);
   const long long off = MANY ? k.inst.pcellOffset[in] : 0;
   const double reachMax = SET == FDM_SET_PARTICLE ? k.maxRadius : k.maxBoxReach;
   I3 b0, b1;
@@ -359,11 +369,13 @@ __device__ __forceinline__ void findPairs(const BuildK& k, int s, int A, V3 x, d
 template <bool MANY>
 __device__ __forceinline__ V3 detectAt(const BuildK& k, int s, V3 x, int in) {
   if (s < 2) return x;
-  return wrapPosition(x, MANY ? k.inst.pgrid[in] : k.pgrid, MANY ? k.inst.periodic[in] : k.periodic);
+  return wrapPosition(x, gridOf<MANY>(k, in), MANY ? k.inst.periodic[in] : k.periodic);
 }
 
+// (four waves per SIMD instead of three, as the time is the chain of loads:
+// 110592 particles 134 -> 117 us)
 template <bool MANY>
-__global__ void __launch_bounds__(256) kBuildFind(BuildK k) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) kBuildFind(BuildK k) {
   constexpr int G = 64 / kFindLanes;  // particles per wave
   struct Group {
     int n, t[kFindMax], g[kFindMax];
