@@ -506,7 +506,7 @@ struct HitSlots {
 // contact law with one hit per lane and the pair sums folded in node order.
 // A pair with more than kMaxHits contacts recomputes its hits chunk by chunk
 // instead of staging them.
-// CULL: first take the particle-level pre-cull test of sweepPair (sphere,
+// CULL: first take a particle-level test of the pair (sphere,
 // SDF box, Lipschitz bound at this step's positions) and leave empty record
 // ranges when it rejects the pair.
 template <int SET, bool CULL = false>
@@ -1771,7 +1771,7 @@ extern "C" int fdm_launchNarrowPhaseSets(const fdm_narrowphase_args* sets, int n
   const NarrowScratch x = {ws->hitGeom, ws->hitCapacity, ws->hitCount};
   fdm_tuning tu = tuning();
   if (ws->tuning && !completeTuning(*ws->tuning, tu)) return FDM_EINVAL;
-  // geometry without the culling tables of sweepPair: the kernel that culls
+  // geometry without the culling tables of sweepRun: the kernel that culls
   // by chunk
   const fdm_geometry& pg = sets[0].pgeo;
   if (!pg.groups || !pg.groupNodes || !pg.cells || (sets[0].wgeo.num > 0 && !sets[0].wgeo.cells)) tu.lawMode = 2;

@@ -40,55 +40,127 @@ __device__ __forceinline__ int nextMirror(const int* list, int m, int last) {
   return best;
 }
 
-__device__ __forceinline__ int segBegin(const fdm_pairs& s, int i) {
-  return min(s.count[i], s.capacity);
-}
-__device__ __forceinline__ int segEnd(const fdm_pairs& s, int i) {
-  return min(s.count[i + 1], s.capacity);
-}
-
 // The kernel's view of the launcher's arguments (reduce.hip).
 int fillReduce(const fdm_reduce_args& g, ReduceK& k);
 
+// Sums of up to two records, loaded together; rows of three are added in turn.
+struct TwoRecs {
+  double f[2][3], t[2][3];
+};
+__device__ __forceinline__ void loadRec(TwoRecs& r, int k, const double* f, const double* t) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    r.f[k][c] = f[c];
+    r.t[k][c] = t[c];
+  }
+}
+// Owned pairs [b, e) of a set.
+__device__ __forceinline__ void addOwned(V3& F, V3& T, const fdm_pairs& s, int b, int e) {
+  for (int p = b; p < e; p += 2) {
+    const int q = p + 1, n0 = s.recCnt[p];
+    int n1 = 0;
+    TwoRecs r;
+    loadRec(r, 0, s.sumF + 3 * (size_t)p, s.sumTA + 3 * (size_t)p);
+    if (q < e) {
+      n1 = s.recCnt[q];
+      loadRec(r, 1, s.sumF + 3 * (size_t)q, s.sumTA + 3 * (size_t)q);
+    }
+    if (n0 > 0) addRec(F, T, r.f[0], r.t[0], false);
+    if (n1 > 0) addRec(F, T, r.f[1], r.t[1], false);
+  }
+}
+
 // Force and torque of particle i: its records in the canonical order (the
 // header of reduce.hip). Bodies without candidate pairs or bonds are told by
-// one word (touch) instead of the counts of every set.
+// one word (touch) instead of the counts of every set. For the others this is
+// a chain of dependent loads, so they are taken in rounds: the counts of all
+// sets; a short mirror list as a whole; records by two, also of pairs without
+// contacts, whose sums are then not added. Measured
+// in kReduceStep: 216 particles 16.3 -> 14.4 us, 8192 spheres of up to twelve
+// bonds 25.5 -> 20.0 us; one particle 10.3 -> 10.6 us.
 __device__ __forceinline__ void foldForces(const ReduceK& a, int i, V3& F, V3& T) {
   F = {0., 0., 0.};
   T = {0., 0., 0.};
   const int touch = a.touch ? a.touch[i] : ~0;
   if (!touch) return;
-  // particle pairs: as target (partners below i), then owned (partners above)
+  int m = 0, p0 = 0, p1 = 0, w0 = 0, w1 = 0, b0 = 0, b1 = 0;
+  int gm[3] = {0, 0, 0}, g0[3] = {0, 0, 0}, g1[3] = {0, 0, 0};
   if (touch & (FDM_TOUCH_A(0) | FDM_TOUCH_T(0))) {
-    const int m = min(a.ppm.count[i], a.ppm.capacity);
-    const int* list = a.ppm.list + (size_t)i * a.ppm.capacity;
-    int last = -1;
-    for (int r = 0; r < m; ++r) {
-      const int p = nextMirror(list, m, last);
-      last = p;
-      addRec(F, T, a.pp.sumF + 3 * (size_t)p, a.pp.sumTB + 3 * (size_t)p, true);
-    }
-    if (m > 0) a.ppm.count[i] = 0;
-    for (int p = segBegin(a.pp, i); p < segEnd(a.pp, i); ++p)
-      if (a.pp.recCnt[p] > 0) addRec(F, T, a.pp.sumF + 3 * (size_t)p, a.pp.sumTA + 3 * (size_t)p, false);
+    m = a.ppm.count[i];
+    p0 = a.pp.count[i];
+    p1 = a.pp.count[i + 1];
   }
-  if (a.havePW && (touch & FDM_TOUCH_A(1)))
-    for (int p = segBegin(a.pw, i); p < segEnd(a.pw, i); ++p)
-      if (a.pw.recCnt[p] > 0) addRec(F, T, a.pw.sumF + 3 * (size_t)p, a.pw.sumTA + 3 * (size_t)p, false);
+  if (a.havePW && (touch & FDM_TOUCH_A(1))) {
+    w0 = a.pw.count[i];
+    w1 = a.pw.count[i + 1];
+  }
+#pragma unroll
+  for (int s = 0; s < 3; ++s)
+    if (a.haveG[s] && (touch & (FDM_TOUCH_A(2 + s) | FDM_TOUCH_T(2 + s)))) {
+      gm[s] = a.gm[s].count[i];
+      g0[s] = a.g[s].count[i];
+      g1[s] = a.g[s].count[i + 1];
+    }
+  if (a.haveBonds && (touch & FDM_TOUCH_BOND)) {
+    b0 = a.bonds.partStart[i];
+    b1 = a.bonds.partStart[i + 1];
+  }
+  // particle pairs: as target (partners below i), then owned (partners above)
+  if (m > 0) {
+    a.ppm.count[i] = 0;
+    m = min(m, a.ppm.capacity);
+    const int* list = a.ppm.list + (size_t)i * a.ppm.capacity;
+    if (m <= 4) {
+      int l[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) l[r] = r < m ? list[r] : INT_MAX;
+      auto order = [](int& x, int& y) __attribute__((always_inline)) {
+        const int lo = min(x, y);
+        y = max(x, y);
+        x = lo;
+      };
+      order(l[0], l[1]);
+      order(l[2], l[3]);
+      order(l[0], l[2]);
+      order(l[1], l[3]);
+      order(l[1], l[2]);
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        if (r >= m) break;
+        const bool two = r + 1 < m;
+        const int p = l[r], q = two ? l[r + 1] : p;
+        TwoRecs x;
+        loadRec(x, 0, a.pp.sumF + 3 * (size_t)p, a.pp.sumTB + 3 * (size_t)p);
+        loadRec(x, 1, a.pp.sumF + 3 * (size_t)q, a.pp.sumTB + 3 * (size_t)q);
+        addRec(F, T, x.f[0], x.t[0], true);
+        if (two) addRec(F, T, x.f[1], x.t[1], true);
+      }
+    } else {
+      int last = -1;
+      for (int r = 0; r < m; ++r) {
+        const int p = nextMirror(list, m, last);
+        last = p;
+        addRec(F, T, a.pp.sumF + 3 * (size_t)p, a.pp.sumTB + 3 * (size_t)p, true);
+      }
+    }
+  }
+  addOwned(F, T, a.pp, min(p0, a.pp.capacity), min(p1, a.pp.capacity));
+  if (a.havePW) addOwned(F, T, a.pw, min(w0, a.pw.capacity), min(w1, a.pw.capacity));
+#pragma unroll
   for (int s = 0; s < 3; ++s) {
-    if (!a.haveG[s] || !(touch & (FDM_TOUCH_A(2 + s) | FDM_TOUCH_T(2 + s)))) continue;
     const fdm_pairs& G = a.g[s];
     const fdm_mirror& M = a.gm[s];
-    const int m = min(M.count[i], M.capacity);
+    const int mm = min(gm[s], M.capacity);
+    int own = min(g0[s], G.capacity);
+    const int ownEnd = min(g1[s], G.capacity);
+    if (mm <= 0 && own >= ownEnd) continue;
     const int* list = M.list + (size_t)i * M.capacity;
-    int own = segBegin(G, i);
-    const int ownEnd = segEnd(G, i);
-    int mp = m > 0 ? nextMirror(list, m, -1) : INT_MAX;
+    int mp = mm > 0 ? nextMirror(list, mm, -1) : INT_MAX;
     int used = 0;
     while (true) {
       while (own < ownEnd && G.recCnt[own] == 0) ++own;
       const bool haveOwn = own < ownEnd;
-      const bool haveMir = used < m;
+      const bool haveMir = used < mm;
       if (!haveOwn && !haveMir) break;
       const int partnerOwn = haveOwn ? G.pairT[own] : INT_MAX;
       const int partnerMir = haveMir ? G.pairA[mp] : INT_MAX;
@@ -98,19 +170,26 @@ __device__ __forceinline__ void foldForces(const ReduceK& a, int i, V3& F, V3& T
       } else {
         addRec(F, T, G.sumF + 3 * (size_t)mp, G.sumTB + 3 * (size_t)mp, true);
         ++used;
-        mp = used < m ? nextMirror(list, m, mp) : INT_MAX;
+        mp = used < mm ? nextMirror(list, mm, mp) : INT_MAX;
       }
     }
-    if (m > 0) M.count[i] = 0;
+    if (mm > 0) M.count[i] = 0;
   }
-  if (a.haveBonds && (touch & FDM_TOUCH_BOND)) {
+  if (b0 < b1) {
     const fdm_bonds& b = a.bonds;
-    for (int e = b.partStart[i]; e < b.partStart[i + 1]; ++e) {
-      const int code = b.partList[e];
-      const int k = code >> 1;
-      if (!b.applied[k]) continue;
-      if ((code & 1) == 0) addRec(F, T, b.outF + 3 * (size_t)k, b.outTi + 3 * (size_t)k, false);
-      else addRec(F, T, b.outF + 3 * (size_t)k, b.outTj + 3 * (size_t)k, true);
+    int n0 = b.partList[b0], n1 = b.partList[min(b0 + 1, b1 - 1)];
+    for (int e = b0; e < b1; e += 2) {
+      const bool two = e + 1 < b1;
+      const int c0 = n0, c1 = n1;
+      n0 = b.partList[min(e + 2, b1 - 1)];  // (the next bonds, a round ahead)
+      n1 = b.partList[min(e + 3, b1 - 1)];
+      const int k0 = c0 >> 1, k1 = c1 >> 1;
+      const int on0 = b.applied[k0], on1 = b.applied[k1];
+      TwoRecs x;
+      loadRec(x, 0, b.outF + 3 * (size_t)k0, ((c0 & 1) ? b.outTj : b.outTi) + 3 * (size_t)k0);
+      loadRec(x, 1, b.outF + 3 * (size_t)k1, ((c1 & 1) ? b.outTj : b.outTi) + 3 * (size_t)k1);
+      if (on0) addRec(F, T, x.f[0], x.t[0], c0 & 1);
+      if (two && on1) addRec(F, T, x.f[1], x.t[1], c1 & 1);
     }
   }
 }
@@ -168,10 +247,7 @@ struct StepBeginK {
   int* blockFlags;   // [gridDim.x] bit 0 grid state changed, 1 visibility changed, 2 wrapped
 };
 
-// Phase A of a step (one thread per particle, then per wall). Each workgroup
-// leaves its largest motion rate and its change flags in a slot of its own
-// (no atomics on shared words); kStepDecide folds the slots.
-// One body of phase A. Everything it reads from the launch arguments is
+// One body of phase A of a step (particles, then walls). Everything it reads from the launch arguments is
 // copied into registers first (selecting between argument structs by
 // reference would make the compiler copy them to per-lane scratch).
 // MANY: bodies of several systems (per-body grids and periodic flags); the
