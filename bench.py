@@ -100,13 +100,12 @@ def log(*a):
 #                only; a body whose template's inverse inertia is exactly
 #                zero (its spin never changes) skips T read and w write
 #                (168 - 24 = 144)
-#   reduce_kick  per particle: pair counts read (particle set 8, wall 8,
-#                three ghost sets 24, mirror counts 16), F T write 24,
-#                template id 4, v w read and write 48, q read 16 (= 148;
-#                148 - 40 = 108 for a body whose spin never changes: no w,
+#   reduce_kick  per particle: the word that tells its sets 4, F T write 24,
+#                template id 4, v w read and write 48, q read 16 (= 96;
+#                96 - 40 = 56 for a body whose spin never changes: no w,
 #                no q); per candidate pair with contacts, read from each
 #                side: its record count 4 and sums 48 (bounded by 104 per
-#                pair: every candidate pair counted)
+#                pair: every candidate pair counted; pair counts not counted)
 #   narrow       per candidate pair: ids 8, both bodies' x q template id 88,
 #                empty record range or the kept pair's record range and pair
 #                sums 80, history ids 16 (= 192); per contact: velocities of
@@ -116,7 +115,7 @@ def kernel_bytes(stage, n, pairs, contacts, fixed=0):
     if stage == "step_begin":
         return 168.0 * n - 24.0 * fixed
     if stage == "reduce_kick":
-        return 148.0 * n - 40.0 * fixed + 104.0 * sum(pairs.values())
+        return 96.0 * n - 40.0 * fixed + 104.0 * sum(pairs.values())
     if stage == "narrow":
         return 192.0 * sum(pairs.values()) + 80.0 * sum(contacts.values())
     return None
