@@ -228,6 +228,11 @@ __global__ __launch_bounds__(kMeshTile) void kMeshDistance(const double* __restr
 // ms, 2.4M and 5120 87 -> 3.5 ms (4.5 with the triangles shuffled), 578K and
 // 20480 82 -> 3.6 ms.
 constexpr int kMeshChunk = 32;
+// Sizes between which the signs are taken from crossings: a solid angle's
+// products of three lengths neither overflow nor vanish. A mesh beyond them, or
+// with a coordinate that is no number, has an infinite "largest coordinate",
+// under which no node counts as decided.
+constexpr double kMeshLeast = 1e-20, kMeshMost = 1e90;
 struct alignas(64) MeshChunk {
   double lo[3], hi[3];       // box of the triangles
   double m;                  // largest |coordinate|
@@ -282,6 +287,9 @@ __global__ void __launch_bounds__(256) kMeshPrep(MeshWork k) {
     for (int q = 0; q < 9; ++q) v[q] = k.tri[9 * (size_t)t + q];
     double box[7];
     box[6] = 0.;
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+      if (!(fabs(v[q]) <= kMeshMost)) box[6] = __builtin_inf();
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       box[a] = fmin(fmin(v[a], v[3 + a]), v[6 + a]);
@@ -402,8 +410,10 @@ __global__ void __launch_bounds__(256) kMeshWinding(MeshWork k) {
   }
   __syncthreads();
   e = edges[0] + edges[1] + edges[2] + edges[3];
-  if (blockIdx.x == 0 && threadIdx.x == 0)
-    *k.largest = fmax(fmax(largest[0], largest[1]), fmax(largest[2], largest[3]));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    big = fmax(fmax(largest[0], largest[1]), fmax(largest[2], largest[3]));
+    *k.largest = big >= kMeshLeast && big <= kMeshMost ? big : __builtin_inf();
+  }
   const long long nxy = (long long)k.m.nx * k.m.ny, col = (long long)blockIdx.x * 256 + threadIdx.x;
   if (col >= nxy) return;
   const bool open = e != 0ull || k.column[col] != 0;

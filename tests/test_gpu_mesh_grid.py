@@ -85,3 +85,25 @@ def test_either_side_of_the_rule(subdivisions, h):
     o2, s2, v2 = po.mesh_grid(v, f, h, 2)
     print(f"{len(f)} triangles x {vals.size} nodes = {len(f) * vals.size / 2**22:.2f} x 2^22", flush=True)
     assert np.array_equal(origin, o2) and size == s2 and np.array_equal(vals, v2)
+
+
+@pytest.mark.parametrize("what", ["no number", "huge", "tiny", "plain"])
+def test_unusual_coordinates_equal_the_point_kernel(what):
+    """Coordinates that are no numbers or whose products leave the range of a
+    double: the grid equals the point queries, which take every triangle's
+    solid angle, at the same nodes."""
+    v, f = torus()
+    v = v.copy()
+    if what == "no number":
+        v[7] = np.nan
+    v = v * {"huge": 1e110, "tiny": 1e-32}.get(what, 1.0)
+    h = float(np.nanmax(np.abs(torus()[0]))) * {"huge": 1e110, "tiny": 1e-32}.get(what, 1.0) / 8
+    m = G.MeshParticle(v, f)
+    origin, h, size, vals = m.build_grid(h)
+    assert len(f) * vals.size >= 1 << 22
+    k, j, i = np.meshgrid(*(np.arange(n) for n in size[::-1]), indexing="ij")
+    val, grad = m.evaluate(origin + h * np.stack([i, j, k], -1).reshape(-1, 3))
+    with np.errstate(all="ignore"):
+        gn = np.sqrt(grad[:, 0] ** 2 + grad[:, 1] ** 2 + grad[:, 2] ** 2)
+        want = np.where(gn > 1e-12, val / gn, np.where(val <= 0.0, -0.5 * h, 0.5 * h))
+    assert np.array_equal(vals, want, equal_nan=True)
