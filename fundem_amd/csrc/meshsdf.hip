@@ -214,20 +214,26 @@ __global__ __launch_bounds__(kMeshTile) void kMeshDistance(const double* __restr
 //    sideways by a 1e-4 of the spacing, as meshes like to have vertices and
 //    edges on grid lines.
 //  - Nodes that this does not decide for certain take the solid angles, eight
-//    partial sums as above, by a workgroup each (kMeshSolid): nodes nearer to the
-//    surface than the ray's shift and rounding, columns whose ray passes an
-//    edge within rounding, and all nodes of an open mesh.
+//    partial sums as above (kMeshSolid): nodes nearer to the surface than the
+//    ray's shift and rounding, columns whose ray passes an edge within
+//    rounding, and all nodes of an open mesh.
 //  - Distance: bricks of 4 x 4 x 4 nodes, one node per lane, whose waves
 //    share the triangles in chunks of 32; a chunk or triangle whose box is
 //    farther than the best distance found is passed by, the chunk nearest to
 //    the brick first (kMeshNearest). The chunks take the triangles in their
 //    order: a mesh in no spatial order is slower, not wrong.
 // Bound by FP64 VALU, and on small grids by the brick with the most triangles
-// in reach. Measured, a whole call of the host class: 57K nodes and 5120
+// in reach. An open mesh pays for every solid angle; on grids of few bricks it
+// finds the nearest triangle in the same loop, as the longest brick cannot hide
+// there (20479 triangles, 15925 nodes: 3.0 ms, 3.7 with kMeshNearest, 2.9-3.3
+// as kMeshDistance; 2601 nodes, 5119 triangles 0.24 ms against 0.42 and 0.62).
+// Measured, a whole call of the host class: 57K nodes and 5120
 // triangles 2.60 -> 0.43 ms (kernels 2.52 -> 0.33), 342K and 5120 13.1 -> 1.05
 // ms, 2.4M and 5120 87 -> 3.5 ms (4.5 with the triangles shuffled), 578K and
 // 20480 82 -> 3.6 ms.
 constexpr int kMeshChunk = 32;
+constexpr int kSolidStep = 4;  // kMeshSolid: triangles per thread between barriers
+constexpr int kSolidMany = 2048;
 // Sizes between which the signs are taken from crossings: a solid angle's
 // products of three lengths neither overflow nor vanish. A mesh beyond them, or
 // with a coordinate that is no number, has an infinite "largest coordinate",
@@ -249,6 +255,7 @@ struct MeshWork {
   int* list;            // nodes not decided
   int* listCount;
   double* largest;      // largest |coordinate| of triangles and grid
+  int* open;            // the mesh is not closed
   double* sdf;
 };
 __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
@@ -321,6 +328,15 @@ __global__ void __launch_bounds__(256) kMeshPrep(MeshWork k) {
   }
 }
 
+// Sum of the chunks' edge sums by a wave: zero for a closed mesh.
+__device__ __forceinline__ unsigned long long edgeSum(const MeshWork& k, int lane) {
+  unsigned long long e = 0ull;
+  for (int c = lane; c < k.nChunks; c += 64) e += k.chunks[c].edges;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+  return e;
+}
+
 // Triangles crossed by the columns' rays: a wave takes 8 x 8 columns, one per
 // lane, and a share of the chunks. A crossing is left at the column's highest
 // node below it. A triangle counts if the ray passes its three edges on one
@@ -333,7 +349,7 @@ __global__ void __launch_bounds__(256) kMeshColumns(MeshWork k, int tilesX, int 
   const int lane = laneId();
   const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   const int tile = wave % tiles, c0 = wave / tiles * perWave, c1 = min(c0 + perWave, k.nChunks);
-  if (c0 >= c1) return;
+  if (c0 >= c1 || edgeSum(k, lane) != 0ull) return;  // (an open mesh takes no crossing)
   const MeshPoints& m = k.m;
   const int i0 = tile % tilesX * 8, j0 = tile / tilesX * 8;
   const int i = i0 + lane % 8, j = j0 + lane / 8;
@@ -413,6 +429,7 @@ __global__ void __launch_bounds__(256) kMeshWinding(MeshWork k) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     big = fmax(fmax(largest[0], largest[1]), fmax(largest[2], largest[3]));
     *k.largest = big >= kMeshLeast && big <= kMeshMost ? big : __builtin_inf();
+    *k.open = e != 0ull ? 1 : 0;
   }
   const long long nxy = (long long)k.m.nx * k.m.ny, col = (long long)blockIdx.x * 256 + threadIdx.x;
   if (col >= nxy) return;
@@ -439,7 +456,7 @@ __device__ __forceinline__ double boxDistance2(V3 p, const double* lo, const dou
 }
 
 template <int WAVES>
-__global__ void __launch_bounds__(64 * WAVES) kMeshNearest(MeshWork k, int bricksX, int bricksY) {
+__global__ void __launch_bounds__(64 * WAVES) kMeshNearest(MeshWork k, int bricksX, int bricksY, int solo) {
   __shared__ unsigned long long bound[64];  // best squared distance of the node so far
   __shared__ double sBest[WAVES][64], sCp[3][WAVES][64];
   __shared__ int sIdx[WAVES][64];
@@ -452,6 +469,7 @@ __global__ void __launch_bounds__(64 * WAVES) kMeshNearest(MeshWork k, int brick
   const int i = i0 + lane % 4, j = j0 + lane / 4 % 4, kk = k0 + lane / 16;
   const bool on = i < m.nx && j < m.ny && kk < m.nz;
   const V3 p = {m.ox + double(i) * m.h, m.oy + double(j) * m.h, m.oz + double(kk) * m.h};
+  if (solo && *k.open) return;
   const double largest = *k.largest;
   // the brick's ball (nodes past the grid's end included)
   const V3 mid = {m.ox + (i0 + 1.5) * m.h, m.oy + (j0 + 1.5) * m.h, m.oz + (k0 + 1.5) * m.h};
@@ -577,32 +595,110 @@ __global__ void __launch_bounds__(64 * WAVES) kMeshNearest(MeshWork k, int brick
   if (!sure && d != 0.0) k.list[atomicAdd(k.listCount, 1)] = (int)id;
 }
 
-// The solid angles of the nodes left, a workgroup each: 256 triangles at a
-// time, added to eight partial sums in the order of kMeshDistance.
-__global__ void __launch_bounds__(kMeshTile) kMeshSolid(MeshWork k) {
-  __shared__ double angle[2][kMeshTile];
-  const int count = *k.listCount;
-  for (int n = blockIdx.x; n < count; n += gridDim.x) {
-    const int id = k.list[n];
-    const V3 p = pointOf(k.m, id);
-    double sum = 0.0;
-    int buf = 0;
-    for (int t0 = 0; t0 < k.nt; t0 += kMeshTile, buf ^= 1) {
-      const int t = t0 + (int)threadIdx.x;
+// The solid angles of NODES nodes by a workgroup: a thread takes every
+// 256 / NODES-th triangle for one node, and 8 * NODES lanes add the angles,
+// staged in LDS, to eight partial sums per node in the order of kMeshDistance.
+// Nodes first, first + 1, ... of the list, whose sign is left; DISTANCE: of
+// the grid, with the nearest triangle found in the same loop.
+struct SolidSlots {
+  double angle[2][kSolidStep * kMeshTile];
+  unsigned long long bound[8];  // best squared distance of a node so far
+};
+template <int NODES, bool DISTANCE>
+__device__ __forceinline__ void solidNodes(const MeshWork& k, int first, int count, SolidSlots& ws) {
+  constexpr int kEach = NODES == 1 ? 1 : kSolidStep;  // triangles per thread between barriers
+  constexpr int kTile = kMeshTile / NODES * kEach;
+  const int node = threadIdx.x % NODES;
+  const int at = min(first + node, count - 1), id = DISTANCE ? at : k.list[at];
+  const V3 p = pointOf(k.m, id);
+  double sum = 0.0, best = DBL_MAX;
+  int buf = 0, bestIdx = INT_MAX;
+  if (DISTANCE) {
+    if ((int)threadIdx.x < NODES) ws.bound[threadIdx.x] = (unsigned long long)__double_as_longlong(DBL_MAX);
+    __syncthreads();
+  }
+  for (int t0 = 0; t0 < k.nt; t0 += kTile, buf ^= 1) {
+    double limit = DBL_MAX;
+    if (DISTANCE) limit = __longlong_as_double((long long)*(volatile unsigned long long*)&ws.bound[node]);
+#pragma unroll 1
+    for (int u = 0; u < kEach; ++u) {
+      const int t = t0 + (u * kMeshTile + (int)threadIdx.x) / NODES;
+      double angle = 0.0;
       if (t < k.nt) {
         const double* v = k.tri + 9 * (size_t)t;
-        angle[buf][threadIdx.x] = solidAngle(p, {v[0], v[1], v[2]}, {v[3], v[4], v[5]}, {v[6], v[7], v[8]});
+        const V3 a = {v[0], v[1], v[2]}, b = {v[3], v[4], v[5]}, c = {v[6], v[7], v[8]};
+        angle = solidAngle(p, a, b, c);
+        if (DISTANCE) {
+          const double lo[3] = {fmin(fmin(a.x, b.x), c.x), fmin(fmin(a.y, b.y), c.y), fmin(fmin(a.z, b.z), c.z)};
+          const double hi[3] = {fmax(fmax(a.x, b.x), c.x), fmax(fmax(a.y, b.y), c.y), fmax(fmax(a.z, b.z), c.z)};
+          if (boxDistance2(p, lo, hi) <= limit * (1.0 + 1e-9)) {
+            const double d2 = vlen2(vsub(p, closestOnTriangle(p, a, b, c)));
+            if (d2 < best) {  // a thread's triangles come in increasing index
+              best = d2;
+              bestIdx = t;
+              limit = fmin(limit, d2);
+            }
+          }
+        }
       }
-      __syncthreads();
-      if (threadIdx.x < kSlices)
-        for (int q = threadIdx.x; q < min(kMeshTile, k.nt - t0); q += kSlices) sum += angle[buf][q];
+      ws.angle[buf][u * kMeshTile + threadIdx.x] = angle;
     }
-    if (threadIdx.x < 64) {
-      double all = readlaneD(sum, 0);
-      for (int s = 1; s < kSlices; ++s) all += readlaneD(sum, s);
-      if (threadIdx.x == 0 && fabs(all / (4.0 * kPi)) > 0.5) k.sdf[id] = -k.sdf[id];
+    // (non-negative numbers order as their bits do)
+    if (DISTANCE) atomicMin(&ws.bound[node], (unsigned long long)__double_as_longlong(limit));
+    __syncthreads();
+    if (threadIdx.x < kSlices * NODES)
+#pragma unroll
+      for (int q = 0; q < kTile / kSlices; ++q) sum += ws.angle[buf][q * kSlices * NODES + threadIdx.x];
+  }
+  double all = 0.0;
+  if (threadIdx.x < 64) {
+    all = __shfl(sum, node);
+    for (int s = 1; s < kSlices; ++s) all += __shfl(sum, s * NODES + node);
+  }
+  const bool inside = fabs(all / (4.0 * kPi)) > 0.5;
+  __syncthreads();
+  if (DISTANCE) {
+    double *d2 = ws.angle[0], *idx = d2 + kMeshTile;
+    const int j = threadIdx.x;
+    d2[j] = best;
+    idx[j] = (double)bestIdx;
+    __syncthreads();
+    if (j < NODES && first + j < count) {
+      for (int q = j + NODES; q < kMeshTile; q += NODES)
+        if (d2[q] < best || (d2[q] == best && idx[q] < (double)bestIdx)) {
+          best = d2[q];
+          bestIdx = (int)idx[q];
+        }
+      V3 cp = {0.0, 0.0, 0.0};
+      if (bestIdx < k.nt) {
+        const double* v = k.tri + 9 * (size_t)bestIdx;
+        cp = closestOnTriangle(p, {v[0], v[1], v[2]}, {v[3], v[4], v[5]}, {v[6], v[7], v[8]});
+      }
+      k.sdf[id] = gridValue(vsub(p, cp), vlen(vsub(p, cp)), inside, k.positiveInside, k.m.h);
     }
     __syncthreads();
+  } else if ((int)threadIdx.x < NODES && first + (int)threadIdx.x < count && inside) {
+    k.sdf[id] = -k.sdf[id];
+  }
+}
+
+// The nodes left. A workgroup for each where they are few, as the chain of
+// tiles is then the time; eight a workgroup from kSolidMany on, where one
+// node's sums, added by eight lanes, held up the other threads (57475 nodes,
+// 5119 triangles 3.40 -> 2.18 ms). solo: the grid of an open mesh, which
+// kMeshNearest left out. Bound by FP64 VALU (some 300 instructions an angle).
+__global__ void __launch_bounds__(kMeshTile) __attribute__((amdgpu_waves_per_eu(4))) kMeshSolid(MeshWork k, int solo) {
+  __shared__ SolidSlots ws;
+  if (solo && *k.open) {
+    const int count = (int)k.m.count;
+    for (int n = 8 * blockIdx.x; n < count; n += 8 * gridDim.x) solidNodes<8, true>(k, n, count, ws);
+    return;
+  }
+  const int count = *k.listCount;
+  if (count < kSolidMany) {
+    for (int n = blockIdx.x; n < count; n += gridDim.x) solidNodes<1, false>(k, n, count, ws);
+  } else {
+    for (int n = 8 * blockIdx.x; n < count; n += 8 * gridDim.x) solidNodes<8, false>(k, n, count, ws);
   }
 }
 
@@ -658,7 +754,7 @@ extern "C" size_t fdm_meshGridWorkspaceBytes(int numTriangles, const int* size) 
   const size_t nodes = (size_t)size[0] * size[1] * size[2], cols = (size_t)size[0] * size[1];
   return alignUp(nodes * sizeof(int)) * 2 + alignUp(cols * sizeof(int)) +
          alignUp(((size_t)numTriangles + kMeshChunk - 1) / kMeshChunk * sizeof(MeshChunk)) +
-         alignUp(sizeof(int)) + alignUp(sizeof(double));
+         2 * alignUp(sizeof(int)) + alignUp(sizeof(double));
 }
 
 extern "C" int fdm_launchMeshSignedDistanceGridWith(const double* triangles, int numTriangles, const double* origin,
@@ -685,6 +781,7 @@ extern "C" int fdm_launchMeshSignedDistanceGridWith(const double* triangles, int
   k.chunks = cv.take<MeshChunk>((size_t)k.nChunks);
   k.listCount = cv.take<int>(1);
   k.largest = cv.take<double>(1);
+  k.open = cv.take<int>(1);
   if (!cv.ok) return FDM_EINVAL;
   const long long work = std::max<long long>(k.m.count, (long long)k.nChunks * kMeshChunk);
   hipLaunchKernelGGL(kMeshPrep, dim3((unsigned)std::min<long long>(blocksFor(work, 256), 4096)), dim3(256), 0, stream, k);
@@ -701,9 +798,10 @@ extern "C" int fdm_launchMeshSignedDistanceGridWith(const double* triangles, int
   // bricks to fill the chip with four each: its time is then the longest
   // brick's
   const unsigned bricks = (unsigned)((long long)bx * by * ((size[2] + 3) / 4));
-  if (bricks < kMeshFewBricks) hipLaunchKernelGGL(kMeshNearest<16>, dim3(bricks), dim3(1024), 0, stream, k, bx, by);
-  else hipLaunchKernelGGL(kMeshNearest<4>, dim3(bricks), dim3(256), 0, stream, k, bx, by);
-  hipLaunchKernelGGL(kMeshSolid, dim3(persistentBlocks(4)), dim3(kMeshTile), 0, stream, k);
+  const int few = bricks < kMeshFewBricks ? 1 : 0;
+  if (few) hipLaunchKernelGGL(kMeshNearest<16>, dim3(bricks), dim3(1024), 0, stream, k, bx, by, few);
+  else hipLaunchKernelGGL(kMeshNearest<4>, dim3(bricks), dim3(256), 0, stream, k, bx, by, few);
+  hipLaunchKernelGGL(kMeshSolid, dim3(persistentBlocks(4)), dim3(kMeshTile), 0, stream, k, few);
   return launchStatus();
 }
 

@@ -107,3 +107,60 @@ def test_unusual_coordinates_equal_the_point_kernel(what):
         gn = np.sqrt(grad[:, 0] ** 2 + grad[:, 1] ** 2 + grad[:, 2] ** 2)
         want = np.where(gn > 1e-12, val / gn, np.where(val <= 0.0, -0.5 * h, 0.5 * h))
     assert np.array_equal(vals, want, equal_nan=True)
+
+
+@pytest.mark.parametrize("name,h", [("solo", 0.08), ("solo remainder", 0.05), ("many bricks", 0.035)])
+def test_open_mesh_on_either_side_of_the_brick_rule(name, h):
+    """Every node of an open mesh takes the solid angles: with the nearest
+    triangle in one loop on grids of few bricks, after kMeshNearest on more
+    than 4096; numbers of nodes and triangles that are no multiple of eight."""
+    v, f = G.icosphere(1.0, 1 if name == "many bricks" else 3)
+    f = f[:-1]
+    m = G.MeshParticle(v * (1.0, 1.1, 1.2), f)
+    origin, hh, size, vals = m.build_grid(h)
+    bricks = int(np.prod([(n + 3) // 4 for n in size]))
+    print(f"{len(f)} triangles, {vals.size} nodes, {bricks} bricks", flush=True)
+    assert len(f) * vals.size >= 1 << 22 and (bricks >= 4096) == (name == "many bricks")
+    assert vals.size % 8 != 0 or name != "solo remainder"
+    o2, s2, v2 = po.mesh_grid(v * (1.0, 1.1, 1.2), f, h, 2)
+    assert np.array_equal(origin, o2) and size == s2 and np.array_equal(vals, v2)
+
+
+@pytest.mark.parametrize("nu,nv,res", [(40, 20, 30), (80, 32, 50), (160, 64, 30)])
+def test_open_mesh_is_not_slower_than_every_triangle_at_every_node(nu, nv, res):
+    """The grid path of an open mesh against the kernel that takes solid angle
+    and distance of every triangle at every node (the shortest of ten launches
+    each; a fifth is left for the spread between runs, less than half of what
+    the path was slower when each node had a workgroup of its own)."""
+    import ctypes as C
+    import torch
+    from fundem_amd import build
+    lib = C.CDLL(build.CORE_LIB)
+    lib.fdm_meshGridWorkspaceBytes.restype = C.c_size_t
+    v, f = G.torus_mesh(1.0, 0.35, nu, nv)
+    f = f[:-1]
+    origin, h, size, vals = G.MeshParticle(v, f).build_grid_by_resolution(res)
+    tri = torch.tensor(v[f].reshape(-1), dtype=torch.float64, device="cuda")
+    out = torch.zeros(vals.size, dtype=torch.float64, device="cuda")
+    n3, o3 = (C.c_int * 3)(*size), (C.c_double * 3)(*origin)
+    need = lib.fdm_meshGridWorkspaceBytes(C.c_int(len(f)), n3)
+    work = torch.zeros(int(need), dtype=torch.uint8, device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    common = (C.c_void_p(tri.data_ptr()), C.c_int(len(f)), o3, C.c_double(h), n3, C.c_int(0), C.c_void_p(out.data_ptr()))
+
+    def shortest(call):
+        best, got = 1e9, None
+        for _ in range(10):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            assert call() == 0
+            b.record()
+            b.synchronize()
+            best, got = min(best, a.elapsed_time(b)), out.cpu().numpy()
+        return best, got
+
+    old, u = shortest(lambda: lib.fdm_launchMeshSignedDistanceGrid(*common, stream))
+    new, w = shortest(lambda: lib.fdm_launchMeshSignedDistanceGridWith(*common, C.c_void_p(work.data_ptr()),
+                                                                       C.c_size_t(need), stream))
+    print(f"{len(f)} triangles, {vals.size} nodes: {1e3 * old:.0f} us, grid path {1e3 * new:.0f} us", flush=True)
+    assert need > 0 and np.array_equal(u, w) and new <= 1.2 * old
