@@ -559,7 +559,19 @@ struct LSParticle {
   // 8192 bodies 0.19 -> 0.14 ms, one body 0.27 -> 0.04 ms.
   void finalize(hipStream_t s, const StateArrays& out = {}) {
     const size_t n = num();
-    if (n == 0 || !x_.get()) return;
+    if (n == 0) return;
+    if (!x_.get()) {  // before initialize(): the bodies as they were added
+      auto rows = [&](const void* host, double* user, size_t width) {
+        if (user) std::memcpy(user, host, width * n * sizeof(double));
+      };
+      rows(position_.data(), out.x, 3);
+      rows(velocity_.data(), out.v, 3);
+      rows(angularVelocity_.data(), out.w, 3);
+      rows(force_.data(), out.F, 3);
+      rows(torque_.data(), out.T, 3);
+      rows(orientation_.data(), out.q, 4);
+      return;
+    }
     if (x_.size() < 3 * n) throw std::runtime_error("download: bodies added since initialize()");
     const size_t blocks = (n + kStageBodies - 1) / kStageBodies;
     const size_t workers = std::min(blocks, kStageSlots);

@@ -31,3 +31,31 @@ def test_every_value_in_its_place(n, precision):
     assert np.isfinite(b["F"]).all() and np.isfinite(b["T"]).all()
     assert not np.array_equal(b["x"], a["x"])
     g.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_state_before_initialize_is_the_bodies_as_added(precision):
+    """The added bodies come back from the host (no step, nothing rounded to
+    the storage precision yet); after initialize() the device's state does."""
+    from fundem_amd import Solver
+
+    class Unstarted(Exception):
+        pass
+
+    class Probe(Solver):
+        def initialize(self, *a):
+            raise Unstarted
+
+    scn = W.cluster(n=30, seed=3, templates=W.superellipsoid_family(2, 5, n_grid=8, n_nodes=20))
+    g = Probe(precision=precision)
+    with pytest.raises(Unstarted):
+        W.apply(scn, g)
+    a = g.state()
+    for key in ("x", "v", "w"):
+        assert np.array_equal(a[key], getattr(scn, key)), key
+    assert np.abs(a["q"] - scn.q).max() <= 4 * np.finfo(float).eps
+    assert not a["F"].any() and not a["T"].any()
+    g.close()
+    empty = Solver(precision=precision)
+    assert empty.state()["x"].shape == (0, 3)
+    empty.close()
