@@ -162,7 +162,8 @@ struct LSParticle {
     t.size[1] = size.y;
     t.size[2] = size.z;
     t.sdfStart = (long long)sdf_.size();
-    for (double v : sdf) sdf_.push_back((float)v);
+    sdf_.resize(sdf_.size() + sdf.size());
+    for (size_t k = 0; k < sdf.size(); ++k) sdf_[t.sdfStart + k] = (float)sdf[k];
     t.nodeStart = (int)(nodes_.size() / 3);
     t.nodeCount = (int)nodes.size();
     double radius = 0.;
@@ -221,11 +222,12 @@ struct LSParticle {
             e[1] = std::max(e[1], std::fabs((double)s[ay + sy] - s[ay]));
             e[2] = std::max(e[2], std::fabs((double)s[az + sz] - s[az]));
           }
-          Lc = std::max(Lc, std::sqrt(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]));
+          Lc = std::max(Lc, e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
         }
-    t.lipschitz = Lc * t.invSpacing * (1.0 + 1e-9);
+    t.lipschitz = std::sqrt(Lc) * t.invSpacing * (1.0 + 1e-9);
     addGroups(t, fn);
-    addCells(t, s, (float)(1e-6 * spacing));
+    t.cellStart = cellCount_;  // (codes: upload())
+    cellCount_ += (long long)(size.x - 1) * (size.y - 1) * (size.z - 1);
     double reach = 0.0;
     for (int c = 0; c < 8; ++c) {
       const double px = origin.x + ((c & 1) ? spacing * (size.x - 1) : 0.0);
@@ -287,127 +289,63 @@ struct LSParticle {
   // FDM_GROUP slots are compact patches; each group's box centre and
   // enclosing radius (over the FP32 coordinates it stores, rounded up).
   void addGroups(fdm_template& t, const std::vector<double3>& fn) {
-    std::vector<int> ids(fn.size());
-    for (size_t k = 0; k < ids.size(); ++k) ids[k] = (int)k;
-    auto at = [&](int k, int a) { return a == 0 ? fn[k].x : a == 1 ? fn[k].y : fn[k].z; };
-    std::vector<std::pair<size_t, size_t>> todo{{0, ids.size()}};
+    struct Node {
+      double c[3];
+      int id;
+    };
+    std::vector<Node> v(fn.size());
+    for (size_t k = 0; k < v.size(); ++k) v[k] = {{fn[k].x, fn[k].y, fn[k].z}, (int)k};
+    auto box = [&](size_t b, size_t e, double* lo, double* hi) {
+      for (int a = 0; a < 3; ++a) lo[a] = hi[a] = v[b].c[a];
+      for (size_t k = b; k < e; ++k)
+        for (int a = 0; a < 3; ++a) {
+          lo[a] = std::min(lo[a], v[k].c[a]);
+          hi[a] = std::max(hi[a], v[k].c[a]);
+        }
+    };
+    double lo[3], hi[3];
+    std::vector<std::pair<size_t, size_t>> todo{{0, v.size()}};
     while (!todo.empty()) {
       const auto [b, e] = todo.back();
       todo.pop_back();
       if (e - b <= FDM_GROUP) continue;
+      box(b, e, lo, hi);
       int axis = 0;
-      double widest = -1.0;
-      for (int a = 0; a < 3; ++a) {
-        double lo = at(ids[b], a), hi = lo;
-        for (size_t k = b; k < e; ++k) {
-          lo = std::min(lo, at(ids[k], a));
-          hi = std::max(hi, at(ids[k], a));
-        }
-        if (hi - lo > widest) {
-          widest = hi - lo;
-          axis = a;
-        }
-      }
+      for (int a = 1; a < 3; ++a)
+        if (hi[a] - lo[a] > hi[axis] - lo[axis]) axis = a;
       const size_t groups = (e - b + FDM_GROUP - 1) / FDM_GROUP;
       const size_t cut = b + groups / 2 * FDM_GROUP;
-      std::nth_element(ids.begin() + b, ids.begin() + cut, ids.begin() + e, [&](int i, int j) {
-        const double u = at(i, axis), v = at(j, axis);
-        return u != v ? u < v : i < j;
+      std::nth_element(v.begin() + b, v.begin() + cut, v.begin() + e, [axis](const Node& i, const Node& j) {
+        return i.c[axis] != j.c[axis] ? i.c[axis] < j.c[axis] : i.id < j.id;
       });
       todo.push_back({b, cut});
       todo.push_back({cut, e});
     }
     t.groupStart = (int)(groups_.size() / 4);
-    t.groupCount = (int)((fn.size() + FDM_GROUP - 1) / FDM_GROUP);
+    t.groupCount = (int)((v.size() + FDM_GROUP - 1) / FDM_GROUP);
+    groupNodes_.resize(4 * FDM_GROUP * size_t(t.groupStart + t.groupCount), 0.f);
+    float* slot = groupNodes_.data() + 4 * FDM_GROUP * size_t(t.groupStart);
     for (int g = 0; g < t.groupCount; ++g) {
-      const size_t b = size_t(g) * FDM_GROUP, e = std::min(ids.size(), b + FDM_GROUP);
-      double lo[3], hi[3];
-      for (int a = 0; a < 3; ++a) lo[a] = hi[a] = at(ids[b], a);
-      for (size_t k = b; k < e; ++k)
-        for (int a = 0; a < 3; ++a) {
-          lo[a] = std::min(lo[a], at(ids[k], a));
-          hi[a] = std::max(hi[a], at(ids[k], a));
-        }
+      const size_t b = size_t(g) * FDM_GROUP, e = std::min(v.size(), b + FDM_GROUP);
+      box(b, e, lo, hi);
       const float c[3] = {(float)(0.5 * (lo[0] + hi[0])), (float)(0.5 * (lo[1] + hi[1])),
                           (float)(0.5 * (lo[2] + hi[2]))};
-      double r = 0.0;
-      for (size_t k = b; k < b + FDM_GROUP; ++k) {
-        const int id = k < e ? ids[k] : -1;
-        float slot[4] = {0.f, 0.f, 0.f, 0.f};
+      double r2 = 0.0;
+      for (size_t k = b; k < b + FDM_GROUP; ++k, slot += 4) {
+        const int id = k < e ? v[k].id : -1;
         if (id >= 0) {
           double d = 0.0;
           for (int a = 0; a < 3; ++a) {
-            slot[a] = (float)at(id, a);
+            slot[a] = (float)v[k].c[a];
             d += ((double)slot[a] - c[a]) * ((double)slot[a] - c[a]);
           }
-          r = std::max(r, std::sqrt(d));
+          r2 = std::max(r2, d);
         }
         std::memcpy(slot + 3, &id, sizeof(float));
-        groupNodes_.insert(groupNodes_.end(), slot, slot + 4);
       }
       groups_.insert(groups_.end(), c, c + 3);
-      groups_.push_back(std::nextafter((float)r, std::numeric_limits<float>::infinity()));
+      groups_.push_back(std::nextafter((float)std::sqrt(r2), std::numeric_limits<float>::infinity()));
     }
-  }
-  // Cell codes of one template (FDM_CELL_UNIT): cells with a corner at or
-  // below `low` (a millionth of the spacing: elsewhere the interpolant stays
-  // positive whatever its rounding) are 0; every other cell takes the
-  // distance between its box and the nearest such cell's box, in units of
-  // 1 / FDM_CELL_UNIT spacings rounded down, saturating past 16 spacings.
-  // The squared distance is a sum over the axes, so it is folded axis by
-  // axis: along x from the nearest marked cell on either side, along y and z
-  // over the 16 cells either way. A grid of more than 2^22 cells keeps all
-  // codes 0 (nothing is culled by them).
-  void addCells(fdm_template& t, const float* s, float low) {
-    const int nx = t.size[0] - 1, ny = t.size[1] - 1, nz = t.size[2] - 1;
-    const size_t n = size_t(nx) * ny * nz;
-    t.cellStart = (long long)cells_.size();
-    cells_.resize(cells_.size() + n, 0);
-    if (n > (size_t(1) << 22)) return;
-    constexpr int kFar = 16 * 16;
-    std::vector<unsigned short> d(n), f(n);
-    std::vector<char> solid(n);
-    const size_t sy = size_t(t.size[0]), sz = sy * t.size[1];
-    for (int z = 0; z < nz; ++z)
-      for (int y = 0; y < ny; ++y) {
-        const float* c = s + size_t(z) * sz + size_t(y) * sy;
-        char* o = solid.data() + (size_t(z) * ny + y) * nx;
-        for (int x = 0; x < nx; ++x)
-          o[x] = c[x] <= low || c[x + 1] <= low || c[x + sy] <= low || c[x + sy + 1] <= low ||
-                 c[x + sz] <= low || c[x + sz + 1] <= low || c[x + sz + sy] <= low ||
-                 c[x + sz + sy + 1] <= low;
-        unsigned short* r = d.data() + (size_t(z) * ny + y) * nx;
-        auto gap2 = [&](int cells) { return (unsigned short)std::min(kFar, cells <= 1 ? 0 : (cells - 1) * (cells - 1)); };
-        for (int x = 0, last = -1000; x < nx; ++x) {
-          if (o[x]) last = x;
-          r[x] = gap2(std::min(x - last, 100));
-        }
-        for (int x = nx - 1, next = 100000; x >= 0; --x) {
-          if (o[x]) next = x;
-          r[x] = std::min(r[x], gap2(std::min(next - x, 100)));
-        }
-      }
-    auto fold = [&](int count, size_t stride, size_t lines, size_t lineStride, size_t run) {
-      for (size_t l = 0; l < lines; ++l)
-        for (int i = 0; i < count; ++i) {
-          unsigned short* out = f.data() + l * lineStride + size_t(i) * stride;
-          std::fill(out, out + run, (unsigned short)kFar);
-          for (int j = std::max(0, i - 16); j <= std::min(count - 1, i + 16); ++j) {
-            const int gap = std::max(std::abs(i - j) - 1, 0);
-            const unsigned short g = (unsigned short)(gap * gap);
-            const unsigned short* in = d.data() + l * lineStride + size_t(j) * stride;
-            for (size_t x = 0; x < run; ++x) out[x] = std::min<unsigned short>(out[x], in[x] + g);
-          }
-        }
-      d.swap(f);
-    };
-    fold(ny, nx, nz, size_t(nx) * ny, nx);
-    fold(nz, size_t(nx) * ny, 1, 0, size_t(nx) * ny);
-    unsigned char code[kFar + 1];
-    for (int q = 0; q <= kFar; ++q)
-      code[q] = (unsigned char)std::min(255, 1 + int(std::floor(FDM_CELL_UNIT * std::sqrt(double(q)) * (1.0 - 1e-9))));
-    unsigned char* o = cells_.data() + t.cellStart;
-    for (size_t k = 0; k < n; ++k) o[k] = solid[k] ? 0 : code[std::min<int>(d[k], kFar)];
   }
 
   // LSParticle::addParticle (LSParticle.h:292-342).
@@ -544,7 +482,17 @@ struct LSParticle {
     dchunks_.upload(chunks_, s);
     dgroups_.upload(groups_, s);
     dgroupNodes_.upload(groupNodes_, s);
-    dcells_.upload(cells_, s);
+    DeviceBuffer<unsigned char> work;
+    if (cellCount_ > 0) {
+      long long most = 0;
+      for (const auto& t : templates_)
+        most = std::max(most, (long long)(t.size[0] - 1) * (t.size[1] - 1) * (t.size[2] - 1));
+      dcells_.allocate((size_t)cellCount_, false);
+      work.allocate(2 * (size_t)cellCount_, false);
+      fdmCheck(fdm_launchCellCodes(dtmpl_.get(), (int)templates_.size(), most, dsdf_.get(), dcells_.get(), cellCount_,
+                                   work.get(), work.size(), s),
+               "cell codes");
+    }
     hipCheck(hipStreamSynchronize(s), "upload");
   }
 
@@ -720,7 +668,7 @@ struct LSParticle {
   std::vector<fdm_material> materials_;
   std::vector<fdm_template> templates_;
   std::vector<float> sdf_, chunks_, groups_, groupNodes_;
-  std::vector<unsigned char> cells_;
+  long long cellCount_ = 0;  // SDF cells of all templates
   std::vector<fdm_real> nodes_;
   std::vector<std::vector<double3>> nodeHost_;
   std::vector<std::vector<int3>> connectivity_;

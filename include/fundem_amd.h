@@ -680,6 +680,14 @@ size_t fdm_buildListsWorkspaceBytes(size_t n);
 int fdm_launchBuildLists(const fdm_build_args* args, void* workspace, size_t workspaceBytes,
                          hipStream_t stream);
 
+/* Cell codes (FDM_CELL_UNIT) of `count` templates on the device from their SDF
+ * values, into cells [totalCells] at each template's cellStart; mostCells: the
+ * cells of the largest grid. workspace: at least 2 * totalCells bytes. Grids
+ * of more than 2^22 cells get zeros. */
+int fdm_launchCellCodes(const fdm_template* templates, int count, long long mostCells, const float* sdf,
+                        unsigned char* cells, long long totalCells, void* workspace, size_t workspaceBytes,
+                        hipStream_t stream);
+
 /* State of bodies first to first + count - 1 as rows for the host, FP64: x v w
  * F T (3 each) and q (4), all rows of one quantity before the next, into
  * out [19 * count] (device or mapped host memory). */
