@@ -12,7 +12,6 @@
 #include <exception>
 #include <iostream>
 #include <limits>
-#include <memory>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -456,7 +455,6 @@ struct LSParticle {
         xb[2 * n + i] = position_[i].z;
       }
       x_.allocate(3 * m, false);
-      allocateStage(n);
       x_.upload(xb, s);
       hipCheck(hipStreamSynchronize(s), "upload");
     }
@@ -523,11 +521,13 @@ struct LSParticle {
     if (x_.size() < 3 * n) throw std::runtime_error("download: bodies added since initialize()");
     const size_t blocks = (n + kStageBodies - 1) / kStageBodies;
     const size_t workers = std::min(blocks, kStageSlots);
-    allocateStage(n);
+    const size_t slotWords = 19 * std::min(n, kStageBodies);
+    if (workers > 1 && stageEvents_.empty()) stageEvents_ = std::vector<Event>(kStageSlots);
+    Lease stage(workers * slotWords);
     int device = 0;
     hipCheck(hipGetDevice(&device), "download");
     auto work = [&](size_t w) {
-      double* slot = stage_.get() + w * 19 * std::min(n, kStageBodies);
+      double* slot = stage.block.p + w * slotWords;
       for (size_t k = w; k < blocks; k += workers) {
         const size_t first = k * kStageBodies, count = std::min(kStageBodies, n - first);
         fdmCheck(fdm_launchPackState(bodies(), (int)first, (int)count, slot, s), "download");
@@ -553,6 +553,7 @@ struct LSParticle {
     };
     if (workers == 1) {
       work(0);
+      stage.idle = true;
       return;
     }
     std::vector<std::exception_ptr> failed(workers);
@@ -575,6 +576,7 @@ struct LSParticle {
     for (size_t w = started; w < workers; ++w) guarded(w);
     for (auto& f : failed)
       if (f) std::rethrow_exception(f);
+    stage.idle = true;
   }
 
   fdm_bodies bodies() {
@@ -677,10 +679,19 @@ struct LSParticle {
   std::vector<int> materialID_, geometryID_, system_;
   int currentSystem_ = 0;
 
-  // pinned slots of finalize()
+  // finalize(): bodies of a block, pinned slots, and their memory (given back
+  // when the last copy from it is done, freed after an error)
   static constexpr size_t kStageBodies = 8192, kStageSlots = 8;
-  struct PinnedFree {
-    void operator()(double* p) const { (void)hipHostFree(p); }
+  struct Lease {
+    explicit Lease(size_t words) : block(PinnedPool::get().take(words)) {}
+    Lease(const Lease&) = delete;
+    Lease& operator=(const Lease&) = delete;
+    ~Lease() {
+      if (idle) PinnedPool::get().give(block);
+      else (void)hipHostFree(block.p);  // (waits for the device)
+    }
+    PinnedPool::Block block;
+    bool idle = false;
   };
   struct Event {
     hipEvent_t e = nullptr;
@@ -694,19 +705,6 @@ struct LSParticle {
       if (e) (void)hipEventDestroy(e);
     }
   };
-  void allocateStage(size_t n) {
-    const size_t words = 19 * std::min(n, kStageBodies) * std::min((n + kStageBodies - 1) / kStageBodies, kStageSlots);
-    if (words <= stageWords_) return;
-    stage_.reset();
-    stageWords_ = 0;
-    double* p = nullptr;
-    hipCheck(hipHostMalloc((void**)&p, words * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
-    stage_.reset(p);
-    if (stageEvents_.empty()) stageEvents_ = std::vector<Event>(kStageSlots);
-    stageWords_ = words;
-  }
-  std::unique_ptr<double, PinnedFree> stage_;
-  size_t stageWords_ = 0;
   std::vector<Event> stageEvents_;
 
   DeviceBuffer<double> x_;

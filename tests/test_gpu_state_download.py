@@ -59,3 +59,31 @@ def test_state_before_initialize_is_the_bodies_as_added(precision):
     empty = Solver(precision=precision)
     assert empty.state()["x"].shape == (0, 3)
     empty.close()
+
+
+def test_reads_by_several_threads_and_of_several_sizes():
+    """The pinned blocks of the reads are kept by the process and taken by
+    whichever read comes: threads with solvers of one block, two and nine, each
+    reading its own bodies again and again; then solvers created and closed."""
+    import threading
+    from fundem_amd import Solver
+    tm = W.superellipsoid_family(2, 5, n_grid=8, n_nodes=20)
+    scns = {n: W.cluster(n=n, seed=n, templates=tm) for n in (3, 9000, 73729, 500)}
+    wrong = []
+
+    def read(n, count):
+        g = Solver()
+        W.apply(scns[n], g)
+        for _ in range(count):
+            if not np.array_equal(g.state()["x"], scns[n].x):
+                wrong.append(n)
+        g.close()
+
+    threads = [threading.Thread(target=read, args=(n, 12)) for n in scns]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for n in (9000, 3, 73729, 500, 3):
+        read(n, 1)
+    assert not wrong
