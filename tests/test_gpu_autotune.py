@@ -39,8 +39,11 @@ def test_autotune_keeps_results(periodic):
         assert np.array_equal(got[key], ref[key]), key
 
 
-SHAPES = [dict(sweep_waves=w, nodes_per_lane=npl, law_mode=1) for w in (1, 4) for npl in (1, 2, 3)] + \
-         [dict(sweep_waves=w, law_mode=2) for w in (1, 2)]
+# (the last one's fields are accepted without effect in law mode 1)
+SHAPES = [dict(law_mode=1, sweep_waves_per_cu=pc) for pc in (4, 16, 64)] + \
+         [dict(law_mode=1, reduce_block=b) for b in (64, 1024)] + \
+         [dict(law_mode=2, sweep_waves=w, sweep_waves_per_cu=pc) for w, pc in ((1, 32), (2, 16), (4, 4))] + \
+         [dict(law_mode=1, sweep_waves=4, nodes_per_lane=3, law_block=64, wall_groups=2)]
 
 
 def _shapes_case(name):
@@ -58,9 +61,10 @@ def _shapes_case(name):
 
 @pytest.mark.parametrize("name", ["pour", "pressed"])
 def test_launch_shapes_keep_results(name):
-    """Every launch shape of one solver (sweep waves per workgroup, how a
-    sweep wave walks a pair's chunks, where the contact law runs) gives the
-    same bits: a 5^3 slice of the pour whose layers collide (particle, wall
+    """Every launch shape of one solver (sweep grid size, the sweep in runs or
+    one pair per wave by chunks with one to four waves per workgroup, reduction
+    workgroup size; steps one at a time, where the reduction has a kernel of
+    its own, as well as joined) gives the same bits: a 5^3 slice of the pour whose layers collide (particle, wall
     and ghost contacts) and a pair held at more than 64 node contacts."""
     from fundem_amd import Solver
     scn, steps = _shapes_case(name)
@@ -69,9 +73,12 @@ def test_launch_shapes_keep_results(name):
         g = Solver()
         g.set_launch_tuning(**shape)
         W.apply(scn, g)
-        g.step(steps)
+        g.step(steps - 20)
+        for _ in range(20):
+            g.step(1)
         assert g.status() == 0
-        assert g.launch_tuning()["nodes_per_lane"] == shape.get("nodes_per_lane", 1)
+        tuning = g.launch_tuning()
+        assert all(tuning[key] == value for key, value in shape.items()), (shape, tuning)
         runs.append((shape, g.state(), [g.contacts(k)["A"].size for k in range(5)]))
         g.close()
     print(f"{name}: contacts per set {runs[0][2]}", flush=True)

@@ -1,9 +1,14 @@
 """Body state to the host in blocks of 8192 bodies through up to eight pinned
 slots, one thread each (LSParticle::finalize): every body's values in its row,
-for one block, its edges, two blocks, and more blocks than slots."""
+for one block, its edges, two blocks, and more blocks than slots: as added, and
+against the oracle's rows after steps in which nearly every body has a force
+and a torque of its own."""
+import dataclasses
+
 import numpy as np
 import pytest
 
+import pyoracle as po
 from fundem_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -14,6 +19,8 @@ pytestmark = pytest.mark.gpu
 def test_every_value_in_its_place(n, precision):
     from fundem_amd import Solver
     scn = W.cluster(n=n, seed=3, templates=W.superellipsoid_family(2, 5, n_grid=8, n_nodes=20))
+    c = scn.x.mean(0)
+    scn = dataclasses.replace(scn, x=c + 0.65 * (scn.x - c))  # in contact with the neighbours
     real = np.float32 if precision == "fp32" else np.float64
     g = Solver(precision=precision)
     W.apply(scn, g)
@@ -24,12 +31,18 @@ def test_every_value_in_its_place(n, precision):
     # (orientations are normalised first: a few roundings of components up to 1)
     assert np.abs(a["q"] - scn.q).max() <= 4 * np.finfo(real).eps
     g.step(3)
-    b, c = g.state(), g.state()
+    o = po.OracleSim(precision == "fp32", True)
+    W.apply(scn, o)
+    o.step(3)
+    b, want = g.state(), o.state()
     for key in b:
-        assert np.array_equal(b[key], c[key]), key
-    # weight and velocity agree: no body of another row
-    assert np.isfinite(b["F"]).all() and np.isfinite(b["T"]).all()
-    assert not np.array_equal(b["x"], a["x"])
+        assert np.array_equal(b[key], want[key]), key
+    if n > 2:
+        # rows that could not be told apart would not show a misplaced one
+        for key in ("F", "T"):
+            rows = np.unique(want[key][np.abs(want[key]).sum(1) > 0], axis=0)
+            assert len(rows) > 0.95 * n, (key, len(rows))
+        assert not np.array_equal(want["F"], want["T"])
     g.close()
 
 
