@@ -360,6 +360,7 @@ __device__ __forceinline__ void decideLast(const StepBeginK& k, float rate, int 
   __shared__ int last;
   const int nb = gridDim.x;
   foldBlock(rate, flags);
+  rate = fmaxf(rate, 0.f);  // (no number, if no body has one: as an int it would exceed every rate)
   int* fold = k.s.fold;
   const int slots = nb <= kFoldSlots ? 1 : kFoldSlots;
   if (nb > 1) {

@@ -5,6 +5,8 @@ Steps queued in one call are chained that way; a call of a single step ends
 with the fold kernel and begins with the step-begin kernel. Both have to give
 the same bits, at the sizes where the decision changes hands: one workgroup of
 256 bodies, two, and 64 and more (a second level of arrival counters)."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -57,3 +59,31 @@ def test_chained_periodic_and_bonded_steps_equal_single_steps():
         ref = run(scn, [1] * steps, False, "fp32", 0)
         assert_same(run(scn, [steps], True, "fp32"), ref)
         assert_same(run(scn, [steps // 2, steps - steps // 2], False, "fp32", 3), ref)
+
+
+def test_a_system_that_is_no_number_leaves_the_others_their_lists():
+    """A batch in which one system of several workgroups has lost its numbers
+    (a run that blew up): the other system's lists are built again as it moves,
+    and its states and contacts are those of the run alone."""
+    from fundem_amd import Solver
+    tm = W.superellipsoid_family(2, 5, n_grid=12, n_nodes=100)
+    lost = W.cluster(n=700, seed=1, templates=tm, walls=False)
+    lost = dataclasses.replace(lost, v=np.full_like(lost.v, np.nan))
+    moving = W.cluster(n=64, seed=2, templates=tm, speed=0.2)
+    moving = dataclasses.replace(moving, v=moving.v - (moving.x - moving.x.mean(0)) / 1e-3)
+    alone = Solver()
+    W.apply(moving, alone)
+    both = Solver()
+    W.apply_batch([lost, moving], both)
+    seen = 0
+    for i in range(8):
+        alone.step(40)
+        both.step(40)
+        a, b = alone.state(), both.state()
+        for key in ("x", "v", "w", "q", "F", "T"):
+            assert np.array_equal(a[key], b[key][700:]), (i, key)
+        u, v = alone.contacts(0), both.contacts(0)
+        assert np.array_equal(u["A"], v["A"][v["A"] >= 700] - 700), i
+        seen += u["A"].size
+    assert seen > 0 and alone.list_builds()[0] > 1
+    assert np.isnan(both.state()["x"][:700]).all()
