@@ -136,7 +136,7 @@ class PinnedPool {
     }
     (void)hipHostFree(b.p);
   }
-  static constexpr size_t kIdle = 2, kLeast = size_t(1) << 17;
+  static constexpr size_t kIdle = 4, kLeast = size_t(1) << 17;
 
  private:
   PinnedPool() { idle_.reserve(kIdle); }

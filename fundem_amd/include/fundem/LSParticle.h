@@ -455,6 +455,8 @@ struct LSParticle {
         xb[2 * n + i] = position_[i].z;
       }
       x_.allocate(3 * m, false);
+      // (the block finalize() will take, so that a read allocates nothing)
+      if (n > 0) PinnedPool::get().give(PinnedPool::get().take(stageWords(n)));
       x_.upload(xb, s);
       hipCheck(hipStreamSynchronize(s), "upload");
     }
@@ -523,7 +525,7 @@ struct LSParticle {
     const size_t workers = std::min(blocks, kStageSlots);
     const size_t slotWords = 19 * std::min(n, kStageBodies);
     if (workers > 1 && stageEvents_.empty()) stageEvents_ = std::vector<Event>(kStageSlots);
-    Lease stage(workers * slotWords);
+    Lease stage(stageWords(n));
     int device = 0;
     hipCheck(hipGetDevice(&device), "download");
     auto work = [&](size_t w) {
@@ -682,6 +684,9 @@ struct LSParticle {
   // finalize(): bodies of a block, pinned slots, and their memory (given back
   // when the last copy from it is done, freed after an error)
   static constexpr size_t kStageBodies = 8192, kStageSlots = 8;
+  static size_t stageWords(size_t n) {
+    return 19 * std::min(n, kStageBodies) * std::min((n + kStageBodies - 1) / kStageBodies, kStageSlots);
+  }
   struct Lease {
     explicit Lease(size_t words) : block(PinnedPool::get().take(words)) {}
     Lease(const Lease&) = delete;
