@@ -177,10 +177,9 @@ def autotune(s, a):
     for line in c["trials"]:
         log("  tune " + line)
     log(f"autotuned in {time.perf_counter() - t0:.1f} s: skin {c['skin']:.3e} m, cell "
-        f"{c['cell_size']:.3e} m (0: the cell rule), sweep {c['sweep_waves']} waves/workgroup, "
-        f"{c['sweep_waves_per_cu']} waves/CU, {c['nodes_per_lane']} node(s) per lane, law mode "
-        f"{c['law_mode']}, law block {c['law_block']}, reduce block "
-        f"{c['reduce_block']} ({c['ms_per_step']:.3f} ms/step in the trials)")
+        f"{c['cell_size']:.3e} m (0: the cell rule), sweep "
+        f"{c['sweep_waves_per_cu']} waves/CU, law mode {c['law_mode']} (of {c['sweep_waves']} "
+        f"waves/workgroup where 2), reduce block {c['reduce_block']} ({c['ms_per_step']:.3f} ms/step in the trials)")
     return {k: (float(v) if not isinstance(v, int) else v) for k, v in c.items() if k != "trials"}
 
 

@@ -782,10 +782,8 @@ __global__ void __launch_bounds__(256) kNarrow(NarrowK a) {
 }
 
 // ---------------------------------------------------------------------------
-// Narrow phase of several sets in three kernels: a pair-level cull (one thread
-// per candidate pair), the node sweep (one wave per kept pair) that stages the
-// geometry of every contact, and the contact law (one thread per kept pair)
-// that walks its contacts in node order.
+// Narrow phase of several sets in one kernel: culls, exact predicate and
+// contact law of runs of pairs (sweepRun).
 
 struct NarrowScratch {
   double* hitGeom;   // [8 * hitCapacity]: contact point, normal, overlap, node id
@@ -1753,7 +1751,7 @@ extern "C" int fdm_launchNarrowPhase(const fdm_narrowphase_args* args, hipStream
 
 extern "C" int fdm_launchNarrowPhaseSets(const fdm_narrowphase_args* sets, int nsets,
                                          const fdm_narrow_workspace* ws, hipStream_t stream) {
-  if (!sets || nsets < 1 || nsets > kMaxSets || !ws || !ws->workHit || !ws->hitGeom ||
+  if (!sets || nsets < 1 || nsets > kMaxSets || !ws || !ws->hitGeom ||
       !ws->hitCount || ws->hitCapacity < FDM_REC_POOLS)
     return FDM_EINVAL;
   NarrowMulti k;

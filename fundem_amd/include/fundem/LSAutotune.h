@@ -22,9 +22,8 @@
 //     each step by their own cell rule), nor for batched systems (their
 //     packings are configured with cells below twice the largest radius: a
 //     coarser candidate changed their contacts and overflowed a mirror list);
-//   - the solver's launch shapes (fdm_tuning): sweep grid size, where the
-//     contact law runs (a kernel of its own, or the sweep's wave),
-//     contact-law and reduction workgroup sizes.
+//   - the solver's launch shapes (fdm_tuning): sweep grid size, the sweep in
+//     runs of pairs or one pair per wave, reduction workgroup size.
 // Each candidate is timed from the same saved point (LSAdjoint::mark /
 // rollback) one knob at a time, keeping the best value of each knob before
 // the next; the solver is left at the saved point with the best settings.

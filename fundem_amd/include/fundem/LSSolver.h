@@ -411,7 +411,9 @@ class LSSolver {
   }
   // Steps queued ahead of the list decisions the host has read (advance);
   // 0 waits for every step's decision before queueing the next. At most
-  // FDM_DECISION_RING - 1; default 8 (two graphs of four steps).
+  // FDM_DECISION_RING - 1, as the last queued step's reduction takes the next
+  // step's decision too and the ring must hold every one not read; default 8
+  // (two graphs of four steps).
   void setLookahead(int steps) {
     lookahead_ = std::max(0, std::min(steps, FDM_DECISION_RING - 1));
   }
@@ -1381,10 +1383,8 @@ class LSSolver {
     na[0].gate = gate;
     {
       Timer t(this, "narrow");
-      fdm_narrow_workspace w;
+      fdm_narrow_workspace w{};
       w.workCapacity = workCapacity_;
-      w.workCount = nullptr;
-      w.workHit = listTmp_.get();
       w.hitGeom = hitGeom_.get();
       w.hitCapacity = hitCapacity_;
       w.hitCount = hitCount_.get();

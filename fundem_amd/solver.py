@@ -229,9 +229,10 @@ class Solver:
     def set_launch_tuning(self, sweep_waves=0, sweep_waves_per_cu=0, law_block=0, reduce_block=0,
                           law_mode=0, nodes_per_lane=0, wall_groups=0):
         """This solver's launch shapes (results do not depend on them); zero
-        keeps the process default of a field. wall_groups: 1 sweeps wall
-        pairs four per wave whatever the system's size, 2 never (0: for wall
-        sets sized for at least 65536 pairs)."""
+        keeps the process default of a field. law_mode 1 sweeps runs of pairs
+        culled by cell codes, 2 one pair per wave culled by chunk (with
+        sweep_waves waves per workgroup); law_block, nodes_per_lane and
+        wall_groups are accepted without effect."""
         t = np.array([sweep_waves, sweep_waves_per_cu, law_block, reduce_block, law_mode,
                       nodes_per_lane, wall_groups], np.int32)
         self._ok(self._lib.fdmx_set_launch_tuning(self.h, _ip_(t)))
@@ -415,7 +416,12 @@ class Solver:
         return dict(radius=r[0], inv_mass=im[0], inertia=I, inv_inertia=Ii, origin=o)
 
     def stage_times(self):
-        """{stage: (total device ms, launches timed)} since set_timing(True)."""
+        """{stage: (total device ms, launches timed)} since set_timing(True):
+        step_begin (with the list decision), list_build, narrow, bonds,
+        reduce_kick; where the lists are built stage by stage (sector boundary,
+        more than 1024 walls) sort_cells, periodic_build, broad_pp, broad_pw
+        and broad_ghost in place of list_build. Timed steps run one at a
+        time, so that the reduction and the next step's begin are apart."""
         names = C.create_string_buffer(4096)
         ms = np.zeros(64)
         calls = np.zeros(64, np.int64)

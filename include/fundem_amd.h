@@ -214,9 +214,8 @@ typedef struct {
   int* hostDecision;   /* optional host-visible ring of FDM_DECISION_RING words: decision
                           number k writes word k % FDM_DECISION_RING with
                           (k << 2) | rebuild << 1 | ghost rebuild, last (for a host that
-                          launches only the work a step needs, and may queue up to
-                          FDM_DECISION_RING - 1 steps ahead of the decisions it has read);
-                          NULL to skip */
+                          launches only the work a step needs; at most FDM_DECISION_RING
+                          decisions may be queued beyond those it has read); NULL to skip */
   int* fold;           /* [FDM_FOLD_WORDS], zero before the first use: where the workgroups of
                           fdm_launchStepBeginDecide and fdm_launchReduceStep meet (NULL: those
                           two are refused); left zero by each launch. One step at a time. */
@@ -378,7 +377,8 @@ int fdm_launchKickDriftHash(fdm_bodies bodies, fdm_geometry geo, fdm_double3 gra
  * periodic); a wrap seen by the prepare stage also rebuilds the next step. */
 int fdm_launchSkinDecide(const fdm_skin* skin, hipStream_t stream);
 /* No counterpart in the reference: the first phase of a step in two
- * launches. fdm_launchStepBegin: kick (when `kick`), drift (when `drift`)
+ * launches, for callers without fdm_skin.fold (the solver's steps take
+ * fdm_launchStepBeginDecide and fdm_launchReduceStep). fdm_launchStepBegin: kick (when `kick`), drift (when `drift`)
  * and cell id (table.hashValue) of every particle, drift and cell id of
  * every wall, the periodic visibility of every particle against its state at
  * the last ghost list build (the flags are stored only where ghostFlag[k] is
@@ -610,7 +610,7 @@ typedef struct {
   int* workList;               /* unused (may be NULL); kept for the layout */
   int workCapacity;            /* at least the sum of the sets' pair capacities */
   int* workCount;              /* unused (may be NULL); kept for the layout */
-  int* workHit;                /* not NULL; unused, kept for the layout */
+  int* workHit;                /* unused (may be NULL); kept for the layout */
   double* hitGeom;             /* [8 * hitCapacity] staged contacts (runs of pairs with more
                                   contacts than one wave holds, 64) */
   int hitCapacity;             /* staged contacts, split into FDM_REC_POOLS pools */
