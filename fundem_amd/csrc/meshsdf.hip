@@ -223,17 +223,17 @@ __global__ __launch_bounds__(kMeshTile) void kMeshDistance(const double* __restr
 //    the brick first (kMeshNearest). The chunks take the triangles in their
 //    order: a mesh in no spatial order is slower, not wrong.
 // Bound by FP64 VALU, and on small grids by the brick with the most triangles
-// in reach. An open mesh pays for every solid angle; on grids of few bricks it
-// finds the nearest triangle in the same loop, as the longest brick cannot hide
-// there (20479 triangles, 15925 nodes: 3.0 ms, 3.7 with kMeshNearest, 2.9-3.3
-// as kMeshDistance; 2601 nodes, 5119 triangles 0.24 ms against 0.42 and 0.62).
-// Measured, a whole call of the host class: 57K nodes and 5120
+// in reach. An open mesh pays for every solid angle, and on grids of few bricks
+// finds the nearest triangle in the same loop (kMeshSoloBricks). Measured, a whole call of the host class: 57K nodes and 5120
 // triangles 2.60 -> 0.43 ms (kernels 2.52 -> 0.33), 342K and 5120 13.1 -> 1.05
 // ms, 2.4M and 5120 87 -> 3.5 ms (4.5 with the triangles shuffled), 578K and
 // 20480 82 -> 3.6 ms.
 constexpr int kMeshChunk = 32;
 constexpr int kSolidStep = 4;  // kMeshSolid: triangles per thread between barriers
-constexpr int kSolidMany = 2048;
+// Nodes from which eight share a workgroup in kMeshSolid (5832 nodes and 5120
+// triangles 489 us with a workgroup each, 497 with eight; 8000 nodes 605 and
+// 583; 1000 nodes 345 and 405).
+constexpr int kSolidMany = 7168;
 // Sizes between which the signs are taken from crossings: a solid angle's
 // products of three lengths neither overflow nor vanish. A mesh beyond them, or
 // with a coordinate that is no number, has an infinite "largest coordinate",
@@ -683,9 +683,9 @@ __device__ __forceinline__ void solidNodes(const MeshWork& k, int first, int cou
 }
 
 // The nodes left. A workgroup for each where they are few, as the chain of
-// tiles is then the time; eight a workgroup from kSolidMany on, where one
-// node's sums, added by eight lanes, held up the other threads (57475 nodes,
-// 5119 triangles 3.40 -> 2.18 ms). solo: the grid of an open mesh, which
+// tiles is then the time; eight a workgroup from kSolidMany on. (With one load
+// and addition after another by the eight lanes that add, and a workgroup per
+// node, 57475 nodes and 5119 triangles took 3.40 ms instead of 2.18.) solo: the grid of an open mesh, which
 // kMeshNearest left out. Bound by FP64 VALU (some 300 instructions an angle).
 __global__ void __launch_bounds__(kMeshTile) __attribute__((amdgpu_waves_per_eu(4))) kMeshSolid(MeshWork k, int solo) {
   __shared__ SolidSlots ws;
@@ -742,6 +742,11 @@ namespace {
 constexpr long long kMeshGridPairs = 1ll << 22;
 // Bricks below which sixteen waves share one (980 bricks: 294 -> 238 us).
 constexpr unsigned kMeshFewBricks = 4096;
+// Bricks below which kMeshSolid finds an open mesh's nearest triangles: some
+// 1.2 ps per node and triangle on top of the angles, where the longest brick of
+// kMeshNearest takes up to 60 ns per triangle, the same at 48000 nodes (324
+// bricks, 20479 triangles 3.0 ms against 3.7; 980 bricks 10.2 against 9.8).
+constexpr unsigned kMeshSoloBricks = 768;
 bool meshGridPath(int nt, const int* size) {
   const long long count = (long long)size[0] * size[1] * size[2];
   return count < (1ll << 30) && count * nt >= kMeshGridPairs;
@@ -798,10 +803,10 @@ extern "C" int fdm_launchMeshSignedDistanceGridWith(const double* triangles, int
   // bricks to fill the chip with four each: its time is then the longest
   // brick's
   const unsigned bricks = (unsigned)((long long)bx * by * ((size[2] + 3) / 4));
-  const int few = bricks < kMeshFewBricks ? 1 : 0;
-  if (few) hipLaunchKernelGGL(kMeshNearest<16>, dim3(bricks), dim3(1024), 0, stream, k, bx, by, few);
-  else hipLaunchKernelGGL(kMeshNearest<4>, dim3(bricks), dim3(256), 0, stream, k, bx, by, few);
-  hipLaunchKernelGGL(kMeshSolid, dim3(persistentBlocks(4)), dim3(kMeshTile), 0, stream, k, few);
+  const int solo = bricks < kMeshSoloBricks ? 1 : 0;
+  if (bricks < kMeshFewBricks) hipLaunchKernelGGL(kMeshNearest<16>, dim3(bricks), dim3(1024), 0, stream, k, bx, by, solo);
+  else hipLaunchKernelGGL(kMeshNearest<4>, dim3(bricks), dim3(256), 0, stream, k, bx, by, solo);
+  hipLaunchKernelGGL(kMeshSolid, dim3(persistentBlocks(4)), dim3(kMeshTile), 0, stream, k, solo);
   return launchStatus();
 }
 

@@ -109,19 +109,20 @@ def test_unusual_coordinates_equal_the_point_kernel(what):
     assert np.array_equal(vals, want, equal_nan=True)
 
 
-@pytest.mark.parametrize("name,h", [("solo", 0.08), ("solo remainder", 0.05), ("many bricks", 0.035)])
+@pytest.mark.parametrize("name,h", [("solo", 0.08), ("bricks", 0.05), ("many bricks", 0.035)])
 def test_open_mesh_on_either_side_of_the_brick_rule(name, h):
     """Every node of an open mesh takes the solid angles: with the nearest
-    triangle in one loop on grids of few bricks, after kMeshNearest on more
-    than 4096; numbers of nodes and triangles that are no multiple of eight."""
+    triangle in one loop on grids of less than 768 bricks, after kMeshNearest
+    (sixteen waves a brick below 4096, four above) on larger ones; numbers of
+    nodes and triangles that are no multiple of eight."""
     v, f = G.icosphere(1.0, 1 if name == "many bricks" else 3)
     f = f[:-1]
     m = G.MeshParticle(v * (1.0, 1.1, 1.2), f)
     origin, hh, size, vals = m.build_grid(h)
     bricks = int(np.prod([(n + 3) // 4 for n in size]))
     print(f"{len(f)} triangles, {vals.size} nodes, {bricks} bricks", flush=True)
-    assert len(f) * vals.size >= 1 << 22 and (bricks >= 4096) == (name == "many bricks")
-    assert vals.size % 8 != 0 or name != "solo remainder"
+    assert len(f) * vals.size >= 1 << 22 and len(f) % 8 and vals.size % 8
+    assert name == ("solo" if bricks < 768 else "bricks" if bricks < 4096 else "many bricks")
     o2, s2, v2 = po.mesh_grid(v * (1.0, 1.1, 1.2), f, h, 2)
     assert np.array_equal(origin, o2) and size == s2 and np.array_equal(vals, v2)
 
@@ -164,3 +165,32 @@ def test_open_mesh_is_not_slower_than_every_triangle_at_every_node(nu, nv, res):
                                                                        C.c_size_t(need), stream))
     print(f"{len(f)} triangles, {vals.size} nodes: {1e3 * old:.0f} us, grid path {1e3 * new:.0f} us", flush=True)
     assert need > 0 and np.array_equal(u, w) and new <= 1.2 * old
+
+
+@pytest.mark.parametrize("n", [17, 19, 20, 24])
+def test_undecided_nodes_of_a_closed_mesh_around_the_eighth(n):
+    """A closed mesh far larger than the range whose signs are taken from
+    crossings: every node takes the solid angles, a workgroup each below 7168
+    nodes and eight a workgroup from there on; the grid equals the kernel that
+    takes every triangle at every node."""
+    import ctypes as C
+    import torch
+    from fundem_amd import build
+    lib = C.CDLL(build.CORE_LIB)
+    lib.fdm_meshGridWorkspaceBytes.restype = C.c_size_t
+    v, f = torus()
+    tri = torch.tensor((1e110 * v[f]).reshape(-1), dtype=torch.float64, device="cuda")
+    n3, o3, h = (C.c_int * 3)(n, n, n), (C.c_double * 3)(*[-1.6e110] * 3), 3.2e110 / (n - 1)
+    need = lib.fdm_meshGridWorkspaceBytes(C.c_int(len(f)), n3)
+    work = torch.zeros(int(need), dtype=torch.uint8, device="cuda")
+    stream, got = C.c_void_p(torch.cuda.current_stream().cuda_stream), []
+    for grid in (False, True):
+        out = torch.zeros(n ** 3, dtype=torch.float64, device="cuda")
+        args = (C.c_void_p(tri.data_ptr()), C.c_int(len(f)), o3, C.c_double(h), n3, C.c_int(0), C.c_void_p(out.data_ptr()))
+        if grid:
+            r = lib.fdm_launchMeshSignedDistanceGridWith(*args, C.c_void_p(work.data_ptr()), C.c_size_t(need), stream)
+        else:
+            r = lib.fdm_launchMeshSignedDistanceGrid(*args, stream)
+        assert r == 0 and need > 0
+        got.append(out.cpu().numpy())
+    assert np.array_equal(got[0], got[1], equal_nan=True)
